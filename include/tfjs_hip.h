@@ -322,6 +322,13 @@ enum {
   TFHIP_PROD = 5, TFHIP_ALL = 6, TFHIP_ANY = 7
 };
 int tfhip_reduce(tfhip_ctx* ctx, int op, int64_t x, int64_t out, int64_t outer, int64_t inner);
+/* The same over a block of neighbouring axes anywhere in the shape: x viewed as [outer, red, inner],
+ * the middle index reduced; out has outer * inner elements.  (The reference brings such axes
+ * innermost with a transposition first, ops/reduction_ops.ts:144-157.)  divisor: 1, or for a
+ * float32 sum the number that every element is divided by before it is added, which is how the
+ * reference takes a mean (ops/reduction_ops.ts:201-238). */
+int tfhip_reduce_axis(tfhip_ctx* ctx, int op, int64_t x, int64_t out, int64_t outer, int64_t red,
+                      int64_t inner, double divisor);
 /* One-pass row softmax; same result as the reference's 10-call composite
  * (ops/softmax.ts:45-79, ops/reduction_ops.ts:56-74) within float32 tolerance. */
 int tfhip_softmax_rows(tfhip_ctx* ctx, int64_t x, int64_t out, int64_t rows, int64_t cols);

@@ -724,6 +724,14 @@ static napi_value js_reduce(napi_env env, napi_callback_info info) {
   return undefined(env);
 }
 
+/* reduceAxis(ctx, op, x, out, outer, red, inner, divisor) */
+static napi_value js_reduce_axis(napi_env env, napi_callback_info info) {
+  ARGS(8);
+  INT(1, op); I64(2, x); I64(3, out); I64(4, outer); I64(5, red); I64(6, inner); F64(7, divisor);
+  CHECK(tfhip_reduce_axis(ctx, op, x, out, outer, red, inner, divisor));
+  return undefined(env);
+}
+
 static napi_value js_softmax_rows(napi_env env, napi_callback_info info) {
   ARGS(5);
   I64(1, x); I64(2, out); I64(3, rows); I64(4, cols);
@@ -847,7 +855,7 @@ static napi_value module_init(napi_env env, napi_value exports) {
       {"conv2d", js_conv2d}, {"depthwiseConv2d", js_depthwise}, {"separableConv2d", js_separable},
       {"separableSingleKernel", js_separable_single_kernel}, {"pool2d", js_pool2d},
       {"binary", js_binary}, {"unary", js_unary}, {"cast", js_cast}, {"copy", js_copy},
-      {"dequantize", js_dequantize}, {"fill", js_fill}, {"reduce", js_reduce},
+      {"dequantize", js_dequantize}, {"fill", js_fill}, {"reduce", js_reduce}, {"reduceAxis", js_reduce_axis},
       {"softmaxRows", js_softmax_rows}, {"gather", js_gather}, {"transpose", js_transpose},
       {"stridedCopy", js_strided_copy}, {"logicalNot", js_logical_not},
       {"batchnorm", js_batchnorm}, {"resizeBilinear", js_resize_bilinear},

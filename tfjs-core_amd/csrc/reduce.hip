@@ -19,6 +19,12 @@ __device__ __forceinline__ float ld(const void* p, int dt, int64_t i) {
   }
 }
 
+// What a mean sums: every element divided by the count first, each quotient rounded to float32
+// (ops/reduction_ops.ts:201-238).  The divisor is the same for the whole launch; 1 is a plain sum.
+__device__ __forceinline__ float quotient(float v, float divisor) {
+  return divisor == 1.f ? v : v / divisor;
+}
+
 constexpr int WAVE = 64;
 constexpr int ROWS_PER_BLOCK = 4;  // 4 wavefronts per workgroup, one row each
 
@@ -27,14 +33,14 @@ constexpr int ROWS_PER_BLOCK = 4;  // 4 wavefronts per workgroup, one row each
 // first index of the strict extremum; ties and NaN keep the earlier index.
 template <typename OutT>
 __global__ __launch_bounds__(WAVE* ROWS_PER_BLOCK) void reduce_rows_kernel(
-    int op, const void* x, int x_dt, OutT* out, int64_t outer, int64_t inner) {
+    int op, const void* x, int x_dt, OutT* out, int64_t outer, int64_t inner, float divisor) {
   const int lane = threadIdx.x & (WAVE - 1);
   const int64_t row = (int64_t)blockIdx.x * ROWS_PER_BLOCK + (threadIdx.x >> 6);
   if (row >= outer) return;
   const int64_t base = row * inner;
   if (op == TFHIP_SUM) {
     double s = 0.0;
-    for (int64_t j = lane; j < inner; j += WAVE) s += (double)ld(x, x_dt, base + j);
+    for (int64_t j = lane; j < inner; j += WAVE) s += (double)quotient(ld(x, x_dt, base + j), divisor);
     for (int off = WAVE / 2; off > 0; off >>= 1) s += __shfl_down(s, off, WAVE);
     if (lane == 0) {
       if (std::is_same<OutT, float>::value) out[row] = (OutT)(float)s;
@@ -94,7 +100,7 @@ __global__ __launch_bounds__(WAVE* ROWS_PER_BLOCK) void reduce_rows_kernel(
 // as the single pass does, so NaN survives only from slot 0 here too.
 __global__ __launch_bounds__(WAVE* ROWS_PER_BLOCK) void reduce_parts_kernel(
     int op, const void* x, int x_dt, double* pval, long long* pidx, int64_t outer, int64_t inner,
-    int parts, int64_t seg, int vec) {
+    int parts, int64_t seg, int vec, float divisor) {
   const int lane = threadIdx.x & (WAVE - 1);
   const int64_t piece = (int64_t)blockIdx.x * ROWS_PER_BLOCK + (threadIdx.x >> 6);
   if (piece >= outer * parts) return;
@@ -122,12 +128,14 @@ __global__ __launch_bounds__(WAVE* ROWS_PER_BLOCK) void reduce_parts_kernel(
 #pragma unroll
         for (int u = 0; u < U; u++)
 #pragma unroll
-          for (int e = 0; e < 4; e++) s[u] = sum ? s[u] + (double)v[u][e] : s[u] * (double)v[u][e];
+          for (int e = 0; e < 4; e++)
+            s[u] = sum ? s[u] + (double)quotient(v[u][e], divisor) : s[u] * (double)v[u][e];
       }
       for (; q < q1; q += WAVE) {
         const f32x4 v = xv[q];
 #pragma unroll
-        for (int e = 0; e < 4; e++) s[0] = sum ? s[0] + (double)v[e] : s[0] * (double)v[e];
+        for (int e = 0; e < 4; e++)
+          s[0] = sum ? s[0] + (double)quotient(v[e], divisor) : s[0] * (double)v[e];
       }
       j = q1 * 4 + lane;  // what is left of a row whose length is no multiple of 4
     }
@@ -136,9 +144,13 @@ __global__ __launch_bounds__(WAVE* ROWS_PER_BLOCK) void reduce_parts_kernel(
 #pragma unroll
       for (int u = 0; u < U; u++) v[u] = ld(x, x_dt, base + j + u * WAVE);
 #pragma unroll
-      for (int u = 0; u < U; u++) s[u] = sum ? s[u] + (double)v[u] : s[u] * (double)v[u];
+      for (int u = 0; u < U; u++)
+        s[u] = sum ? s[u] + (double)quotient(v[u], divisor) : s[u] * (double)v[u];
     }
-    for (; j < j1; j += WAVE) s[0] = sum ? s[0] + (double)ld(x, x_dt, base + j) : s[0] * (double)ld(x, x_dt, base + j);
+    for (; j < j1; j += WAVE) {
+      const float v = ld(x, x_dt, base + j);
+      s[0] = sum ? s[0] + (double)quotient(v, divisor) : s[0] * (double)v;
+    }
     double t = sum ? (s[0] + s[1]) + (s[2] + s[3]) : (s[0] * s[1]) * (s[2] * s[3]);
     for (int off = WAVE / 2; off > 0; off >>= 1) {
       const double o = __shfl_down(t, off, WAVE);
@@ -267,6 +279,147 @@ __global__ __launch_bounds__(WAVE* ROWS_PER_BLOCK) void reduce_finish_kernel(
     if (op == TFHIP_ARGMAX || op == TFHIP_ARGMIN) out[row] = (OutT)idx;
     else if (std::is_same<OutT, float>::value) out[row] = (OutT)best;
     else out[row] = (OutT)(int32_t)best;
+  }
+}
+
+// Reduction over axes that are not the innermost ones: x viewed as [outer, red, inner], the middle
+// index reduced (a bias gradient, batch-norm statistics: [pixels, channels] over the pixels).
+// Bound by the one read of x.  A workgroup is a block of `cl` column lanes (of VEC neighbouring
+// columns each, so that a row of lanes reads one contiguous run) by THREADS / cl row lanes; the
+// row lanes stride over the slice of `red` the workgroup owns with UNROLL loads in flight, and meet
+// in LDS in a fixed order, so the result does not depend on scheduling.  parts > 1: `red` is cut
+// into that many slices over workgroups, whose partial results reduce_finish_kernel combines.
+// The rules are those of reduce_rows_kernel: sums and products in double, an extremum starts from
+// element 0 and is replaced only by a strictly better value, equal values keep the lower index.
+// Before, such an axis was first transposed to the inside: [100352, 128] summed over its rows took
+// 84 us for the transposition and 15 for the sum, and a mean 34 more for the division.
+enum { COL_SUM = 0, COL_EXTREMUM = 1, COL_LOGICAL = 2 };
+template <int KIND, typename OutT, int VEC, int THREADS>
+__global__ __launch_bounds__(THREADS) void reduce_cols_kernel(
+    int op, const void* x, int x_dt, OutT* out, double* pval, long long* pidx, int64_t red,
+    int64_t inner, int cl_shift, int col_blocks, int parts, int64_t seg, float divisor) {
+  constexpr int UNROLL = 8;
+  // partial results, [row lane][column] with a row of one spare element (bank conflicts)
+  __shared__ double s_val[THREADS * VEC + THREADS];
+  __shared__ int64_t s_idx[KIND == COL_EXTREMUM ? THREADS * VEC + THREADS : 1];
+  const int cl = 1 << cl_shift, rl = THREADS >> cl_shift;
+  const int lc = threadIdx.x & (cl - 1), lr = threadIdx.x >> cl_shift;
+  // workgroup -> (outer, slice, column block), column blocks of a slice next to each other
+  const int cb = blockIdx.x % col_blocks;
+  const int64_t t = blockIdx.x / col_blocks;
+  const int part = (int)(t % parts);
+  const int64_t o = t / parts;
+  const int64_t col = ((int64_t)cb * cl + lc) * VEC;
+  const int64_t base = o * red * inner + col;
+  const int64_t r0 = part * seg, r1 = min(red, r0 + seg);
+  const bool want_max = op == TFHIP_MAX || op == TFHIP_ARGMAX;
+  const bool in = col < inner;  // (VEC divides inner: the lane's columns are in or out together)
+
+  double acc[VEC];
+  float best[VEC];
+  int64_t idx[VEC];
+  int hit[VEC];
+#pragma unroll
+  for (int e = 0; e < VEC; e++) {
+    acc[e] = op == TFHIP_PROD ? 1.0 : 0.0;
+    best[e] = KIND == COL_EXTREMUM && in ? ld(x, x_dt, base + e) : 0.f;
+    idx[e] = 0;
+    hit[e] = 0;
+  }
+  auto load = [&](int64_t r, float (&v)[VEC]) {
+    if (VEC == 4) {
+      const f32x4 q = *reinterpret_cast<const f32x4*>(static_cast<const float*>(x) + base + r * inner);
+#pragma unroll
+      for (int e = 0; e < VEC; e++) v[e] = q[e];
+    } else {
+#pragma unroll
+      for (int e = 0; e < VEC; e++) v[e] = ld(x, x_dt, base + r * inner + e);
+    }
+  };
+  auto take = [&](int64_t r, const float (&v)[VEC]) {
+#pragma unroll
+    for (int e = 0; e < VEC; e++) {
+      if (KIND == COL_SUM) {
+        if (op == TFHIP_SUM) acc[e] += (double)quotient(v[e], divisor);
+        else acc[e] *= (double)v[e];
+      } else if (KIND == COL_EXTREMUM) {
+        if (want_max ? v[e] > best[e] : v[e] < best[e]) {
+          best[e] = v[e];
+          idx[e] = r;
+        }
+      } else {
+        hit[e] |= (v[e] != 0.f) == (op == TFHIP_ANY);
+      }
+    }
+  };
+  if (in) {
+    int64_t r = r0 + lr;
+    for (; r + (int64_t)(UNROLL - 1) * rl < r1; r += (int64_t)UNROLL * rl) {
+      float v[UNROLL][VEC];
+#pragma unroll
+      for (int u = 0; u < UNROLL; u++) load(r + (int64_t)u * rl, v[u]);
+#pragma unroll
+      for (int u = 0; u < UNROLL; u++) take(r + (int64_t)u * rl, v[u]);
+    }
+    for (; r < r1; r += rl) {
+      float v[VEC];
+      load(r, v);
+      take(r, v);
+    }
+  }
+  const int cols = cl * VEC, pitch = cols + 1;
+#pragma unroll
+  for (int e = 0; e < VEC; e++) {
+    const int at = lr * pitch + lc * VEC + e;
+    s_val[at] = KIND == COL_SUM ? acc[e] : KIND == COL_EXTREMUM ? (double)best[e] : (double)hit[e];
+    if (KIND == COL_EXTREMUM) s_idx[at] = idx[e];
+  }
+  __syncthreads();
+  // `share` neighbouring lanes of one wavefront finish a column together
+  auto merge = [&](double& v, int64_t& i, double ov, int64_t oi) {
+    if (KIND == COL_SUM) {
+      v = op == TFHIP_SUM ? v + ov : v * ov;
+    } else if (KIND == COL_EXTREMUM) {
+      if ((want_max ? ov > v : ov < v) || (ov == v && oi < i)) {
+        v = ov;
+        i = oi;
+      }
+    } else {
+      v = v != 0.0 || ov != 0.0 ? 1.0 : 0.0;
+    }
+  };
+  const int share = min(WAVE, max(1, rl / VEC));
+  const int j = threadIdx.x & (share - 1), mine = threadIdx.x / share;
+  const int64_t c_out = (int64_t)cb * cols + mine;
+  const bool owner = mine < cols && c_out < inner;
+  double v = 0.0;
+  int64_t vi = 0;
+  if (owner) {
+    v = s_val[j * pitch + mine];
+    if (KIND == COL_EXTREMUM) vi = s_idx[j * pitch + mine];
+    for (int r = j + share; r < rl; r += share)
+      merge(v, vi, s_val[r * pitch + mine], KIND == COL_EXTREMUM ? s_idx[r * pitch + mine] : 0);
+  }
+  for (int off = share >> 1; off > 0; off >>= 1) {
+    const double ov = __shfl_down(v, off, WAVE);
+    const int64_t oi = KIND == COL_EXTREMUM ? __shfl_down(vi, off, WAVE) : 0;
+    merge(v, vi, ov, oi);
+  }
+  if (!owner || j != 0) return;
+  const int64_t at = o * inner + c_out;
+  if (parts > 1) {
+    pval[at * parts + part] = v;
+    if (KIND == COL_EXTREMUM) pidx[at * parts + part] = vi;
+  } else if (KIND == COL_SUM) {
+    if (std::is_same<OutT, float>::value) out[at] = (OutT)(float)v;
+    else out[at] = (OutT)(int32_t)(uint32_t)(int64_t)v;
+  } else if (KIND == COL_EXTREMUM) {
+    if (op == TFHIP_ARGMAX || op == TFHIP_ARGMIN) out[at] = (OutT)vi;
+    else if (std::is_same<OutT, float>::value) out[at] = (OutT)(float)v;
+    else out[at] = (OutT)(int32_t)(float)v;
+  } else {
+    const bool any = v != 0.0;
+    out[at] = (OutT)(op == TFHIP_ANY ? any : !any);
   }
 }
 
@@ -456,16 +609,12 @@ static unsigned grid_cap(tfhip_ctx* ctx, int64_t items, int block) {
 
 using namespace tfhip;
 
-extern "C" int tfhip_reduce(tfhip_ctx* ctx, int op, int64_t x, int64_t out, int64_t outer,
-                            int64_t inner) {
-  if (!ctx) return TFHIP_EINVAL;
+// Checks what the two entry points share.
+static int check_reduce(tfhip_ctx* ctx, int op, const Buf* bx, const Buf* bo, int64_t x_n, int64_t out_n) {
   if (op < TFHIP_SUM || op > TFHIP_ANY) return ctx->fail(TFHIP_EINVAL, "reduce: unknown op %d", op);
-  TFHIP_GET(ctx, bx, x);
-  TFHIP_GET(ctx, bo, out);
-  if (outer < 0 || inner < 0 || bx->numel != outer * inner || bo->numel != outer)
+  if (x_n < 0 || out_n < 0 || bx->numel != x_n || bo->numel != out_n)
     return ctx->fail(TFHIP_EINVAL, "reduce: buffers hold %lld and %lld elements, need %lld and %lld",
-                     (long long)bx->numel, (long long)bo->numel, (long long)(outer * inner),
-                     (long long)outer);
+                     (long long)bx->numel, (long long)bo->numel, (long long)x_n, (long long)out_n);
   if (bx->dtype == TFHIP_UINT8Q) return ctx->fail(TFHIP_EINVAL, "reduce: quantised input");
   const bool arg = op == TFHIP_ARGMAX || op == TFHIP_ARGMIN;
   if (arg && bo->dtype != TFHIP_INT32)
@@ -473,12 +622,34 @@ extern "C" int tfhip_reduce(tfhip_ctx* ctx, int op, int64_t x, int64_t out, int6
   const bool logical = op == TFHIP_ALL || op == TFHIP_ANY;
   if (logical ? bo->dtype != TFHIP_BOOL : (bo->dtype != TFHIP_INT32 && bo->dtype != TFHIP_FLOAT32))
     return ctx->fail(TFHIP_EINVAL, "reduce: output must be float32 or int32 (bool for all/any)");
-  if (outer == 0) return TFHIP_OK;
-  if (inner == 0) {
-    if (op == TFHIP_PROD) return tfhip_fill(ctx, out, 1.0);
-    if (op != TFHIP_SUM) return ctx->fail(TFHIP_EINVAL, "reduce: empty axis has no extremum");
-    return tfhip_fill(ctx, out, 0.0);
-  }
+  return TFHIP_OK;
+}
+
+static int launch_reduce_finish(tfhip_ctx* ctx, int op, const double* pval, const long long* pidx,
+                                const Buf* bo, int64_t outer, int parts) {
+  const dim3 grid((unsigned)ceil_div(outer, ROWS_PER_BLOCK)), block(WAVE * ROWS_PER_BLOCK);
+  if (bo->dtype == TFHIP_FLOAT32)
+    tfhip::launch(ctx, reduce_finish_kernel<float>, grid, block, 0, op, pval, pidx, (float*)bo->ptr,
+                  outer, parts);
+  else if (bo->dtype == TFHIP_BOOL)
+    tfhip::launch(ctx, reduce_finish_kernel<uint8_t>, grid, block, 0, op, pval, pidx,
+                  (uint8_t*)bo->ptr, outer, parts);
+  else
+    tfhip::launch(ctx, reduce_finish_kernel<int32_t>, grid, block, 0, op, pval, pidx,
+                  (int32_t*)bo->ptr, outer, parts);
+  TFHIP_LAUNCH_CHECK_NAMED(ctx, "reduce_finish");
+  return TFHIP_OK;
+}
+
+static int empty_axis(tfhip_ctx* ctx, int op, int64_t out) {
+  if (op == TFHIP_PROD) return tfhip_fill(ctx, out, 1.0);
+  if (op != TFHIP_SUM) return ctx->fail(TFHIP_EINVAL, "reduce: empty axis has no extremum");
+  return tfhip_fill(ctx, out, 0.0);
+}
+
+// Rows of `inner` elements (the innermost axes reduced).
+static int reduce_rows(tfhip_ctx* ctx, int op, const Buf* bx, const Buf* bo, int64_t outer,
+                       int64_t inner, float divisor) {
   if (ceil_div(outer, ROWS_PER_BLOCK) > 0x7fffffffLL) return ctx->fail(TFHIP_ENOTSUP, "reduce: too many rows");
   const dim3 block(WAVE * ROWS_PER_BLOCK);
   // Fewer rows than the machine has room for wavefronts, and rows long enough to be worth a
@@ -500,34 +671,125 @@ extern "C" int tfhip_reduce(tfhip_ctx* ctx, int op, int64_t x, int64_t out, int6
       double* pval = static_cast<double*>(partial.ptr);
       long long* pidx = reinterpret_cast<long long*>(pval + pieces);
       tfhip::launch(ctx, reduce_parts_kernel, dim3((unsigned)ceil_div(pieces, ROWS_PER_BLOCK)), block, 0,
-                    op, bx->ptr, bx->dtype, pval, pidx, outer, inner, (int)parts, seg, vec);
+                    op, bx->ptr, bx->dtype, pval, pidx, outer, inner, (int)parts, seg, vec, divisor);
       TFHIP_LAUNCH_CHECK_NAMED(ctx, "reduce_parts");
-      const dim3 fgrid((unsigned)ceil_div(outer, ROWS_PER_BLOCK));
-      if (bo->dtype == TFHIP_FLOAT32)
-        tfhip::launch(ctx, reduce_finish_kernel<float>, fgrid, block, 0, op, pval, pidx,
-                      (float*)bo->ptr, outer, (int)parts);
-      else if (bo->dtype == TFHIP_BOOL)
-        tfhip::launch(ctx, reduce_finish_kernel<uint8_t>, fgrid, block, 0, op, pval, pidx,
-                      (uint8_t*)bo->ptr, outer, (int)parts);
-      else
-        tfhip::launch(ctx, reduce_finish_kernel<int32_t>, fgrid, block, 0, op, pval, pidx,
-                      (int32_t*)bo->ptr, outer, (int)parts);
-      TFHIP_LAUNCH_CHECK_NAMED(ctx, "reduce_finish");
-      return TFHIP_OK;
+      return launch_reduce_finish(ctx, op, pval, pidx, bo, outer, (int)parts);
     }
   }
   const dim3 grid((unsigned)ceil_div(outer, ROWS_PER_BLOCK));
   if (bo->dtype == TFHIP_FLOAT32)
     tfhip::launch(ctx, reduce_rows_kernel<float>, grid, block, 0, op, bx->ptr,
-                       bx->dtype, (float*)bo->ptr, outer, inner);
+                       bx->dtype, (float*)bo->ptr, outer, inner, divisor);
   else if (bo->dtype == TFHIP_BOOL)
     tfhip::launch(ctx, reduce_rows_kernel<uint8_t>, grid, block, 0, op, bx->ptr,
-                       bx->dtype, (uint8_t*)bo->ptr, outer, inner);
+                       bx->dtype, (uint8_t*)bo->ptr, outer, inner, divisor);
   else
     tfhip::launch(ctx, reduce_rows_kernel<int32_t>, grid, block, 0, op, bx->ptr,
-                       bx->dtype, (int32_t*)bo->ptr, outer, inner);
+                       bx->dtype, (int32_t*)bo->ptr, outer, inner, divisor);
   TFHIP_LAUNCH_CHECK(ctx);
   return TFHIP_OK;
+}
+
+extern "C" int tfhip_reduce(tfhip_ctx* ctx, int op, int64_t x, int64_t out, int64_t outer,
+                            int64_t inner) {
+  if (!ctx) return TFHIP_EINVAL;
+  TFHIP_GET(ctx, bx, x);
+  TFHIP_GET(ctx, bo, out);
+  if (outer < 0 || inner < 0) return ctx->fail(TFHIP_EINVAL, "reduce: negative extent");
+  if (int rc = check_reduce(ctx, op, bx, bo, outer * inner, outer)) return rc;
+  if (outer == 0) return TFHIP_OK;
+  if (inner == 0) return empty_axis(ctx, op, out);
+  return reduce_rows(ctx, op, bx, bo, outer, inner, 1.f);
+}
+
+template <int KIND, typename OutT>
+static int launch_reduce_cols(tfhip_ctx* ctx, int op, const Buf* bx, const Buf* bo, int64_t outer,
+                              int64_t red, int64_t inner, float divisor) {
+  const bool vec = bx->dtype == TFHIP_FLOAT32 && inner % 4 == 0 &&
+                   (reinterpret_cast<uintptr_t>(bx->ptr) & 15) == 0;
+  const int64_t lanes = vec ? inner / 4 : inner;  // column lanes of a row
+  // One launch while a row lane of a tall workgroup (512 lanes) has few elements to walk, or where
+  // there are workgroups for every CU anyway: a second launch costs about 4 us.  A trip of eight
+  // loads takes about 2.5 us whatever it reads, so the workgroup is made as tall as it takes to
+  // have one or two trips, down to four column lanes (runs of 64 bytes): [1000, 512] 14.1 us with
+  // sixteen column lanes, 9.5 with four (12 for the transposition and the row sum before).
+  // Beyond 2048 elements the reduced axis is cut instead.
+  auto shift_for = [&](int most) {
+    int s = 0;
+    while ((1 << s) < most && (int64_t)(1 << s) < lanes) s++;
+    return s;
+  };
+  int tall = shift_for(16);
+  while (tall > 2 && red > 8 * (int64_t)(512 >> tall)) tall--;
+  const int64_t tall_groups = outer * ceil_div(lanes, 1 << tall);
+  const bool single = red <= 16 * (int64_t)(512 >> tall) || tall_groups >= 2 * ctx->num_cus || ctx->no_alloc;
+  if (single) {
+    const int64_t col_blocks = ceil_div(lanes, 1 << tall), grid = outer * col_blocks;
+    if (grid > 0x7fffffffLL || col_blocks > 0x7fffffffLL)
+      return ctx->fail(TFHIP_ENOTSUP, "reduce: too many columns");
+    if (vec)
+      tfhip::launch(ctx, (reduce_cols_kernel<KIND, OutT, 4, 512>), dim3((unsigned)grid), dim3(512), 0, op,
+                    bx->ptr, bx->dtype, (OutT*)bo->ptr, nullptr, nullptr, red, inner, tall, (int)col_blocks,
+                    1, red, divisor);
+    else
+      tfhip::launch(ctx, (reduce_cols_kernel<KIND, OutT, 1, 512>), dim3((unsigned)grid), dim3(512), 0, op,
+                    bx->ptr, bx->dtype, (OutT*)bo->ptr, nullptr, nullptr, red, inner, tall, (int)col_blocks,
+                    1, red, divisor);
+    TFHIP_LAUNCH_CHECK_NAMED(ctx, "reduce_cols");
+    return TFHIP_OK;
+  }
+  // Slices of at least 16 elements a row lane, about eight workgroups of 256 lanes per CU.
+  const int wide = shift_for(64);
+  const int64_t col_blocks = ceil_div(lanes, 1 << wide), rl = 256 >> wide;
+  int64_t parts = std::min<int64_t>(ceil_div(8 * (int64_t)ctx->num_cus, outer * col_blocks),
+                                    ceil_div(red, 16 * rl));
+  const int64_t seg = ceil_div(ceil_div(red, parts), rl) * rl;
+  parts = ceil_div(red, seg);
+  const int64_t cells = outer * inner * parts, grid = outer * col_blocks * parts;
+  if (grid > 0x7fffffffLL) return ctx->fail(TFHIP_ENOTSUP, "reduce: too many columns");
+  Temp partial(ctx);
+  if (!partial.get((size_t)cells * 16)) return TFHIP_EDEVICE;
+  double* pval = static_cast<double*>(partial.ptr);
+  long long* pidx = reinterpret_cast<long long*>(pval + cells);
+  if (vec)
+    tfhip::launch(ctx, (reduce_cols_kernel<KIND, OutT, 4, 256>), dim3((unsigned)grid), dim3(256), 0, op,
+                  bx->ptr, bx->dtype, (OutT*)bo->ptr, pval, pidx, red, inner, wide, (int)col_blocks,
+                  (int)parts, seg, divisor);
+  else
+    tfhip::launch(ctx, (reduce_cols_kernel<KIND, OutT, 1, 256>), dim3((unsigned)grid), dim3(256), 0, op,
+                  bx->ptr, bx->dtype, (OutT*)bo->ptr, pval, pidx, red, inner, wide, (int)col_blocks,
+                  (int)parts, seg, divisor);
+  TFHIP_LAUNCH_CHECK_NAMED(ctx, "reduce_cols");
+  if (parts == 1) return ctx->fail(TFHIP_EDEVICE, "reduce: bad plan");
+  return launch_reduce_finish(ctx, op, pval, pidx, bo, outer * inner, (int)parts);
+}
+
+extern "C" int tfhip_reduce_axis(tfhip_ctx* ctx, int op, int64_t x, int64_t out, int64_t outer,
+                                 int64_t red, int64_t inner, double divisor) {
+  if (!ctx) return TFHIP_EINVAL;
+  TFHIP_GET(ctx, bx, x);
+  TFHIP_GET(ctx, bo, out);
+  if (outer < 0 || red < 0 || inner < 0) return ctx->fail(TFHIP_EINVAL, "reduce: negative extent");
+  if (int rc = check_reduce(ctx, op, bx, bo, outer * red * inner, outer * inner)) return rc;
+  if (divisor != 1.0 && (op != TFHIP_SUM || bo->dtype != TFHIP_FLOAT32 || !((float)divisor != 0.f)))
+    return ctx->fail(TFHIP_EINVAL, "reduce: only a float32 sum has a divisor, and it is not 0");
+  if (bo->numel == 0) return TFHIP_OK;
+  if (red == 0) return empty_axis(ctx, op, out);
+  if (inner == 1) return reduce_rows(ctx, op, bx, bo, outer, red, (float)divisor);
+  switch (op) {
+    case TFHIP_SUM:
+    case TFHIP_PROD:
+      return bo->dtype == TFHIP_FLOAT32
+                 ? launch_reduce_cols<COL_SUM, float>(ctx, op, bx, bo, outer, red, inner, (float)divisor)
+                 : launch_reduce_cols<COL_SUM, int32_t>(ctx, op, bx, bo, outer, red, inner, 1.f);
+    case TFHIP_ALL:
+    case TFHIP_ANY:
+      return launch_reduce_cols<COL_LOGICAL, uint8_t>(ctx, op, bx, bo, outer, red, inner, 1.f);
+    default:
+      return bo->dtype == TFHIP_FLOAT32
+                 ? launch_reduce_cols<COL_EXTREMUM, float>(ctx, op, bx, bo, outer, red, inner, 1.f)
+                 : launch_reduce_cols<COL_EXTREMUM, int32_t>(ctx, op, bx, bo, outer, red, inner, 1.f);
+  }
 }
 
 extern "C" int tfhip_softmax_rows(tfhip_ctx* ctx, int64_t x, int64_t out, int64_t rows,

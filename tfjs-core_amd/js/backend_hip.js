@@ -807,6 +807,20 @@ class MathBackendHIP extends KernelBackend {
                      util.sizeFromShape(reduceShape));
     return out;
   }
+  // Extension of the plug-in API: any of the reductions over neighbouring axes anywhere in the
+  // shape, without a transposition; a sum may divide every element by `divisor` first (tf.mean).
+  reduceBlock(op, x, axes, divisor) {
+    const first = axes[0], last = axes[axes.length - 1];
+    const outDtype = op === 'all' || op === 'any' ? 'bool' : op === 'argMax' || op === 'argMin' ? 'int32' :
+        op === 'sum' || op === 'prod' ? util.upcastType(x.dtype, 'int32') :
+        x.dtype === 'float32' ? 'float32' : 'int32';
+    const out = this.out(x.shape.slice(0, first).concat(x.shape.slice(last + 1)), outDtype);
+    this.napi.reduceAxis(this.ctx, REDUCE[op], this.h(x), this.h(out),
+                         util.sizeFromShape(x.shape.slice(0, first)),
+                         util.sizeFromShape(x.shape.slice(first, last + 1)),
+                         util.sizeFromShape(x.shape.slice(last + 1)), divisor);
+    return out;
+  }
   sum(x, axes) { return this.reduce('sum', x, axes, util.upcastType(x.dtype, 'int32')); }
   topk(x, k, sorted) {
     const cols = x.shape[x.rank - 1];

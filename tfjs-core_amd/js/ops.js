@@ -837,6 +837,15 @@ const clipByValue = op('clipByValue', (x, clipValueMin, clipValueMax) => {
 const relu6 = op('relu6', x => clipByValue(x, 0, 6));
 
 // ---- reductions -------------------------------------------------------------------------
+// The axes in ascending order when they are neighbours, else null.  Backends with `reduceBlock`
+// (feature detection) reduce such axes where they are; for the others, and for axes that are
+// apart, the axes are brought innermost first, as the reference does.
+function axisBlock(axes) {
+  if (axes.length === 0 || typeof ENGINE.backend.reduceBlock !== 'function') return null;
+  const sorted = axes.slice().sort((a, b) => a - b);
+  return sorted[sorted.length - 1] - sorted[0] === sorted.length - 1 ? sorted : null;
+}
+
 function reduceOp(name, method) {
   return op(name, (x, axis, keepDims) => {
     let $x = convertToTensor(x, 'x', name);
@@ -848,14 +857,16 @@ function reduceOp(name, method) {
     let axes = origAxes;
     const permutedAxes = axis_util.getAxesPermutation(axes, $x.rank);
     let reduceInput = $x;
-    if (permutedAxes != null) {
+    const block = permutedAxes == null ? null : axisBlock(axes);
+    if (permutedAxes != null && block == null) {
       reduceInput = transpose($x, permutedAxes);
       axes = axis_util.getInnerMostAxes(axes.length, $x.rank);
     }
-    // dy (and y) stretched back over the reduced axes, which are the innermost ones here
+    // dy (and y) stretched back over the reduced axes
     const expand = t => reshape(t, reduceInput.shape.map((d, i) => axes.indexOf(i) === -1 ? d : 1));
     const res = ENGINE.runKernel((backend, save) => {
-      const y = backend[method](reduceInput, axes);
+      const y = block == null ? backend[method](reduceInput, axes) :
+                                backend.reduceBlock(method, reduceInput, block, 1);
       save([reduceInput, y]);
       return y;
     }, {$x: reduceInput}, ['sum', 'max', 'min'].indexOf(name) === -1 ? null : (dy, saved) => ({
@@ -885,6 +896,9 @@ function argOp(name, method) {
     let axes = util.parseAxisParam(axis, $x.shape);
     const permutedAxes = axis_util.getAxesPermutation(axes, $x.rank);
     if (permutedAxes != null) {
+      if (axisBlock(axes) != null) {
+        return ENGINE.runKernel(backend => backend.reduceBlock(method, $x, axes, 1), {$x});
+      }
       $x = transpose($x, permutedAxes);
       axes = axis_util.getInnerMostAxes(axes.length, $x.rank);
     }
@@ -1203,7 +1217,14 @@ const mean = op('mean', (x, axis, keepDims) => {
   const axes = util.parseAxisParam(axis, $x.shape);
   const reduceSize = util.sizeFromShape(axes.map(a => $x.shape[a]));
   const xf = $x.dtype === 'float32' ? $x : cast($x, 'float32');
-  return sum(div(xf, scalar(reduceSize)), axis, keepDims);
+  const block = reduceSize > 0 ? axisBlock(axes) : null;
+  if (block == null) return sum(div(xf, scalar(reduceSize)), axis, keepDims);
+  const keptShape = $x.shape.map((d, i) => block.indexOf(i) === -1 ? d : 1);
+  const res = ENGINE.runKernel(
+      backend => backend.reduceBlock('sum', xf, block, reduceSize), {xf}, dy => ({
+        xf: () => div(mul(reshape(dy, keptShape), ones($x.shape, 'float32')), scalar(reduceSize))
+      }));
+  return keepDims ? reshape(res, axis_util.expandShapeToKeepDim(res.shape, axes)) : res;
 });
 
 // ops/array_ops.ts:905-920

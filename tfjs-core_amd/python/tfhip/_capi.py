@@ -99,6 +99,7 @@ _SIGNATURES = {
     "tfhip_dequantize": [_PTR, _I64, _I64, C.POINTER(QParams)],
     "tfhip_fill": [_PTR, _I64, C.c_double],
     "tfhip_reduce": [_PTR, _INT, _I64, _I64, _I64, _I64],
+    "tfhip_reduce_axis": [_PTR, _INT, _I64, _I64, _I64, _I64, _I64, C.c_double],
     "tfhip_softmax_rows": [_PTR, _I64, _I64, _I64, _I64],
     "tfhip_gather": [_PTR, _I64, _I64, _I64, _I64, _I64, _I64, _I64],
     "tfhip_transpose": [_PTR, _I64, C.POINTER(C.c_int32), _INT, C.POINTER(C.c_int32), _I64],

@@ -620,6 +620,22 @@ class MathBackendHIP(object):
                                        su.size_from_shape(red_shape)))
         return out
 
+    def reduce_block(self, op, x, axes, divisor=1.0):
+        """Extension of the plug-in API: `op` ("sum", "prod", "max", "min", "all", "any", "arg_max",
+        "arg_min") over neighbouring axes anywhere in the shape, without a transposition; a sum
+        may divide every element by `divisor` first (tf.mean)."""
+        dtype = {"all": "bool", "any": "bool", "arg_max": "int32", "arg_min": "int32"}.get(op)
+        if dtype is None:
+            dtype = su.upcast_type(x.dtype, "int32") if op in ("sum", "prod") else \
+                "float32" if x.dtype == "float32" else "int32"
+        first, last = axes[0], axes[-1]
+        out = self._out(x.shape[:first] + x.shape[last + 1:], dtype)
+        self._ck(self.lib.tfhip_reduce_axis(
+            self.ctx, capi.REDUCE[op.replace("_", "")], self._h(x), self._h(out),
+            su.size_from_shape(x.shape[:first]), su.size_from_shape(x.shape[first:last + 1]),
+            su.size_from_shape(x.shape[last + 1:]), float(divisor)))
+        return out
+
     def sum(self, x, axes):
         return self._reduce("sum", x, axes, su.upcast_type(x.dtype, "int32"))
 

@@ -442,17 +442,33 @@ def relu6(x):
 
 
 # ---- reductions (ops/reduction_ops.ts) ----
-def _reduce(method, x, axis, keep_dims):
+def _axis_block(axes):
+    """The axes in ascending order when they are neighbours, else None.  Backends with
+    `reduce_block` (feature detection) reduce such axes where they are; for the others, and for
+    axes that are apart, the axes are brought innermost first, as the reference does."""
+    axes = sorted(axes)
+    if axes and axes[-1] - axes[0] == len(axes) - 1 and hasattr(ENGINE.backend, "reduce_block"):
+        return axes
+    return None
+
+
+def _reduce(method, x, axis, keep_dims, divisor=None):
     x = _conv(x, "x", method)
 
     def run():
         axes = su.parse_axis_param(axis, x.shape)
         perm = su.get_axes_permutation(axes, x.rank)
+        block = _axis_block(axes) if perm is not None or divisor is not None else None
         xt, red = x, axes
-        if perm is not None:
-            xt = transpose(x, perm)
-            red = su.get_inner_most_axes(len(axes), x.rank)
-        r = ENGINE.run_kernel(lambda be: getattr(be, method)(xt, red))
+        if block is not None:
+            r = ENGINE.run_kernel(lambda be: be.reduce_block(method, x, block, divisor or 1.0))
+        else:
+            if divisor is not None:
+                xt = div(x, tensor(divisor))
+            if perm is not None:
+                xt = transpose(xt, perm)
+                red = su.get_inner_most_axes(len(axes), x.rank)
+            r = ENGINE.run_kernel(lambda be: getattr(be, method)(xt, red))
         if keep_dims:
             out_shape, _ = su.compute_out_and_reduce_shapes(x.shape, axes)
             r = reshape(r, su.expand_shape_to_keep_dim(out_shape, axes))
@@ -556,6 +572,8 @@ def _arg(method, x, axis):
         perm = su.get_axes_permutation(axes, x.rank)
         xt = x
         if perm is not None:
+            if _axis_block(axes) is not None:
+                return ENGINE.run_kernel(lambda be: be.reduce_block(method, x, axes))
             xt = transpose(x, perm)
             axes = su.get_inner_most_axes(1, x.rank)
         return ENGINE.run_kernel(lambda be: getattr(be, method)(xt, axes[0]))
@@ -1114,7 +1132,7 @@ def mean(x, axis=None, keep_dims=False):
         for a in axes:
             n *= xt.shape[a]
         xf = xt if xt.dtype == "float32" else cast(xt, "float32")
-        return sum(div(xf, tensor(float(n))), axis, keep_dims)
+        return _reduce("sum", xf, axis, keep_dims, float(n))
     return ENGINE.tidy(run)
 
 
