@@ -5,6 +5,7 @@
 // the order the reference's loops do, so sums round the same way and nothing depends on
 // scheduling (no atomics on data).
 #include <climits>
+#include <type_traits>
 
 #include "tfhip_internal.h"
 
@@ -107,6 +108,145 @@ __global__ __launch_bounds__(256) void scatter_rows_kernel(const int64_t* flat, 
     }
     if (live) out[g] = (T)acc;
   }
+}
+
+// The same for slices of 32 elements and more (an embedding's gradient).  The kernel above walks
+// the whole index list for every 256 result elements, which is what it is bound by: 10240 updates
+// of 128 into 20000 rows took 1980 us; 64 here.  A workgroup owns the rows f with
+// f % groups = its number (so that the frequent rows of a text, which have neighbouring numbers,
+// go to different workgroups) and 64 columns for each of CW wavefronts side by side: it walks the
+// list once, 4096 entries at a time with 16 loads in flight per lane, and packs the entries of its
+// rows, in order, into LDS.  A wavefront then takes a row, finds its entries by ballot and adds
+// them in ascending order, up to 64 updates in flight: what bounds it is the most frequent row, a
+// chain of hundreds of additions.  The sums lie in LDS between passes; every one is taken in the
+// order of the list, as above.
+constexpr int SCATTER_PASS = 4096;
+template <typename T, typename Acc, int CW>
+__global__ __launch_bounds__(256) void scatter_groups_kernel(const int64_t* __restrict__ flat,
+                                                             const T* __restrict__ updates, T* __restrict__ out,
+                                                             int rows, int64_t slice, int64_t n_updates,
+                                                             T start, int sum_dupes, int scalar_update,
+                                                             int group_shift, int local_rows) {
+  constexpr int PER = SCATTER_PASS / 256, CB = 64 * CW, ROW_WAVES = 4 / CW;
+  extern __shared__ __attribute__((aligned(16))) char scatter_lds[];
+  Acc* sums = reinterpret_cast<Acc*>(scatter_lds);  // [local_rows][CB]
+  __shared__ unsigned list[SCATTER_PASS];           // local row << 12 | entry of the pass
+  __shared__ int first[PER * 4 + 1];                // where a wavefront's entries of a load begin
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int groups = 1 << group_shift, mine = (int)blockIdx.x;
+  const int own = (wave % CW) * 64 + lane;          // column within the block
+  const int64_t col = (int64_t)blockIdx.y * CB + own;
+  const bool stored = col < slice;
+  const int64_t read_col = stored ? col : 0;        // (a column past the slice: summed, not stored)
+  for (int i = tid; i < local_rows * CB; i += 256) sums[i] = (Acc)start;
+  for (int64_t i0 = 0; i0 < n_updates; i0 += SCATTER_PASS) {
+    int64_t f[PER];
+#pragma unroll
+    for (int u = 0; u < PER; u++) {
+      const int64_t i = i0 + u * 256 + tid;
+      f[u] = i < n_updates ? flat[i] : -1;
+    }
+    unsigned long long hit[PER];
+#pragma unroll
+    for (int u = 0; u < PER; u++) {
+      const bool in = f[u] >= 0 && f[u] < rows && ((int)f[u] & (groups - 1)) == mine;
+      hit[u] = __ballot(in);
+      if (lane == 0) first[u * 4 + wave] = __popcll(hit[u]);
+    }
+    __syncthreads();
+    if (wave == 0) {  // 64 counts into their prefix sums
+      int n = first[lane];
+      const int count = n;
+      for (int off = 1; off < 64; off <<= 1) {
+        const int o = __shfl_up(n, off, 64);
+        if (lane >= off) n += o;
+      }
+      first[lane] = n - count;
+      if (lane == 63) first[64] = n;
+    }
+    __syncthreads();
+    const int total = __builtin_amdgcn_readfirstlane(first[64]);
+#pragma unroll
+    for (int u = 0; u < PER; u++)
+      if (hit[u] >> lane & 1)
+        list[first[u * 4 + wave] + __popcll(hit[u] & ((1ull << lane) - 1))] =
+            (unsigned)((int)f[u] >> group_shift) << 12 | (unsigned)(u * 256 + tid);
+    __syncthreads();
+    const T* pass_updates = updates + (scalar_update ? 0 : i0 * slice);
+    const int64_t step = scalar_update ? 0 : slice;
+    const int64_t at_col = scalar_update ? 0 : read_col;
+    for (int r = wave / CW; r < local_rows && total > 0; r += ROW_WAVES) {
+      Acc acc = sums[r * CB + own];
+      for (int c0 = 0; c0 < total; c0 += 64) {
+        const unsigned e = c0 + lane < total ? list[c0 + lane] : ~0u;
+        unsigned long long left = __ballot((int)(e >> 12) == r);
+        // up to U updates in flight, added in ascending order.  (No branches around the loads, or
+        // each would be waited for: past the last entry the one before is read again.)
+        auto take = [&](auto most) {
+          constexpr int U = decltype(most)::value;
+          T x[U];
+          const int n = min(U, (int)__popcll(left));
+          int at = 0;
+#pragma unroll
+          for (int u = 0; u < U; u++) {
+            at = left ? __builtin_ctzll(left) : at;
+            left &= left - 1;
+            const int entry = __builtin_amdgcn_readlane((int)e, at) & (SCATTER_PASS - 1);
+            x[u] = (pass_updates + entry * step)[at_col];
+          }
+#pragma unroll
+          for (int u = 0; u < U; u++)
+            if (u < n) acc = sum_dupes ? (Acc)(acc + x[u]) : (Acc)x[u];
+        };
+        while (left) {
+          const int n = __popcll(left);
+          if (n > 16) take(std::integral_constant<int, 64>());
+          else if (n > 2) take(std::integral_constant<int, 16>());
+          else take(std::integral_constant<int, 2>());
+        }
+      }
+      sums[r * CB + own] = acc;
+    }
+    __syncthreads();
+  }
+  __syncthreads();
+  for (int r = wave / CW; r < local_rows; r += ROW_WAVES) {
+    const int64_t row = mine + (int64_t)r * groups;
+    if (row >= rows) break;
+    if (stored) out[row * slice + col] = (T)sums[r * CB + own];
+  }
+}
+
+template <typename T, typename Acc, int CW>
+static void launch_scatter_groups(tfhip_ctx* ctx, const int64_t* flat, const T* updates, T* out, int rows,
+                                  int64_t slice, int64_t n_updates, T start, int sum_dupes, int scalar_update) {
+  constexpr int CB = 64 * CW, MOST_LOCAL = (40 << 10) / (CB * (int)sizeof(Acc));  // 40 KB of sums
+  const int64_t col_blocks = ceil_div(slice, CB);
+  // enough groups that a group's sums fit, and four workgroups per CU where there are rows for them
+  int shift = 0;
+  while (ceil_div(rows, (int64_t)1 << shift) > MOST_LOCAL ||
+         (((int64_t)1 << shift) * col_blocks < 4 * ctx->num_cus && ((int64_t)2 << shift) <= rows))
+    shift++;
+  const int local_rows = (int)ceil_div(rows, (int64_t)1 << shift);
+  tfhip::launch(ctx, (scatter_groups_kernel<T, Acc, CW>), dim3(1u << shift, (unsigned)col_blocks), dim3(256),
+                (size_t)local_rows * CB * sizeof(Acc), flat, updates, out, rows, slice, n_updates, start,
+                sum_dupes, scalar_update, shift, local_rows);
+}
+template <typename T, typename Acc>
+static void launch_scatter(tfhip_ctx* ctx, const int64_t* flat, const T* updates, T* out, int64_t rows,
+                           int64_t slice, int64_t n_updates, T start, int sum_dupes, int scalar_update) {
+  // (half a wavefront of columns, and column blocks that a grid's second dimension holds)
+  if (slice >= 32 && n_updates > 0 && slice <= 65535 * 256) {
+    if (slice <= 64)
+      launch_scatter_groups<T, Acc, 1>(ctx, flat, updates, out, (int)rows, slice, n_updates, start, sum_dupes, scalar_update);
+    else if (slice <= 128)
+      launch_scatter_groups<T, Acc, 2>(ctx, flat, updates, out, (int)rows, slice, n_updates, start, sum_dupes, scalar_update);
+    else
+      launch_scatter_groups<T, Acc, 4>(ctx, flat, updates, out, (int)rows, slice, n_updates, start, sum_dupes, scalar_update);
+    return;
+  }
+  tfhip::launch(ctx, (scatter_rows_kernel<T, Acc>), dim3(blocks_for(ctx, rows * slice)), dim3(256), 0, flat,
+                updates, out, rows, slice, n_updates, start, sum_dupes, scalar_update);
 }
 
 // Source rows / columns of a resized pixel as the reference computes them, in double.
@@ -376,21 +516,17 @@ extern "C" int tfhip_scatter_nd(tfhip_ctx* ctx, int64_t indices, int64_t updates
     return ctx->fail(TFHIP_EINVAL, "scatterND: updates and result must both be float32 or both int32");
   if (bo->numel == 0) return TFHIP_OK;
   if (rows > INT_MAX) return ctx->fail(TFHIP_ENOTSUP, "scatterND: more than 2^31 - 1 result slices");
-  const dim3 grid(blocks_for(ctx, bo->numel)), block(256);
   const int sum = flags & TFHIP_SCATTER_SUM ? 1 : 0, one = scalar_update ? 1 : 0;
   const int64_t* fl = (const int64_t*)flat.ptr;
   if (bo->dtype == TFHIP_INT32)
-    tfhip::launch(ctx, (scatter_rows_kernel<int32_t, int32_t>), grid, block, 0, fl,
-                       (const int32_t*)bu->ptr, (int32_t*)bo->ptr, rows, slice, num_updates,
-                       (int32_t)default_value, sum, one);
+    launch_scatter<int32_t, int32_t>(ctx, fl, (const int32_t*)bu->ptr, (int32_t*)bo->ptr, rows, slice, num_updates,
+                                     (int32_t)default_value, sum, one);
   else if (flags & TFHIP_SCATTER_WIDE_SUM)
-    tfhip::launch(ctx, (scatter_rows_kernel<float, double>), grid, block, 0, fl,
-                       (const float*)bu->ptr, (float*)bo->ptr, rows, slice, num_updates,
-                       (float)default_value, sum, one);
+    launch_scatter<float, double>(ctx, fl, (const float*)bu->ptr, (float*)bo->ptr, rows, slice, num_updates,
+                                  (float)default_value, sum, one);
   else
-    tfhip::launch(ctx, (scatter_rows_kernel<float, float>), grid, block, 0, fl,
-                       (const float*)bu->ptr, (float*)bo->ptr, rows, slice, num_updates,
-                       (float)default_value, sum, one);
+    launch_scatter<float, float>(ctx, fl, (const float*)bu->ptr, (float*)bo->ptr, rows, slice, num_updates,
+                                 (float)default_value, sum, one);
   TFHIP_LAUNCH_CHECK(ctx);
   return TFHIP_OK;
 }
