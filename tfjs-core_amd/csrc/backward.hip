@@ -86,14 +86,33 @@ __global__ __launch_bounds__(256) void depthwise_der_filter_partial_kernel(
         ((red[0][lane] + red[1][lane]) + red[2][lane]) + red[3][lane];
 }
 
-// dW[tap][d1][dm] = sum of the slices' partial sums, ascending slice order.
-__global__ void depthwise_der_filter_finish_kernel(const double* partial, float* dw, int64_t w_n,
-                                                   int slices) {
-  const int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (g >= w_n) return;
+// dW[tap][d1][dm] = sum of the slices' partial sums: a workgroup takes 32 elements, its 8 rows of
+// lanes every 8th slice with 8 loads in flight, and the 8 sums are added in ascending order.  One
+// lane per element walking its slices alone was a chain of loads: 1152 elements of 512 slices took
+// 94 us, 4 here.
+__global__ __launch_bounds__(256) void depthwise_der_filter_finish_kernel(const double* partial, float* dw,
+                                                                          int64_t w_n, int slices) {
+  __shared__ double sums[8][32];
+  const int lane = threadIdx.x & 31, row = threadIdx.x >> 5;
+  const int64_t g = (int64_t)blockIdx.x * 32 + lane;
   double s = 0.0;
-  for (int i = 0; i < slices; i++) s += partial[(int64_t)i * w_n + g];
-  dw[g] = (float)s;
+  if (g < w_n) {
+    int i = row;
+    for (; i + 56 < slices; i += 64) {
+      double v[8];
+#pragma unroll
+      for (int u = 0; u < 8; u++) v[u] = partial[(int64_t)(i + 8 * u) * w_n + g];
+#pragma unroll
+      for (int u = 0; u < 8; u++) s += v[u];
+    }
+    for (; i < slices; i += 8) s += partial[(int64_t)i * w_n + g];
+  }
+  sums[row][lane] = s;
+  __syncthreads();
+  if (row == 0 && g < w_n) {
+    for (int r = 1; r < 8; r++) s += sums[r][lane];
+    dw[g] = (float)s;
+  }
 }
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
@@ -113,17 +132,11 @@ __global__ void flip_depthwise_filter_kernel(const float* w, float* out, int KH,
 template <int S>
 __global__ __launch_bounds__(256) void depthwise_der_input_vec_kernel(
     const float* __restrict__ dy, const float* __restrict__ w, float* __restrict__ dx,
-    const tfhip_conv2d_info ci) {
-  const int c4 = ci.in_c / 4;
-  const int64_t total = (int64_t)ci.batch * ci.in_h * ci.in_w * c4;
-  const int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const tfhip_conv2d_info ci, uint32_t total, Divisor by_c4, Divisor by_w, Divisor by_h) {
+  const uint32_t g = blockIdx.x * blockDim.x + threadIdx.x;
   if (g >= total) return;
-  const int cq = (int)(g % c4);
-  int64_t t = g / c4;
-  const int xc = (int)(t % ci.in_w);
-  t /= ci.in_w;
-  const int xr = (int)(t % ci.in_h);
-  const int n = (int)(t / ci.in_h);
+  uint32_t t = g;
+  const int cq = (int)by_c4.divmod(t), xc = (int)by_w.divmod(t), xr = (int)by_h.divmod(t), n = (int)t;
   const int sh = S ? S : ci.stride_h, sw = S ? S : ci.stride_w;
   const int xr_corner = xr - (ci.filter_h - 1 - ci.pad_top);
   const int xc_corner = xc - (ci.filter_w - 1 - ci.pad_left);
@@ -143,7 +156,7 @@ __global__ __launch_bounds__(256) void depthwise_der_input_vec_kernel(
       acc += d * f;
     }
   }
-  *reinterpret_cast<f32x4*>(dx + g * 4) = acc;
+  *reinterpret_cast<f32x4*>(dx + (int64_t)g * 4) = acc;
 }
 
 // dW of a 3x3 depthwise filter (multiplier 1): one pass over the output pixels of a slice;
@@ -153,7 +166,7 @@ __global__ __launch_bounds__(256) void depthwise_der_input_vec_kernel(
 // wavefronts) are then added in a fixed order through LDS.  partial[slice][tap][c] in double.
 __global__ __launch_bounds__(256) void depthwise3x3_der_filter_partial_kernel(
     const float* __restrict__ x, const float* __restrict__ dy, double* __restrict__ partial,
-    const tfhip_conv2d_info ci, int quads_per_wave, int64_t pixels_per_slice) {
+    const tfhip_conv2d_info ci, int quads_per_wave, int64_t pixels_per_slice, Divisor by_w, Divisor by_h) {
   extern __shared__ __attribute__((aligned(16))) float red[];  // [256 lanes][9 taps][4]
   const int tid = threadIdx.x;
   const int c4 = ci.in_c / 4;
@@ -170,10 +183,8 @@ __global__ __launch_bounds__(256) void depthwise3x3_der_filter_partial_kernel(
   for (int k = 0; k < 9; k++) acc[k] = f32x4{0.f, 0.f, 0.f, 0.f};
   if (live) {
     for (int64_t px = p0 + sub; px < p1; px += subs) {
-      const int yc = (int)(px % ci.out_w);
-      const int64_t t = px / ci.out_w;
-      const int yr = (int)(t % ci.out_h);
-      const int n = (int)(t / ci.out_h);
+      uint32_t t = (uint32_t)px;
+      const int yc = (int)by_w.divmod(t), yr = (int)by_h.divmod(t), n = (int)t;
       const f32x4 d = *reinterpret_cast<const f32x4*>(dy + px * ci.out_c + cq * 4);
       const int xr0 = yr * ci.stride_h - ci.pad_top, xc0 = yc * ci.stride_w - ci.pad_left;
       const float* xn = x + (int64_t)n * ci.in_h * ci.in_w * ci.in_c + cq * 4;
@@ -282,30 +293,25 @@ __global__ void pool2d_backprop_kernel(const float* dy, const float* x, float* d
 // the window scan and the dy gather are 16-byte accesses, the winner is tracked per channel.
 __global__ __launch_bounds__(256) void pool2d_backprop_vec_kernel(
     const float* __restrict__ dy, const float* __restrict__ x, float* __restrict__ dx,
-    const tfhip_conv2d_info ci, int kind) {
+    const tfhip_conv2d_info ci, int kind, uint32_t total, Divisor by_c4, Divisor by_w, Divisor by_h,
+    Divisor by_sh, Divisor by_sw) {
   const int eff_h = ci.filter_h + (ci.filter_h - 1) * (ci.dilation_h - 1);
   const int eff_w = ci.filter_w + (ci.filter_w - 1) * (ci.dilation_w - 1);
   const int pad_top = eff_h - 1 - ci.pad_top, pad_left = eff_w - 1 - ci.pad_left;
-  const int c4 = ci.in_c / 4;
-  const int64_t total = (int64_t)ci.batch * ci.in_h * ci.in_w * c4;
-  const int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const uint32_t g = blockIdx.x * blockDim.x + threadIdx.x;
   if (g >= total) return;
-  const int cq = (int)(g % c4);
-  int64_t t = g / c4;
-  const int xc = (int)(t % ci.in_w);
-  t /= ci.in_w;
-  const int xr = (int)(t % ci.in_h);
-  const int n = (int)(t / ci.in_h);
+  uint32_t t = g;
+  const int cq = (int)by_c4.divmod(t), xc = (int)by_w.divmod(t), xr = (int)by_h.divmod(t), n = (int)t;
   const float* xn = x + (int64_t)n * ci.in_h * ci.in_w * ci.in_c + cq * 4;
   const float* dyn = dy + (int64_t)n * ci.out_h * ci.out_w * ci.out_c + cq * 4;
   f32x4 acc = {0.f, 0.f, 0.f, 0.f};
   for (int wr = 0; wr < eff_h; wr += ci.dilation_h) {
     const int num_r = xr - pad_top + wr;
-    const int yr = num_r / ci.stride_h;
+    const int yr = (int)by_sh.quotient((uint32_t)max(num_r, 0));
     if (num_r < 0 || yr * ci.stride_h != num_r || yr >= ci.out_h) continue;
     for (int wc = 0; wc < eff_w; wc += ci.dilation_w) {
       const int num_c = xc - pad_left + wc;
-      const int yc = num_c / ci.stride_w;
+      const int yc = (int)by_sw.quotient((uint32_t)max(num_c, 0));
       if (num_c < 0 || yc * ci.stride_w != num_c || yc >= ci.out_w) continue;
       const f32x4 d = *reinterpret_cast<const f32x4*>(dyn + ((int64_t)yr * ci.out_w + yc) * ci.out_c);
       if (kind != TFHIP_POOL_MAX) {
@@ -339,7 +345,7 @@ __global__ __launch_bounds__(256) void pool2d_backprop_vec_kernel(
     }
   }
   if (kind != TFHIP_POOL_MAX) acc *= 1.0f / (float)(ci.filter_h * ci.filter_w);
-  *reinterpret_cast<f32x4*>(dx + g * 4) = acc;
+  *reinterpret_cast<f32x4*>(dx + (int64_t)g * 4) = acc;
 }
 
 static int check_geometry(tfhip_ctx* ctx, const char* op, const tfhip_conv2d_info* ci,
@@ -408,19 +414,23 @@ extern "C" int tfhip_depthwise_conv2d_der_input(tfhip_ctx* ctx, int64_t dy, int6
     strncat(ctx->last_kernel, "_as_der_input", sizeof ctx->last_kernel - strlen(ctx->last_kernel) - 1);
     return TFHIP_OK;
   }
-  if (ch_mul == 1 && ci->in_c % 4 == 0 && aligned16(dyf) && aligned16(wf) && aligned16(dxf)) {
+  if (ch_mul == 1 && ci->in_c % 4 == 0 && x_n / 4 <= INDEX32 - 256 && aligned16(dyf) && aligned16(wf) &&
+      aligned16(dxf)) {
     const unsigned blocks = (unsigned)ceil_div(x_n / 4, 256);
     const int s = ci->stride_h == ci->stride_w && ci->stride_h <= 2 ? ci->stride_h : 0;
     ctx->name_kernel("depthwise_der_input_vec_s%d", s);
     if (s == 1)
       tfhip::launch(ctx, depthwise_der_input_vec_kernel<1>, dim3(blocks), dim3(256), 0,
-                         dyf, wf, dxf, *ci);
+                         dyf, wf, dxf, *ci, (uint32_t)(x_n / 4), Divisor(ci->in_c / 4),
+                         Divisor(ci->in_w), Divisor(ci->in_h));
     else if (s == 2)
       tfhip::launch(ctx, depthwise_der_input_vec_kernel<2>, dim3(blocks), dim3(256), 0,
-                         dyf, wf, dxf, *ci);
+                         dyf, wf, dxf, *ci, (uint32_t)(x_n / 4), Divisor(ci->in_c / 4),
+                         Divisor(ci->in_w), Divisor(ci->in_h));
     else
       tfhip::launch(ctx, depthwise_der_input_vec_kernel<0>, dim3(blocks), dim3(256), 0,
-                         dyf, wf, dxf, *ci);
+                         dyf, wf, dxf, *ci, (uint32_t)(x_n / 4), Divisor(ci->in_c / 4),
+                         Divisor(ci->in_w), Divisor(ci->in_h));
     TFHIP_LAUNCH_CHECK(ctx);
     return TFHIP_OK;
   }
@@ -458,7 +468,7 @@ extern "C" int tfhip_depthwise_conv2d_der_filter(tfhip_ctx* ctx, int64_t x, int6
   if ((rc = as_f32(ctx, bdy, &tdy, &dyf))) return rc;
   const int64_t pixels = (int64_t)ci->batch * ci->out_h * ci->out_w;
   if (ch_mul == 1 && ci->filter_h == 3 && ci->filter_w == 3 && ci->in_c % 4 == 0 && aligned16(xf) &&
-      aligned16(dyf) && pixels > 0) {
+      aligned16(dyf) && pixels > 0 && pixels <= INDEX32) {
     const int c4 = ci->in_c / 4;
     int qpw = 1;                       // channel quads per workgroup: a power of two <= 64
     while (qpw < 64 && qpw < c4) qpw *= 2;
@@ -475,9 +485,9 @@ extern "C" int tfhip_depthwise_conv2d_der_filter(tfhip_ctx* ctx, int64_t x, int6
     ctx->name_kernel("depthwise3x3_der_filter");
     tfhip::launch(ctx, depthwise3x3_der_filter_partial_kernel, dim3((unsigned)blocks_c, (unsigned)slices),
                        dim3(256), (size_t)(256 * 9 * 4 * sizeof(float)), xf, dyf,
-                       static_cast<double*>(tpart.ptr), *ci, qpw, per_slice);
+                       static_cast<double*>(tpart.ptr), *ci, qpw, per_slice, Divisor(ci->out_w), Divisor(ci->out_h));
     TFHIP_LAUNCH_CHECK(ctx);
-    tfhip::launch(ctx, depthwise_der_filter_finish_kernel, dim3((unsigned)ceil_div(w_n, 256)), dim3(256),
+    tfhip::launch(ctx, depthwise_der_filter_finish_kernel, dim3((unsigned)ceil_div(w_n, 32)), dim3(256),
                        0, static_cast<const double*>(tpart.ptr),
                        static_cast<float*>(bdw->ptr), w_n, (int)slices);
     TFHIP_LAUNCH_CHECK(ctx);
@@ -495,7 +505,7 @@ extern "C" int tfhip_depthwise_conv2d_der_filter(tfhip_ctx* ctx, int64_t x, int6
   tfhip::launch(ctx, depthwise_der_filter_partial_kernel,
                      dim3((unsigned)channel_blocks, (unsigned)taps, (unsigned)slices), dim3(256), 0, xf, dyf, static_cast<double*>(tpart.ptr), *ci, ch_mul, per_slice);
   TFHIP_LAUNCH_CHECK(ctx);
-  tfhip::launch(ctx, depthwise_der_filter_finish_kernel, dim3((unsigned)ceil_div(w_n, 256)), dim3(256),
+  tfhip::launch(ctx, depthwise_der_filter_finish_kernel, dim3((unsigned)ceil_div(w_n, 32)), dim3(256),
                      0, static_cast<const double*>(tpart.ptr),
                      static_cast<float*>(bdw->ptr), w_n, (int)slices);
   TFHIP_LAUNCH_CHECK(ctx);
@@ -524,10 +534,12 @@ extern "C" int tfhip_pool2d_backprop(tfhip_ctx* ctx, int64_t dy, int64_t x, int6
   if ((rc = as_f32(ctx, bdy, &tdy, &dyf))) return rc;
   if ((rc = as_f32(ctx, bx, &tx, &xf))) return rc;
   float* dxf = static_cast<float*>(bdx->ptr);
-  if (ci->in_c % 4 == 0 && aligned16(dyf) && aligned16(xf) && aligned16(dxf)) {
+  if (ci->in_c % 4 == 0 && x_n / 4 <= INDEX32 - 256 && aligned16(dyf) && aligned16(xf) && aligned16(dxf)) {
     ctx->name_kernel(
              kind == TFHIP_POOL_MAX ? "max_pool_backprop_vec" : "avg_pool_backprop_vec");
-    tfhip::launch(ctx, pool2d_backprop_vec_kernel, dim3((unsigned)ceil_div(x_n / 4, 256)), dim3(256), 0, dyf, xf, dxf, *ci, kind);
+    tfhip::launch(ctx, pool2d_backprop_vec_kernel, dim3((unsigned)ceil_div(x_n / 4, 256)), dim3(256), 0, dyf, xf, dxf, *ci, kind,
+                  (uint32_t)(x_n / 4), Divisor(ci->in_c / 4), Divisor(ci->in_w), Divisor(ci->in_h),
+                  Divisor(ci->stride_h), Divisor(ci->stride_w));
     TFHIP_LAUNCH_CHECK(ctx);
     return TFHIP_OK;
   }

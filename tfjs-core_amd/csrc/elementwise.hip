@@ -144,13 +144,35 @@ __global__ void binary_f32_vec_kernel(int op, const f32x4* a, const f32x4* b, f3
   }
 }
 
-// float32 [rows, C] (op) float32 [C] with C % 4 == 0: bias add / per-channel prelu.
-__global__ void binary_f32_rowvec_kernel(int op, const f32x4* a, const f32x4* b, f32x4* out,
-                                         int64_t n4, int c4, int b_is_first) {
-  const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n4; i += stride) {
-    const f32x4 x = a[i], y = b[i % c4];
-    f32x4 r;
+// A float32 tensor (op) a small one that repeats along it: bias add, per-channel prelu, a scalar.
+// The large one in 16-byte accesses; VEC: so is the small one (its length is a multiple of 4),
+// otherwise the four elements are found by counting on from one remainder.  Bound by HBM: on
+// [100352, 128] with [128], 25.9 us with a 64-bit remainder per access and 17.0 with this one.
+template <bool VEC>
+__global__ void binary_f32_repeat_kernel(int op, const f32x4* a, const float* b, f32x4* out, uint32_t n4,
+                                         Divisor len, int b_is_first) {
+  const uint32_t stride = gridDim.x * blockDim.x;
+  for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n4; i += stride) {
+    const f32x4 x = a[i];
+    f32x4 y, r;
+    if (VEC) {  // (len counts quads)
+      uint32_t q = i;
+      y = reinterpret_cast<const f32x4*>(b)[len.divmod(q)];
+    } else {
+      // 4 i mod len from i mod len, whose fourfold may pass 2^31: the elements of a quad first
+      uint32_t q = i;
+      uint32_t at = len.divmod(q);
+#pragma unroll
+      for (int d = 0; d < 2; d++) {
+        at += at;
+        if (at >= len.d) at -= len.d;
+      }
+#pragma unroll
+      for (int e = 0; e < 4; e++) {
+        y[e] = b[at];
+        if (++at == len.d) at = 0;
+      }
+    }
 #pragma unroll
     for (int e = 0; e < 4; e++) r[e] = b_is_first ? bin_f(op, y[e], x[e]) : bin_f(op, x[e], y[e]);
     out[i] = r;
@@ -364,14 +386,17 @@ extern "C" int tfhip_binary(tfhip_ctx* ctx, int op, int64_t a, const int32_t* a_
     TFHIP_LAUNCH_CHECK(ctx);
     return TFHIP_OK;
   }
-  const int last = rank ? bc.out_dim[rank - 1] : 1;
-  if (!predicate && all_f32 && !a_bcast && !b_bcast && last % 4 == 0 && aligned16(ba->ptr) &&
-      aligned16(bb->ptr) && aligned16(bo->ptr) &&
-      ((a_len == n && b_len == last) || (b_len == n && a_len == last))) {
-    const bool b_small = b_len == last && a_len == n;
-    tfhip::launch(ctx, binary_f32_rowvec_kernel, dim3(grid_for(ctx, n / 4, block)), dim3(block), 0, op, (const f32x4*)(b_small ? ba->ptr : bb->ptr),
-                       (const f32x4*)(b_small ? bb->ptr : ba->ptr), (f32x4*)bo->ptr, n / 4,
-                       last / 4, b_small ? 0 : 1);
+  if (!predicate && all_f32 && !a_bcast && !b_bcast && (a_len == n || b_len == n) && n % 4 == 0 &&
+      n / 4 <= INDEX32 / 2 && aligned16(ba->ptr) && aligned16(bb->ptr) && aligned16(bo->ptr)) {
+    // (no dimension of either is stretched: the smaller one, of `len` elements, repeats)
+    const bool b_small = a_len == n;
+    const int64_t len = b_small ? b_len : a_len;
+    const f32x4* large = (const f32x4*)(b_small ? ba->ptr : bb->ptr);
+    const float* small = (const float*)(b_small ? bb->ptr : ba->ptr);
+    const bool vec = len % 4 == 0;
+    tfhip::launch(ctx, vec ? binary_f32_repeat_kernel<true> : binary_f32_repeat_kernel<false>,
+                  dim3(grid_for(ctx, n / 4, block)), dim3(block), 0, op, large, small, (f32x4*)bo->ptr,
+                  (uint32_t)(n / 4), Divisor(vec ? len / 4 : len), b_small ? 0 : 1);
     TFHIP_LAUNCH_CHECK(ctx);
     return TFHIP_OK;
   }

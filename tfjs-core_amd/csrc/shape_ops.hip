@@ -34,6 +34,49 @@ __global__ void strided_copy_kernel(const T* __restrict__ x, T* __restrict__ out
   }
 }
 
+// The same where every index fits 32 bits, over the dimensions that are left when those that run
+// on into each other on both sides are one.  Four elements in flight per lane.  Mirroring
+// [16, 480, 640, 3]: 65 us with 64-bit divisions by the four extents, 21.7 with these.
+struct Box32 {
+  int rank;
+  int32_t x_offset, out_offset;
+  Divisor region[MAXBOX];
+  int32_t x_stride[MAXBOX], out_stride[MAXBOX];
+};
+template <typename T>
+__global__ void strided_copy32_kernel(const T* __restrict__ x, T* __restrict__ out, uint32_t n, Box32 b) {
+  constexpr int U = 4;
+  const uint32_t stride = gridDim.x * blockDim.x;
+  for (uint32_t i0 = blockIdx.x * blockDim.x + threadIdx.x; i0 < n; i0 += U * stride) {
+    int32_t src[U], dst[U];
+    uint32_t rem[U];
+    T v[U];
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      rem[u] = i0 + u * stride;
+      src[u] = b.x_offset;
+      dst[u] = b.out_offset;
+    }
+#pragma unroll
+    for (int d = MAXBOX - 1; d >= 0; d--) {
+      if (d < b.rank) {
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+          const int32_t c = (int32_t)b.region[d].divmod(rem[u]);
+          src[u] += c * b.x_stride[d];
+          dst[u] += c * b.out_stride[d];
+        }
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < U; u++)
+      if (i0 + u * stride < n) v[u] = x[src[u]];
+#pragma unroll
+    for (int u = 0; u < U; u++)
+      if (i0 + u * stride < n) out[dst[u]] = v[u];
+  }
+}
+
 __global__ void logical_not_kernel(const uint8_t* x, uint8_t* out, int64_t n) {
   const int64_t stride = (int64_t)gridDim.x * blockDim.x;
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride)
@@ -52,6 +95,29 @@ __global__ void batchnorm_kernel(const float* x, const float* mean, int64_t n_me
     const float s = scale ? scale[i % n_scale] : 1.f;
     const float o = offset ? offset[i % n_off] : 0.f;
     out[i] = o + (x[i] - m) * s / sqrtf(v + eps);
+  }
+}
+
+// The same over [rows, C] with every operand given per channel: the statistics of four channels in
+// 16-byte accesses.  Bound by HBM: [100352, 128] 42 us with four 64-bit remainders per element,
+// 18.0 with one per four.
+typedef float bn_f32x4 __attribute__((ext_vector_type(4)));
+__global__ void batchnorm_channels_kernel(const bn_f32x4* __restrict__ x, const bn_f32x4* __restrict__ mean,
+                                          const bn_f32x4* __restrict__ variance,
+                                          const bn_f32x4* __restrict__ offset,
+                                          const bn_f32x4* __restrict__ scale, float eps,
+                                          bn_f32x4* __restrict__ out, uint32_t n4, Divisor c4) {
+  const uint32_t stride = gridDim.x * blockDim.x;
+  for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n4; i += stride) {
+    uint32_t q = i;
+    const uint32_t c = c4.divmod(q);
+    const bn_f32x4 v = x[i], m = mean[c], var = variance[c];
+    const bn_f32x4 s = scale ? scale[c] : bn_f32x4{1.f, 1.f, 1.f, 1.f};
+    const bn_f32x4 o = offset ? offset[c] : bn_f32x4{0.f, 0.f, 0.f, 0.f};
+    bn_f32x4 r;
+#pragma unroll
+    for (int e = 0; e < 4; e++) r[e] = o[e] + (v[e] - m[e]) * s[e] / sqrtf(var[e] + eps);
+    out[i] = r;
   }
 }
 
@@ -174,6 +240,37 @@ extern "C" int tfhip_strided_copy(tfhip_ctx* ctx, int64_t x, int64_t out, int ra
                      (long long)o_hi, (long long)bo->numel);
   if (bx->ptr == bo->ptr) return ctx->fail(TFHIP_EINVAL, "strided copy: in place is not supported");
   const dim3 grid(grid_for(ctx, n, 256)), block(256);
+  // (indices of the elements in flight past the last one stay below 2^31 too)
+  if (x_hi <= INDEX32 && o_hi <= INDEX32 && n <= INDEX32 - 4LL * 256 * grid.x) {
+    Box32 c = {};
+    c.x_offset = (int32_t)x_offset;
+    c.out_offset = (int32_t)out_offset;
+    int64_t extent[MAXBOX];
+    for (int d = 0; d < rank; d++) {
+      if (region[d] == 1) continue;
+      // an outer dimension whose step is the whole of this one on both sides joins it
+      const int l = c.rank - 1;
+      if (l >= 0 && c.x_stride[l] == x_strides[d] * region[d] && c.out_stride[l] == out_strides[d] * region[d]) {
+        extent[l] *= region[d];
+        c.x_stride[l] = (int32_t)x_strides[d];
+        c.out_stride[l] = (int32_t)out_strides[d];
+        continue;
+      }
+      extent[c.rank] = region[d];
+      c.x_stride[c.rank] = (int32_t)x_strides[d];
+      c.out_stride[c.rank++] = (int32_t)out_strides[d];
+    }
+    for (int d = 0; d < c.rank; d++) c.region[d] = Divisor(extent[d]);
+    const dim3 grid4(grid_for(ctx, ceil_div(n, 4), 256));
+    if (dtype_size(bx->dtype) == 4)
+      tfhip::launch(ctx, strided_copy32_kernel<int32_t>, grid4, block, 0, (const int32_t*)bx->ptr,
+                    (int32_t*)bo->ptr, (uint32_t)n, c);
+    else
+      tfhip::launch(ctx, strided_copy32_kernel<uint8_t>, grid4, block, 0, (const uint8_t*)bx->ptr,
+                    (uint8_t*)bo->ptr, (uint32_t)n, c);
+    TFHIP_LAUNCH_CHECK(ctx);
+    return TFHIP_OK;
+  }
   if (dtype_size(bx->dtype) == 4)
     tfhip::launch(ctx, strided_copy_kernel<int32_t>, grid, block, 0,
                        (const int32_t*)bx->ptr, (int32_t*)bo->ptr, n, b);
@@ -219,6 +316,16 @@ extern "C" int tfhip_batchnorm(tfhip_ctx* ctx, int64_t x, int64_t mean, int64_t 
     return rc;
   if (boff && (rc = as_f32(ctx, boff, &to, &of))) return rc;
   if (bs && (rc = as_f32(ctx, bs, &ts, &sf))) return rc;
+  const int64_t c = bm->numel, n = bx->numel;
+  auto al = [](const void* q) { return (reinterpret_cast<uintptr_t>(q) & 15) == 0; };
+  if (c % 4 == 0 && n % c == 0 && n / 4 <= INDEX32 / 2 && bv->numel == c && (!boff || boff->numel == c) &&
+      (!bs || bs->numel == c) && al(xf) && al(mf) && al(vf) && al(of) && al(sf) && al(bo->ptr)) {
+    tfhip::launch(ctx, batchnorm_channels_kernel, dim3(grid_for(ctx, n / 4, 256)), dim3(256), 0,
+                  (const bn_f32x4*)xf, (const bn_f32x4*)mf, (const bn_f32x4*)vf, (const bn_f32x4*)of,
+                  (const bn_f32x4*)sf, epsilon, (bn_f32x4*)bo->ptr, (uint32_t)(n / 4), Divisor(c / 4));
+    TFHIP_LAUNCH_CHECK(ctx);
+    return TFHIP_OK;
+  }
   tfhip::launch(ctx, batchnorm_kernel, dim3(grid_for(ctx, bx->numel, 256)), dim3(256), 0, xf, mf, bm->numel, vf, bv->numel, of, boff ? boff->numel : 1, sf,
                      bs ? bs->numel : 1, epsilon, (float*)bo->ptr, bx->numel);
   TFHIP_LAUNCH_CHECK(ctx);

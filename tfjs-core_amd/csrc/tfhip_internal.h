@@ -302,6 +302,34 @@ int depthwise_forward_f32(tfhip_ctx* ctx, const float* x, const float* w, float*
 
 inline int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
+// Division of 32-bit indices by a number that is the same for a whole launch: a multiplication and
+// a shift (Granlund and Montgomery, "Division by invariant integers using multiplication", 1994)
+// for 1 <= d < 2^31 and n < 2^31.  The hardware has no integer division: a 32-bit one is some 25
+// instructions, a 64-bit one over a hundred, more than an elementwise kernel has time for.
+struct Divisor {
+  uint32_t d = 1, mul = 1, shift = 0;
+  Divisor() = default;
+  explicit Divisor(int64_t divisor) : d((uint32_t)divisor) {
+    while ((1ull << shift) < d) shift++;
+    mul = (uint32_t)(((1ull << 32) * ((1ull << shift) - d)) / d + 1);
+  }
+  __host__ __device__ __forceinline__ uint32_t quotient(uint32_t n) const {
+#ifdef __HIP_DEVICE_COMPILE__
+    const uint32_t hi = __umulhi(n, mul);
+#else
+    const uint32_t hi = (uint32_t)(((uint64_t)n * mul) >> 32);
+#endif
+    return (hi + n) >> shift;
+  }
+  // n becomes the quotient, the remainder is returned
+  __host__ __device__ __forceinline__ uint32_t divmod(uint32_t& n) const {
+    const uint32_t q = quotient(n), r = n - q * d;
+    n = q;
+    return r;
+  }
+};
+constexpr int64_t INDEX32 = 0x7fffffff;  // what such indices may go up to
+
 // Every kernel of the library is launched through here, on the context's stream.  The
 // arguments are converted to the kernel's parameter types as a <<<>>> launch would.  Inside a
 // time() region the launch carries its own start / stop events.
