@@ -1,0 +1,139 @@
+"""Products whose float32 operands are split into three bf16 parts for the matrix cores, at the edges
+of their tiles, against the same contraction in float64."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def tf():
+    import tfhip as tf
+    tf.set_backend("hip")
+    return tf
+
+
+def _kernel(tf):
+    be = tf.backend()
+    return be.lib.tfhip_last_kernel(be.ctx).decode()
+
+
+def _bound(k, magnitude):
+    """Every 16 k of a sum are rounded once in float32 (2^-24 of a partial sum, which the sum of the
+    products' magnitudes bounds), the products that are left out are below 2^-22 of theirs, and a
+    block, a cut along K and the bias add a few roundings more."""
+    return (k / 16.0 + 16) * 2.0 ** -24 * magnitude
+
+
+def _check(got, want, magnitude, k):
+    bound = _bound(k, magnitude)
+    worst = np.max(np.abs(got - want) - bound)
+    assert worst <= 0, (worst, np.abs(got - want).max())
+
+
+@pytest.mark.parametrize("batch,m,k,n,ta,tb", [
+    (1, 2048, 1024, 1024, True, False), (1, 2051, 783, 1027, True, True),   # odd: element-wise loads
+    (1, 2048, 260, 1000, False, True), (1, 1500, 1036, 1284, False, True),  # K and N past a tile
+    (1, 4096, 20, 4100, True, True), (1, 2052, 16, 2044, True, False),     # one step and a little
+    (1, 128, 4096, 4096, True, False),                                     # cut along K, summed in blocks
+    (96, 300, 50, 300, False, False), (40, 301, 67, 203, False, True), (3, 1000, 700, 640, True, False),
+])
+def test_matmul(tf, batch, m, k, n, ta, tb):
+    print("split matmul", batch, m, k, n, ta, tb, flush=True)
+    rng = np.random.default_rng(m + 3 * k + 7 * n)
+    a = rng.uniform(-1, 1, (batch, k, m) if ta else (batch, m, k)).astype(np.float32)
+    b = (rng.standard_normal((batch, n, k) if tb else (batch, k, n)) * 10).astype(np.float32)
+    with tf.tidy():
+        got = tf.matmul(tf.tensor(a), tf.tensor(b), ta, tb).data_sync().astype(np.float64)
+        assert _kernel(tf).startswith("gemm_split_"), _kernel(tf)
+    a64 = a.astype(np.float64).transpose(0, 2, 1) if ta else a.astype(np.float64)
+    b64 = b.astype(np.float64).transpose(0, 2, 1) if tb else b.astype(np.float64)
+    _check(got, a64 @ b64, np.abs(a64) @ np.abs(b64), k)
+
+
+@pytest.mark.parametrize("m,k,n,ta,tb", [(2100, 1024, 1030, True, False), (4100, 300, 1100, False, True)])
+def test_values_that_bf16_parts_do_not_hold(tf, m, k, n, ta, tb):
+    """Infinities, NaN, values next to the largest and rows of tiny ones: as in float32."""
+    rng = np.random.default_rng(k)
+    a = rng.uniform(0.5, 1, (m, k)).astype(np.float32)
+    b = rng.uniform(-1, 1, (k, n)).astype(np.float32)
+    a[3, 5], a[300, 80], a[500, 7] = np.inf, np.nan, 3.4e38
+    a[700] *= np.float32(1e-36)     # below 2^-110: part of the bf16 parts would vanish
+    a[800] = 0
+    b[11, 200] = -np.inf
+    b[7] *= np.float32(0.01)        # (3.4e38 times it is finite)
+    with tf.tidy():
+        got = tf.matmul(tf.tensor(np.ascontiguousarray(a.T) if ta else a),
+                        tf.tensor(np.ascontiguousarray(b.T) if tb else b), ta, tb).data_sync()
+        assert _kernel(tf).startswith("gemm_split_"), _kernel(tf)
+    a64, b64 = a.astype(np.float64), b.astype(np.float64)
+    with np.errstate(invalid="ignore"):
+        want = a64 @ b64
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    assert np.array_equal(np.isposinf(got), np.isposinf(want)) and np.array_equal(np.isneginf(got), np.isneginf(want))
+    assert not got[800, np.isfinite(want[800])].any()
+    fin = np.isfinite(want)
+    magnitude = np.abs(np.nan_to_num(a64, posinf=0)) @ np.abs(np.nan_to_num(b64, neginf=0))
+    # (a tile that holds such a value is summed in float32, once per two k)
+    assert np.all(np.abs(np.where(fin, got - np.where(fin, want, 0), 0)) <= (k / 2 + 16) * 2.0 ** -24 * magnitude)
+
+
+def _conv64(x, w, stride, dil, pad, oh, ow):
+    p = np.pad(x, ((0, 0), (pad[0], pad[0] + 64), (pad[1], pad[1] + 64), (0, 0)))
+    y = 0
+    for i in range(w.shape[0]):
+        for j in range(w.shape[1]):
+            r, c = i * dil, j * dil
+            y = y + p[:, r:r + (oh - 1) * stride + 1:stride, c:c + (ow - 1) * stride + 1:stride] @ w[i, j]
+    return y
+
+
+@pytest.mark.parametrize("n,h,w,cin,cout,f,stride,dil", [
+    (8, 33, 47, 64, 136, 3, 1, 1), (16, 29, 31, 20, 200, 5, 1, 1),   # Cin above and off the step of 16
+    (48, 56, 40, 36, 96, 3, 2, 1), (16, 40, 41, 32, 128, 3, 1, 3), (320, 7, 9, 96, 128, 3, 1, 1),
+    (64, 31, 30, 4, 132, 5, 1, 1),                                   # four taps in a step
+])
+def test_conv2d_and_its_gradients(tf, n, h, w, cin, cout, f, stride, dil):
+    """The convolution, whose loader walks the taps by additions, and the gradients, which are split."""
+    print("split conv", n, h, w, cin, cout, f, stride, dil, flush=True)
+    rng = np.random.default_rng(n + h + cin + cout)
+    x = rng.standard_normal((n, h, w, cin)).astype(np.float32)
+    wt = rng.standard_normal((f, f, cin, cout)).astype(np.float32)
+    bias = rng.standard_normal(cout).astype(np.float32)
+    oh, ow = -(-h // stride), -(-w // stride)
+    eff = (f - 1) * dil + 1
+    pad = (max((oh - 1) * stride + eff - h, 0) // 2, max((ow - 1) * stride + eff - w, 0) // 2)
+    x64, w64 = x.astype(np.float64), wt.astype(np.float64)
+    with tf.tidy():
+        got = tf.fused.conv2d(tf.tensor(x), tf.tensor(wt), stride, "same", dilations=dil, bias=tf.tensor(bias),
+                              activation="relu").data_sync()
+        assert "im2col" in _kernel(tf), _kernel(tf)
+    want = _conv64(x64, w64, stride, dil, pad, oh, ow) + bias
+    magnitude = _conv64(np.abs(x64), np.abs(w64), stride, dil, pad, oh, ow) + np.abs(bias)
+    _check(got, np.maximum(want, 0), magnitude, f * f * cin * 8)   # (in float32: rounded once per two k)
+    if dil > 1:
+        return
+    dy = rng.standard_normal((n, oh, ow, cout)).astype(np.float32)
+    d64 = dy.astype(np.float64)
+    with tf.tidy():
+        dw = tf.conv2d_der_filter(tf.tensor(x), tf.tensor(dy), wt.shape, stride, "same").data_sync()
+        kernel_w = _kernel(tf)
+        dx = tf.conv2d_der_input(x.shape, tf.tensor(dy), tf.tensor(wt), stride, "same").data_sync()
+        kernel_x = _kernel(tf)
+    assert kernel_w.startswith("gemm_split_"), kernel_w
+    assert stride > 1 or kernel_x.startswith("gemm_split_"), kernel_x
+    for i in range(f):
+        for j in range(f):
+            p = np.pad(x64, ((0, 0), (pad[0], pad[0] + 64), (pad[1], pad[1] + 64), (0, 0)))
+            part = p[:, i:i + (oh - 1) * stride + 1:stride, j:j + (ow - 1) * stride + 1:stride].reshape(-1, cin).T
+            flat = d64.reshape(-1, cout)
+            _check(dw[i, j], part @ flat, np.abs(part) @ np.abs(flat), n * oh * ow)
+    want, magnitude = np.zeros((n, h + 2 * f, w + 2 * f, cin)), np.zeros((n, h + 2 * f, w + 2 * f, cin))
+    for i in range(f):
+        for j in range(f):
+            at = (slice(None), slice(i, i + (oh - 1) * stride + 1, stride), slice(j, j + (ow - 1) * stride + 1, stride))
+            want[at] += d64 @ w64[i, j].T
+            magnitude[at] += np.abs(d64) @ np.abs(w64[i, j].T)
+    inside = (slice(None), slice(pad[0], pad[0] + h), slice(pad[1], pad[1] + w))
+    # (the float32 gather of a strided layer rounds once per two k)
+    _check(dx, want[inside], magnitude[inside], f * f * cout * (1 if stride == 1 else 8))
