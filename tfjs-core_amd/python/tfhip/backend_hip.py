@@ -17,8 +17,12 @@ _NP_OF_CODE = {capi.FLOAT32: np.float32, capi.INT32: np.int32, capi.BOOL: np.uin
                capi.UINT8Q: np.uint8}
 
 
+_SHAPE_ARRAYS = [C.c_int32 * max(1, n) for n in range(9)]  # (making an array type costs more than an array)
+
+
 def _shape_arr(shape):
-    return (C.c_int32 * max(1, len(shape)))(*shape)
+    n = len(shape)
+    return (_SHAPE_ARRAYS[n] if n < 9 else C.c_int32 * n)(*shape)
 
 
 def _info_c(ci):

@@ -21,7 +21,7 @@ class Tensor(object):
 
     def __init__(self, shape, dtype, data_id=None, values=None, backend=None, quant=None,
                  storage_dtype=None):
-        self.shape = tuple(int(d) for d in shape)
+        self.shape = tuple(map(int, shape))
         self.dtype = dtype or "float32"
         self.size = su.size_from_shape(self.shape)
         self.rank = len(self.shape)
@@ -156,11 +156,10 @@ class Engine(object):
         rec = self.ref.get(t.data_id)
         if rec is None:
             nbytes = t.size * (1 if storage_dtype in ("bool", "uint8q") else 4)
-            self.ref[t.data_id] = [0, backend, nbytes]
+            rec = self.ref[t.data_id] = [0, backend, nbytes]
             self.num_data_buffers += 1
             self.num_bytes += nbytes
             backend.register(t.data_id, t.shape, storage_dtype)
-            rec = self.ref[t.data_id]
         rec[0] += 1
         self.num_tensors += 1
         if self.scopes:
@@ -200,12 +199,17 @@ class Engine(object):
         self.scopes.append([])
 
     def end_scope(self, result=None):
-        keep = set(id(t) for t in _flatten_tensors(result))
         scope = self.scopes.pop()
+        if not scope:
+            return
+        # (one tensor is what nearly every operation returns)
+        keep = (result,) if isinstance(result, Tensor) else _flatten_tensors(result)
+        keep = {id(t) for t in keep}
+        outer = self.scopes[-1] if self.scopes else None
         for t in scope:
             if id(t) in keep:
-                if self.scopes:
-                    self.scopes[-1].append(t)
+                if outer is not None:
+                    outer.append(t)
             elif not t.is_disposed:
                 t.dispose()
 
@@ -231,10 +235,10 @@ class Engine(object):
     def run_kernel(self, forward):
         """ENGINE.runKernel without a tape (engine.ts:435-498): the forward function gets the
         active backend; intermediates made inside are released when it returns."""
-        self.start_scope()
+        self.scopes.append([])
         result = None
         try:
-            result = forward(self.backend)
+            result = forward(self._backend or self.backend)
             return result
         finally:
             self.end_scope(result)

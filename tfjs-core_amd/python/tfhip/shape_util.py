@@ -120,6 +120,8 @@ def compute_pool2d_info(in_shape, filter_size, strides, dilations, pad, rounding
 
 
 def broadcast_shape(shape_a, shape_b):
+    if shape_a == shape_b:
+        return tuple(shape_a)
     result = []
     n = max(len(shape_a), len(shape_b))
     for i in range(n):
