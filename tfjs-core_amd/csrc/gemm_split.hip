@@ -21,7 +21,7 @@
 // LDS layout.  Per operand three planes (h, m, l) of [k / 8][slot][8 bf16]: the matrix instruction
 // takes 8 consecutive k of a row per lane, and 32 lanes read 512 consecutive bytes.  A slot is a
 // row of A or a column of B; where the operand lies with rows (columns) contiguous in memory a
-// thread takes 4 k x 4 rows and turns them around in registers, and the slots of 64 rows are
+// thread takes 2 k x 4 rows and turns them around in registers, and the slots of 64 rows are
 // dealt so that the 4 rows of a thread go to 4 runs of 16 slots (see slot_of): without that the
 // writes of a wavefront would meet in a quarter of the banks.
 //
@@ -102,7 +102,10 @@ struct Staging {
 // total, always downwards: measured with K = 256 signed values, 1.4e-7 relative with a bias of
 // -6e-9 against 0.8e-7 without one.)  BLOCKED > 0: `hi` starts from zero every BLOCKED steps and
 // joins a total of its own, for sums so long that one rounding per 16 k of the whole would be
-// more than the two-level sum of the float32 kernels shows.
+// more than the two-level sum of the float32 kernels shows.  Measured against 64 bits, float32
+// kernels and these: matMul of signed values with K = 128 1.25e-7 and 0.62e-7, 1024 1.54e-7 and
+// 0.83e-7 (1.63e-7 without blocks), 4096 2.1e-7 and 1.2e-7; of positive ones 0.69 and 0.62, 0.72
+// and 0.56, 1.26 and 0.82; gradients of convolutions 2.2e-7 to 7.1e-7 and 1.1e-7 to 2.3e-7.
 template <class T, int AMODE, int BMODE, int BLOCKED, bool VEC>
 __global__ __launch_bounds__(T::THREADS, 2) void gemm_split_kernel(const GemmArgs p) {
   constexpr int BM = T::BM, BN = T::BN, TM = T::TM, TN = T::TN, THREADS = T::THREADS;
@@ -114,7 +117,6 @@ __global__ __launch_bounds__(T::THREADS, 2) void gemm_split_kernel(const GemmArg
   constexpr int BUF = 3 * SA::PLANE + 3 * SB::PLANE;
   __shared__ __attribute__((aligned(16))) char lds[2 * BUF];
   static_assert(BM * 64 + BN * 64 <= BUF, "room for float32 operands");
-  __shared__ float lut[BMODE == B_UINT8 ? 256 : 1];  // what the codes stand for
   __shared__ int redo_of[T::WM * T::WN];
 
   const int tid = threadIdx.x;
@@ -122,10 +124,6 @@ __global__ __launch_bounds__(T::THREADS, 2) void gemm_split_kernel(const GemmArg
   const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave / T::WN, wn = wave % T::WN;
   const int l32 = lane & 31, g = lane >> 5;
-  if (BMODE == B_UINT8) {
-    for (int i = tid; i < 256; i += THREADS) lut[i] = dequant((unsigned)i, p.qscale, p.qmin);
-    __syncthreads();
-  }
 
   const WorkItem cur = work_item(p, blockIdx.x);
   if (cur.tile < 0) return;
@@ -135,8 +133,7 @@ __global__ __launch_bounds__(T::THREADS, 2) void gemm_split_kernel(const GemmArg
   tile_row_col(p, cur.tile - batch * tiles_per_batch, tm, tn);
   const int bm0 = tm * BM, bn0 = tn * BN;
   const __amdgpu_buffer_rsrc_t ra = make_rsrc(p.A + batch * p.strideA, p.a_bytes);
-  const __amdgpu_buffer_rsrc_t rb = make_rsrc(
-      static_cast<const char*>(p.B) + batch * p.strideB * (BMODE == B_UINT8 ? 1 : 4), p.b_bytes);
+  const __amdgpu_buffer_rsrc_t rb = make_rsrc(static_cast<const float*>(p.B) + batch * p.strideB, p.b_bytes);
 
   // ---- what this thread stages ----
   unsigned a_at[SA::PER], b_at[SB::PER];  // byte offset of the item at k = 0; OOB_OFFSET: no such row
@@ -147,7 +144,6 @@ __global__ __launch_bounds__(T::THREADS, 2) void gemm_split_kernel(const GemmArg
   int g_inner = 0, g_middle = 0, g_row = 0, g_col = 0;
   unsigned g_at = 0;
   int k_next = 0;
-  constexpr unsigned B_EL = BMODE == B_UINT8 ? 1 : 4;
   auto setup = [&]() {
     k_next = cur.kt0 * SK;
 #pragma unroll
@@ -194,7 +190,7 @@ __global__ __launch_bounds__(T::THREADS, 2) void gemm_split_kernel(const GemmArg
     for (int i = 0; i < SB::PER; i++) {
       const int col = bn0 + (B_KC ? row_of(SB::row(tid, i)) : SB::row(tid, i));
       const bool ok = col < p.N;
-      b_at[i] = ok ? (B_KC ? (unsigned)col * p.ldb + SB::k(tid, 0) : (unsigned)SB::k(tid, i) * p.ldb + col) * B_EL
+      b_at[i] = ok ? (B_KC ? (unsigned)col * p.ldb + SB::k(tid, 0) : (unsigned)SB::k(tid, i) * p.ldb + col) * 4u
                    : OOB_OFFSET;
     }
   };
@@ -267,13 +263,7 @@ __global__ __launch_bounds__(T::THREADS, 2) void gemm_split_kernel(const GemmArg
       for (int i = 0; i < SB::PER; i++) {
         const int left = p.N - bn0 - SB::row(tid, i);
 #pragma unroll
-        for (int e = 0; e < 2; e++) {
-          const int base = (k0 + e) * p.ldb * (int)B_EL;
-          if (BMODE == B_UINT8)
-            o.b[2 * i + e][0] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rb, (int)b_at[i], base, 0));
-          else
-            o.b[2 * i + e] = load4(rb, b_at[i], base, left);
-        }
+        for (int e = 0; e < 2; e++) o.b[2 * i + e] = load4(rb, b_at[i], (k0 + e) * p.ldb * 4, left);
       }
     }
   };
@@ -359,18 +349,6 @@ __global__ __launch_bounds__(T::THREADS, 2) void gemm_split_kernel(const GemmArg
       }
     }
   };
-  // uint8 weights: codes into values.  (A code that was not read is 0 and stands for a finite
-  // weight: items at or beyond K of A are zero, and columns at or beyond N are not stored.)
-  auto decode = [&](Raw& o) {
-    if (BMODE != B_UINT8) return;
-#pragma unroll
-    for (int i = 0; i < SB::REGS; i++) {
-      const unsigned w = __builtin_bit_cast(unsigned, o.b[i][0]);
-#pragma unroll
-      for (int e = 0; e < 4; e++) o.b[i][e] = lut[(w >> (8 * e)) & 0xffu];
-    }
-  };
-
   f32x16 hi[TM][TN], lo[TM][TN], total[TM][TN];
   const f32x16 zero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
   auto clear = [&](f32x16 (&sum)[TM][TN]) {
@@ -426,7 +404,6 @@ __global__ __launch_bounds__(T::THREADS, 2) void gemm_split_kernel(const GemmArg
       advance();
       read(buf, 1, fm);
       read(buf, 2, fl);
-      decode(raw);
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int n = 0; n < BEFORE; n++) {
@@ -447,7 +424,6 @@ __global__ __launch_bounds__(T::THREADS, 2) void gemm_split_kernel(const GemmArg
     Frags f0, f1;
     load(raw);
     advance();
-    decode(raw);
 #pragma unroll
     for (int t = 0; t < A_PIECES + B_PIECES; t++) stage_piece(lds, raw, t);
     load(raw);
@@ -494,8 +470,7 @@ __global__ __launch_bounds__(T::THREADS, 2) void gemm_split_kernel(const GemmArg
       for (int kt = cur.kt0; kt < cur.kt1; kt++) {
         load(raw);
         advance();
-        decode(raw);
-        put_exact(SA(), lds, raw.a);
+          put_exact(SA(), lds, raw.a);
         put_exact(SB(), lds + BM * 64, raw.b);
         __syncthreads();
 #pragma unroll
@@ -670,7 +645,7 @@ static double float32_cost(const GemmArgs& p, int batch, int cus, int amode, int
 template <class T, int AMODE, int BMODE, int BLOCKED, bool VEC>
 static int launch_cfg(tfhip_ctx* ctx, GemmArgs p, const SplitPlan& pl) {
   static const char* const a_names[] = {"rowmajor", "transposed", "im2col", "im2col_up", "im2col_t"};
-  static const char* const b_names[] = {"f32", "f32t", "u8"};
+  static const char* const b_names[] = {"f32", "f32t"};
   ctx->name_kernel("gemm_split_%dx%d_%s_%s%s%s", T::BM, T::BN, a_names[AMODE], b_names[BMODE],
                    VEC ? "" : "_unaligned", pl.splits > 1 ? pl.full ? "_tailk" : "_splitk" : "");
   p.tiles_m = pl.tiles_m;
@@ -751,7 +726,7 @@ int launch_split(tfhip_ctx* ctx, const GemmArgs& q, int batch, int amode, int bm
     amode = A_IM2COL;
   }
   const bool vec = q.a_vec && q.b_vec;
-  if (!vec && (amode == A_IM2COL || amode == A_IM2COL_T || bmode == B_UINT8)) return -1;
+  if (bmode == B_UINT8 || (!vec && (amode == A_IM2COL || amode == A_IM2COL_T))) return -1;
   GemmArgs p = q;
   p.a_bytes = (unsigned)a_bytes;
   p.b_bytes = (unsigned)b_bytes;
