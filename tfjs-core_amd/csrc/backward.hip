@@ -474,10 +474,12 @@ extern "C" int tfhip_depthwise_conv2d_der_filter(tfhip_ctx* ctx, int64_t x, int6
     while (qpw < 64 && qpw < c4) qpw *= 2;
     const int64_t blocks_c = ceil_div(c4, qpw);
     const int subs = 256 / qpw;
-    // two workgroups per CU, and at least 32 pixels per lane so that the reduction through
-    // LDS and the partial sums stay a small part of the work
+    // two workgroups per CU, and at least 8 pixels per lane.  A lane's pixels are a chain of loads
+    // of about 0.8 us each, which a layer with fewer of them is bound by: [8, 14, 14, 512] 25.4 us
+    // with at least 32 pixels, 12.8 with 8 (16.9 with 16); [64, 28, 28, 256] stride 2 32.9 -> 19.8,
+    // [32, 56, 56, 128] 39.0 -> 36.6 (40.0 with four workgroups per CU: more partial sums).
     int64_t slices = ceil_div((int64_t)ctx->num_cus * 2, blocks_c);
-    if (slices > ceil_div(pixels, (int64_t)subs * 32)) slices = ceil_div(pixels, (int64_t)subs * 32);
+    if (slices > ceil_div(pixels, (int64_t)subs * 8)) slices = ceil_div(pixels, (int64_t)subs * 8);
     if (slices < 1) slices = 1;
     if (slices > 65535) slices = 65535;
     const int64_t per_slice = ceil_div(pixels, slices);
