@@ -137,3 +137,65 @@ def test_conv2d_and_its_gradients(tf, n, h, w, cin, cout, f, stride, dil):
     inside = (slice(None), slice(pad[0], pad[0] + h), slice(pad[1], pad[1] + w))
     # (the float32 gather of a strided layer rounds once per two k)
     _check(dx, want[inside], magnitude[inside], f * f * cout * (1 if stride == 1 else 8))
+
+
+def _float32_bound(k, magnitude):
+    """A tile that holds a value the bf16 parts do not is summed in float32, once per two k; a product
+    that is denormal is rounded to a multiple of 2^-149."""
+    return (k / 2 + 16) * 2.0 ** -24 * magnitude + k * 2.0 ** -149
+
+
+@pytest.mark.parametrize("batch,m,k,n,ta,tb", [
+    (1, 2048, 1024, 1024, True, False), (1, 4096, 64, 4096, True, False),  # 64 x 128 and 128 x 128 tiles
+    (1, 128, 4096, 4096, True, False), (1, 2051, 783, 1027, True, True),   # cut along K; element-wise loads
+    (40, 301, 67, 203, False, True), (96, 300, 50, 300, False, False),
+])
+def test_small_operands_against_large_ones(tf, batch, m, k, n, ta, tb):
+    """The last parts of a value below 2^-110 are none that bf16 holds, whatever it is multiplied with."""
+    print("split small operands", batch, m, k, n, ta, tb, flush=True)
+    rng = np.random.default_rng(m + k + n)
+    a = rng.uniform(-1, 1, (batch, m, k)).astype(np.float32)
+    b = rng.uniform(-1, 1, (batch, k, n)).astype(np.float32)
+    scaled = lambda x, e: (x.astype(np.float64) * 2.0 ** e).astype(np.float32)
+    for row, e in ((0, -112), (m // 2, -120), (m - 1, -140)):
+        a[-1, row] = scaled(a[-1, row], e)
+    a[0, 5, 0] = 2.0 ** -130                       # one such value among ordinary ones
+    for col, e in ((0, 60), (n // 2, 100), (n - 1, 20)):
+        b[-1, :, col] = scaled(b[-1, :, col], e)
+    b[0, 0, 3] = 2.0 ** 120
+    with tf.tidy():
+        got = tf.matmul(tf.tensor(a.transpose(0, 2, 1).copy() if ta else a),
+                        tf.tensor(b.transpose(0, 2, 1).copy() if tb else b), ta, tb).data_sync().astype(np.float64)
+        assert _kernel(tf).startswith("gemm_split_"), _kernel(tf)
+    a64, b64 = a.astype(np.float64), b.astype(np.float64)
+    worst = np.max(np.abs(got - a64 @ b64) / _float32_bound(k, np.abs(a64) @ np.abs(b64)))
+    assert worst <= 1, worst
+
+
+@pytest.mark.parametrize("n,h,w,cin,cout", [(8, 33, 47, 64, 136), (320, 7, 9, 96, 128)])
+def test_small_operands_against_large_ones_in_gathers(tf, n, h, w, cin, cout):
+    print("split small operands, gradients", n, h, w, cin, cout, flush=True)
+    rng = np.random.default_rng(n + cin)
+    x, dy = (rng.standard_normal((n, h, w, c)).astype(np.float32) for c in (cin, cout))
+    wt = rng.standard_normal((3, 3, cin, cout)).astype(np.float32)
+    x[..., 1] *= np.float32(2.0 ** -122)
+    dy[..., 2] *= np.float32(2.0 ** 60)
+    with tf.tidy():
+        dw = tf.conv2d_der_filter(tf.tensor(x), tf.tensor(dy), wt.shape, 1, "same").data_sync()
+        assert _kernel(tf).startswith("gemm_split_"), _kernel(tf)
+    p = np.pad(x.astype(np.float64), ((0, 0), (1, 1), (1, 1), (0, 0)))
+    flat = dy.reshape(-1, cout).astype(np.float64)
+    for i in range(3):
+        for j in range(3):
+            part = p[:, i:i + h, j:j + w].reshape(-1, cin).T
+            assert np.all(np.abs(dw[i, j] - part @ flat) <= _float32_bound(n * h * w, np.abs(part) @ np.abs(flat)))
+    dy[..., 2] *= np.float32(2.0 ** -60)
+    dy[0] *= np.float32(2.0 ** -122)
+    wt[:, :, 3] *= np.float32(2.0 ** 60)
+    with tf.tidy():
+        dx = tf.conv2d_der_input(x.shape, tf.tensor(dy), tf.tensor(wt), 1, "same").data_sync()
+        assert _kernel(tf).startswith("gemm_split_"), _kernel(tf)
+    back = np.ascontiguousarray(wt[::-1, ::-1].transpose(0, 1, 3, 2)).astype(np.float64)
+    d64 = dy.astype(np.float64)
+    want, magnitude = _conv64(d64, back, 1, 1, (1, 1), h, w), _conv64(np.abs(d64), np.abs(back), 1, 1, (1, 1), h, w)
+    assert np.all(np.abs(dx - want) <= _float32_bound(9 * cout, magnitude))
