@@ -200,3 +200,34 @@ def test_shape_op_wrappers_validate_before_the_backend():
     assert ops.strided_slice_info([2, 3], [1, -1], [2, -4], [2, -1])[:2] == ([1, 2], [1, 3])
     assert ops.strided_slice_info([2, 3, 1, 2], [1, 0, 0, 0], [2, 3, 1, 2], [1, 1])[:2] == (
         [1, 0, 0, 0], [1, 3, 1, 2])
+
+
+@pytest.mark.parametrize("axes", [[0, 0, 2], [0, 2, 2], [2, 0, 2], [-3, 0, 2]])
+def test_repeated_axes_are_not_a_block(axes):
+    """An axis that is given twice next to one that is left out: refused, on every path."""
+    import numpy as np
+    import tfhip
+    from tfhip.engine import ENGINE
+    blocks = []
+
+    class Blocks(FakeBackend):
+        def reduce_block(self, op, x, axes, divisor=1.0):
+            blocks.append(axes)
+            shape = x.shape[:axes[0]] + x.shape[axes[-1] + 1:]
+            return tfhip.engine.Tensor(shape, x.dtype, None, np.zeros(shape, np.float32), self)
+
+    tfhip.register_backend("fake-block-test", Blocks, 0)
+    prev = ENGINE.backend_name
+    try:
+        tfhip.set_backend("fake-block-test")
+        x = tfhip.tensor(np.zeros((2, 3, 4), np.float32))
+        for op in (tfhip.sum, tfhip.mean, tfhip.max, tfhip.min, tfhip.prod, tfhip.any, tfhip.all):
+            with pytest.raises(Exception):
+                op(x, axes)
+        assert not blocks
+        tfhip.sum(x, [1, 0])
+        assert blocks == [[0, 1]]
+    finally:
+        tfhip.remove_backend("fake-block-test")
+        if prev:
+            ENGINE.set_backend(prev)

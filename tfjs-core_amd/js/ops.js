@@ -837,13 +837,13 @@ const clipByValue = op('clipByValue', (x, clipValueMin, clipValueMax) => {
 const relu6 = op('relu6', x => clipByValue(x, 0, 6));
 
 // ---- reductions -------------------------------------------------------------------------
-// The axes in ascending order when they are neighbours, else null.  Backends with `reduceBlock`
-// (feature detection) reduce such axes where they are; for the others, and for axes that are
-// apart, the axes are brought innermost first, as the reference does.
+// The axes in ascending order when they are neighbours, none of them twice, else null.
+// Backends with `reduceBlock` (feature detection) reduce such axes where they are; for the others,
+// and for axes that are apart, the axes are brought innermost first, as the reference does.
 function axisBlock(axes) {
   if (axes.length === 0 || typeof ENGINE.backend.reduceBlock !== 'function') return null;
   const sorted = axes.slice().sort((a, b) => a - b);
-  return sorted[sorted.length - 1] - sorted[0] === sorted.length - 1 ? sorted : null;
+  return sorted.every((a, i) => a === sorted[0] + i) ? sorted : null;
 }
 
 function reduceOp(name, method) {

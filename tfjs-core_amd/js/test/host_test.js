@@ -102,6 +102,31 @@ test('MobileNet stem: same padding on even input puts the pad at bottom/right', 
   assert.deepStrictEqual(dw.outShape, [1, 56, 56, 64]);
 });
 
+test('an axis given twice next to one left out is no block of axes', async () => {
+  const blocks = [];
+  class Blocks extends StorageBackend {
+    reduceBlock(op, x, axes) {
+      blocks.push(axes);
+      const shape = x.shape.slice(0, axes[0]).concat(x.shape.slice(axes[axes.length - 1] + 1));
+      const out = Tensor.make(shape, {}, x.dtype, this);
+      this.write(out.dataId, new Float32Array(out.size));
+      return out;
+    }
+  }
+  await withBackend('block-test', new Blocks(), () => {
+    tf.tidy(() => {
+      const x = tf.tensor(new Float32Array(24), [2, 3, 4]);
+      [[0, 0, 2], [0, 2, 2], [2, 0, 2], [-3, 0, 2]].forEach(axes => {
+        [tf.sum, tf.mean, tf.max, tf.min, tf.prod].forEach(op => assert.throws(() => op(x, axes)));
+        [tf.any, tf.all].forEach(op => assert.throws(() => op(tf.tensor([1, 0], [1, 1, 2], 'bool'), axes)));
+      });
+      assert.deepStrictEqual(blocks, []);
+      tf.sum(x, [1, 0]);
+      assert.deepStrictEqual(blocks, [[0, 1]]);
+    });
+  });
+});
+
 test('broadcast and axis helpers', () => {
   const bu = tf.backend_util;
   assert.deepStrictEqual(bu.assertAndGetBroadcastShape([2, 1], [1, 3]), [2, 3]);

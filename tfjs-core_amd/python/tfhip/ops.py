@@ -443,11 +443,11 @@ def relu6(x):
 
 # ---- reductions (ops/reduction_ops.ts) ----
 def _axis_block(axes):
-    """The axes in ascending order when they are neighbours, else None.  Backends with
-    `reduce_block` (feature detection) reduce such axes where they are; for the others, and for
-    axes that are apart, the axes are brought innermost first, as the reference does."""
+    """The axes in ascending order when they are neighbours, none of them twice, else None.
+    Backends with `reduce_block` (feature detection) reduce such axes where they are; for the
+    others, and for axes that are apart, the axes are brought innermost first, as the reference does."""
     axes = sorted(axes)
-    if axes and axes[-1] - axes[0] == len(axes) - 1 and hasattr(ENGINE.backend, "reduce_block"):
+    if axes and axes == list(range(axes[0], axes[0] + len(axes))) and hasattr(ENGINE.backend, "reduce_block"):
         return axes
     return None
 
