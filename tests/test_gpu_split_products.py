@@ -139,6 +139,23 @@ def test_conv2d_and_its_gradients(tf, n, h, w, cin, cout, f, stride, dil):
     _check(dx, want[inside], magnitude[inside], f * f * cout * (1 if stride == 1 else 8))
 
 
+@pytest.mark.parametrize("k", [1, 2, 3, 4])
+@pytest.mark.parametrize("batch,m,n,ta,tb", [(1, 2048, 2048, True, False), (64, 512, 512, False, False),
+                                             (96, 201, 201, False, True)])
+def test_sums_of_few_products_are_rounded_once_each(tf, batch, m, n, ta, tb, k):
+    """Where the parts left out would show: an outer product is the rounded product of its factors."""
+    print("few products", batch, m, k, n, ta, tb, flush=True)
+    rng = np.random.default_rng(m + k)
+    a, b = rng.uniform(-1, 1, (batch, m, k)).astype(np.float32), rng.uniform(-1, 1, (batch, k, n)).astype(np.float32)
+    with tf.tidy():
+        got = tf.matmul(tf.tensor(a.transpose(0, 2, 1).copy() if ta else a),
+                        tf.tensor(b.transpose(0, 2, 1).copy() if tb else b), ta, tb).data_sync()
+    if k == 1:
+        np.testing.assert_array_equal(got, a * b)
+    a64, b64 = a.astype(np.float64), b.astype(np.float64)
+    assert np.all(np.abs(got - a64 @ b64) <= k * 2.0 ** -24 * (np.abs(a64) @ np.abs(b64)))
+
+
 def _float32_bound(k, magnitude):
     """A tile that holds a value the bf16 parts do not is summed in float32, once per two k; a product
     that is denormal is rounded to a multiple of 2^-149."""

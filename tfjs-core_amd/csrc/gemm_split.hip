@@ -4,7 +4,7 @@
 // rounded to 8, and what then remains has at most 8 bits left, which is l.  bf16 has the
 // exponents of float32, and the product of two bf16 values is exact in float32, so
 //   a * b = ah bh + (ah bm + am bh) + (ah bl + am bm + al bh)
-// up to terms of 2^-24 of it and of either sign.  Six bf16 matrix instructions (32 x 32 x 16, 1024
+// up to terms below 2^-22 of it and of either sign.  Six bf16 matrix instructions (32 x 32 x 16, 1024
 // flop per clock and SIMD) then do what eight float32 ones (32 x 32 x 2, 64 flop per clock) do.
 //
 // Kernel shape.  WM x WN wavefronts own a BM x BN tile, each TM x 2 accumulators of 32 x 32.  K is
@@ -44,6 +44,11 @@ typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
 constexpr int SK = 16;           // k per step
 constexpr int SPLIT_PLAIN_K = 128;  // matMul: longer ranges of K are summed in blocks
 constexpr int SPLIT_BLOCK = 8;      // of this many steps
+// Fewer products than this stay in float32, which rounds once per product or two: the largest error
+// seen over 4 to 17 M results, in 2^-24 of the products' magnitudes, float32 kernels and these: K = 1
+// 1.0 and 4.1, 2 1.9 and 4.1, 3 2.8 and 3.6, 4 3.2 and 3.6, 5 3.5 and 3.3, 8 4.3 and 2.6; relative
+// (2-norm) 2.5e-8 and 3.1e-8, 3.1 and 3.1, 3.6 and 3.2, 4.0 and 3.2, 4.4 and 3.2, 5.4 and 3.2.
+constexpr int SPLIT_LEAST_K = 5;
 constexpr int SPLIT_FOLD = 4;       // steps per block where a tile is summed in float32
 
 // The slot of row (column) r of a tile and its inverse: within 64, row 4c + e goes to slot
@@ -112,7 +117,8 @@ struct Staging {
 // more than the two-level sum of the float32 kernels shows.  Measured against 64 bits, float32
 // kernels and these: matMul of signed values with K = 128 1.25e-7 and 0.62e-7, 1024 1.54e-7 and
 // 0.83e-7 (1.63e-7 without blocks), 4096 2.1e-7 and 1.2e-7; of positive ones 0.69 and 0.62, 0.72
-// and 0.56, 1.26 and 0.82; gradients of convolutions 2.2e-7 to 7.1e-7 and 1.1e-7 to 2.3e-7.
+// and 0.56, 1.26 and 0.82; gradients of convolutions 2.2e-7 to 7.1e-7 and 1.1e-7 to 2.3e-7.  What is
+// left out shows where there are few products (see SPLIT_LEAST_K).
 template <class T, int AMODE, int BMODE, int BLOCKED, bool VEC>
 __global__ __launch_bounds__(T::THREADS, 2) void gemm_split_kernel(const GemmArgs p) {
   constexpr int BM = T::BM, BN = T::BN, TM = T::TM, TN = T::TN, THREADS = T::THREADS;
@@ -717,7 +723,7 @@ static int launch_mode(tfhip_ctx* ctx, const GemmArgs& p, int batch, int amode32
 // the two estimates above are compared.
 int launch_split(tfhip_ctx* ctx, const GemmArgs& q, int batch, int amode, int bmode, bool kblocked,
                  long long a_bytes, long long b_bytes) {
-  if (q.M < 1 || q.N < 1 || q.K < 1 || batch < 1) return -1;
+  if (q.M < 1 || q.N < 1 || q.K < SPLIT_LEAST_K || batch < 1) return -1;
   if (batch == 1 && amode == A_ROWMAJOR && bmode != B_TRANSPOSED) return -1;
   if (amode == A_IM2COL) return -1;
   // 32-bit byte offsets, also of the steps past the last k and of a tile of the result
