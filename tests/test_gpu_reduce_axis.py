@@ -22,6 +22,9 @@ def tf():
     ((5, 7), (0,)), ((1, 9), (0,)), # fewer elements than row lanes
     ((4, 33, 20, 128), (0, 1, 2)),  # the statistics of a batch norm
     ((2, 70001, 8), (1,)),          # a slice that ends before the others
+    ((100003, 3, 2), (1,)),         # many short sums: one row lane, 512 columns of many outer indices
+    ((70001, 5, 8), (1,)),          # the same, four columns per lane, some row lanes without elements
+    ((1003, 33, 7), (1,)), ((5000, 9, 12), (1,)), ((300, 300, 20), (1,)),   # a few row lanes
 ])
 def test_reduce_axis(tf, shape, axes):
     print("reduce axis", shape, axes, flush=True)
@@ -62,3 +65,13 @@ def test_reduce_axis_ties_and_nan(tf):
     assert idx[2] == 17 and np.isnan(top[3]) and top[4] == 1
     np.testing.assert_array_equal(idx, want_idx)
     np.testing.assert_array_equal(top, want_top)
+
+
+def test_more_outer_indices_than_a_launch_has_workgroups(tf):
+    """8.4 million of them at one workgroup of 512 each would be more lanes than 32 bits count."""
+    x = np.random.default_rng(4).standard_normal((8400000, 2, 2)).astype(np.float32)
+    with tf.tidy():
+        t = tf.tensor(x)
+        got, top = tf.sum(t, 1).data_sync(), tf.arg_max(t, 1).data_sync()
+    np.testing.assert_array_equal(got, x.astype(np.float64).sum(1).astype(np.float32))
+    np.testing.assert_array_equal(top, x.argmax(1))

@@ -284,8 +284,9 @@ __global__ __launch_bounds__(WAVE* ROWS_PER_BLOCK) void reduce_finish_kernel(
 
 // Reduction over axes that are not the innermost ones: x viewed as [outer, red, inner], the middle
 // index reduced (a bias gradient, batch-norm statistics: [pixels, channels] over the pixels).
-// Bound by the one read of x.  A workgroup is a block of `cl` column lanes (of VEC neighbouring
-// columns each, so that a row of lanes reads one contiguous run) by THREADS / cl row lanes; the
+// Bound by the one read of x.  A cell is VEC neighbouring columns of one outer index; all cells are
+// counted through, so that a workgroup takes 1 << cl_shift of them whatever the extents are, one
+// per cell lane (neighbouring lanes read one contiguous run), by THREADS >> cl_shift row lanes.  The
 // row lanes stride over the slice of `red` the workgroup owns with UNROLL loads in flight, and meet
 // in LDS in a fixed order, so the result does not depend on scheduling.  parts > 1: `red` is cut
 // into that many slices over workgroups, whose partial results reduce_finish_kernel combines.
@@ -297,23 +298,24 @@ enum { COL_SUM = 0, COL_EXTREMUM = 1, COL_LOGICAL = 2 };
 template <int KIND, typename OutT, int VEC, int THREADS>
 __global__ __launch_bounds__(THREADS) void reduce_cols_kernel(
     int op, const void* x, int x_dt, OutT* out, double* pval, long long* pidx, int64_t red,
-    int64_t inner, int cl_shift, int col_blocks, int parts, int64_t seg, float divisor) {
-  constexpr int UNROLL = 8;
+    int64_t inner, uint32_t cells, Divisor lanes, int cl_shift, uint32_t cell_blocks, int parts,
+    int64_t seg, float divisor) {
+  constexpr int UNROLL = 8, TAIL = 4;
   // partial results, [row lane][column] with a row of one spare element (bank conflicts)
   __shared__ double s_val[THREADS * VEC + THREADS];
   __shared__ int64_t s_idx[KIND == COL_EXTREMUM ? THREADS * VEC + THREADS : 1];
   const int cl = 1 << cl_shift, rl = THREADS >> cl_shift;
   const int lc = threadIdx.x & (cl - 1), lr = threadIdx.x >> cl_shift;
-  // workgroup -> (outer, slice, column block), column blocks of a slice next to each other
-  const int cb = blockIdx.x % col_blocks;
-  const int64_t t = blockIdx.x / col_blocks;
-  const int part = (int)(t % parts);
-  const int64_t o = t / parts;
-  const int64_t col = ((int64_t)cb * cl + lc) * VEC;
-  const int64_t base = o * red * inner + col;
+  // workgroup -> (slice, block of cells), the blocks of a slice next to each other
+  const int part = (int)(blockIdx.x / cell_blocks);
+  const uint32_t cb = blockIdx.x - part * cell_blocks;
+  const uint32_t cell = cb * cl + lc;
+  const bool in = cell < cells;
+  uint32_t o = in ? cell : 0;
+  const int64_t col = (int64_t)lanes.divmod(o) * VEC;
+  const int64_t base = (int64_t)o * red * inner + col;
   const int64_t r0 = part * seg, r1 = min(red, r0 + seg);
   const bool want_max = op == TFHIP_MAX || op == TFHIP_ARGMAX;
-  const bool in = col < inner;  // (VEC divides inner: the lane's columns are in or out together)
 
   double acc[VEC];
   float best[VEC];
@@ -361,17 +363,45 @@ __global__ __launch_bounds__(THREADS) void reduce_cols_kernel(
 #pragma unroll
       for (int u = 0; u < UNROLL; u++) take(r + (int64_t)u * rl, v[u]);
     }
-    for (; r < r1; r += rl) {
-      float v[VEC];
-      load(r, v);
-      take(r, v);
+    // (what is left, or all of a short axis: in flight together too, past the end the first again)
+    for (; r < r1; r += (int64_t)TAIL * rl) {
+      float v[TAIL][VEC];
+#pragma unroll
+      for (int u = 0; u < TAIL; u++) load(r + (int64_t)u * rl < r1 ? r + (int64_t)u * rl : r, v[u]);
+#pragma unroll
+      for (int u = 0; u < TAIL; u++)
+        if (r + (int64_t)u * rl < r1) take(r + (int64_t)u * rl, v[u]);
     }
+  }
+  // a column's result, or that of this slice of it
+  auto put = [&](int64_t at, double v, int64_t vi) {
+    if (parts > 1) {
+      pval[at * parts + part] = v;
+      if (KIND == COL_EXTREMUM) pidx[at * parts + part] = vi;
+    } else if (KIND == COL_SUM) {
+      if (std::is_same<OutT, float>::value) out[at] = (OutT)(float)v;
+      else out[at] = (OutT)(int32_t)(uint32_t)(int64_t)v;
+    } else if (KIND == COL_EXTREMUM) {
+      if (op == TFHIP_ARGMAX || op == TFHIP_ARGMIN) out[at] = (OutT)vi;
+      else if (std::is_same<OutT, float>::value) out[at] = (OutT)(float)v;
+      else out[at] = (OutT)(int32_t)(float)v;
+    } else {
+      const bool any = v != 0.0;
+      out[at] = (OutT)(op == TFHIP_ANY ? any : !any);
+    }
+  };
+  auto mine = [&](int e) { return KIND == COL_SUM ? acc[e] : KIND == COL_EXTREMUM ? (double)best[e] : (double)hit[e]; };
+  if (rl == 1) {
+    if (!in) return;
+#pragma unroll
+    for (int e = 0; e < VEC; e++) put((int64_t)cell * VEC + e, mine(e), idx[e]);
+    return;
   }
   const int cols = cl * VEC, pitch = cols + 1;
 #pragma unroll
   for (int e = 0; e < VEC; e++) {
     const int at = lr * pitch + lc * VEC + e;
-    s_val[at] = KIND == COL_SUM ? acc[e] : KIND == COL_EXTREMUM ? (double)best[e] : (double)hit[e];
+    s_val[at] = mine(e);
     if (KIND == COL_EXTREMUM) s_idx[at] = idx[e];
   }
   __syncthreads();
@@ -389,37 +419,20 @@ __global__ __launch_bounds__(THREADS) void reduce_cols_kernel(
     }
   };
   const int share = min(WAVE, max(1, rl / VEC));
-  const int j = threadIdx.x & (share - 1), mine = threadIdx.x / share;
-  const int64_t c_out = (int64_t)cb * cols + mine;
-  const bool owner = mine < cols && c_out < inner;
-  double v = 0.0;
-  int64_t vi = 0;
-  if (owner) {
-    v = s_val[j * pitch + mine];
-    if (KIND == COL_EXTREMUM) vi = s_idx[j * pitch + mine];
+  const int j = threadIdx.x & (share - 1);
+  // (the same number of trips for all lanes: both are powers of two)
+  for (int c = threadIdx.x / share; c < cols; c += THREADS / share) {
+    double v = s_val[j * pitch + c];
+    int64_t vi = KIND == COL_EXTREMUM ? s_idx[j * pitch + c] : 0;
     for (int r = j + share; r < rl; r += share)
-      merge(v, vi, s_val[r * pitch + mine], KIND == COL_EXTREMUM ? s_idx[r * pitch + mine] : 0);
-  }
-  for (int off = share >> 1; off > 0; off >>= 1) {
-    const double ov = __shfl_down(v, off, WAVE);
-    const int64_t oi = KIND == COL_EXTREMUM ? __shfl_down(vi, off, WAVE) : 0;
-    merge(v, vi, ov, oi);
-  }
-  if (!owner || j != 0) return;
-  const int64_t at = o * inner + c_out;
-  if (parts > 1) {
-    pval[at * parts + part] = v;
-    if (KIND == COL_EXTREMUM) pidx[at * parts + part] = vi;
-  } else if (KIND == COL_SUM) {
-    if (std::is_same<OutT, float>::value) out[at] = (OutT)(float)v;
-    else out[at] = (OutT)(int32_t)(uint32_t)(int64_t)v;
-  } else if (KIND == COL_EXTREMUM) {
-    if (op == TFHIP_ARGMAX || op == TFHIP_ARGMIN) out[at] = (OutT)vi;
-    else if (std::is_same<OutT, float>::value) out[at] = (OutT)(float)v;
-    else out[at] = (OutT)(int32_t)(float)v;
-  } else {
-    const bool any = v != 0.0;
-    out[at] = (OutT)(op == TFHIP_ANY ? any : !any);
+      merge(v, vi, s_val[r * pitch + c], KIND == COL_EXTREMUM ? s_idx[r * pitch + c] : 0);
+    for (int off = share >> 1; off > 0; off >>= 1) {
+      const double ov = __shfl_down(v, off, WAVE);
+      const int64_t oi = KIND == COL_EXTREMUM ? __shfl_down(vi, off, WAVE) : 0;
+      merge(v, vi, ov, oi);
+    }
+    const int64_t at = (int64_t)cb * cols + c;
+    if (j == 0 && at < (int64_t)cells * VEC) put(at, v, vi);
   }
 }
 
@@ -702,66 +715,76 @@ extern "C" int tfhip_reduce(tfhip_ctx* ctx, int op, int64_t x, int64_t out, int6
   return reduce_rows(ctx, op, bx, bo, outer, inner, 1.f);
 }
 
+// The plan of a reduction over a middle axis: cells per workgroup (a power of two), workgroups, and
+// slices the axis is cut into.
+struct ColPlan {
+  int shift = 0, parts = 1;
+  int64_t cell_blocks = 0, seg = 0;
+};
+static ColPlan plan_reduce_cols(int64_t cells, int64_t lanes, int64_t red, int cus) {
+  auto shift_for = [&](int most) {  // (no more than the cells of one outer index, which lie side by side)
+    int s = 0;
+    while ((1 << s) < most && ((int64_t)1 << s) < lanes) s++;
+    return s;
+  };
+  ColPlan pl;
+  // One launch while a row lane of a tall workgroup (512 lanes) has few elements to walk, or where
+  // there are workgroups for every CU anyway: a second launch costs about 4 us.  A trip of eight
+  // loads takes about 2.5 us whatever it reads, so the workgroup is made as tall as it takes to
+  // have one or two trips, down to four cell lanes (runs of 64 bytes): [1000, 512] 14.1 us with
+  // sixteen cell lanes, 9.5 with four (12 for the transposition and the row sum before).
+  // Beyond 2048 elements the reduced axis is cut instead.
+  pl.shift = shift_for(16);
+  while (pl.shift > 2 && red > 8 * (int64_t)(512 >> pl.shift)) pl.shift--;
+  // And as wide as leaves every row lane eight elements while two workgroups per CU remain: with
+  // many cells and a short axis most row lanes would have nothing.  A workgroup per outer index and
+  // 16 lanes of it against this: [100352, 4, 8] 266 -> 6.4 us, [4000000, 2, 2] 7540 -> 37,
+  // [100000, 10, 32] 272 -> 25, [4096, 64, 16] 14.4 -> 5.6.
+  // (A launch counts its lanes in 32 bits: no more than 2^22 workgroups and a few.)
+  while (pl.shift < 9 && ((8 * (int64_t)(512 >> pl.shift) > red && cells >> (pl.shift + 1) >= 2 * cus) ||
+                          cells >> pl.shift >= 1 << 22))
+    pl.shift++;
+  pl.cell_blocks = ceil_div(cells, (int64_t)1 << pl.shift);
+  pl.seg = red;
+  if (red <= 16 * (int64_t)(512 >> pl.shift) || pl.cell_blocks >= 2 * cus) return pl;
+  // Slices of at least 16 elements a row lane, about eight workgroups of 256 lanes per CU.  (At
+  // least two of them: red is more than 16 times the row lanes, and there are fewer than 2 cus
+  // blocks of at most as many cells.)
+  pl.shift = shift_for(64);
+  pl.cell_blocks = ceil_div(cells, (int64_t)1 << pl.shift);
+  const int64_t rl = 256 >> pl.shift;
+  const int64_t parts = std::min<int64_t>(ceil_div(8 * (int64_t)cus, pl.cell_blocks), ceil_div(red, 16 * rl));
+  pl.seg = ceil_div(ceil_div(red, parts), rl) * rl;
+  pl.parts = (int)ceil_div(red, pl.seg);
+  return pl;
+}
+
 template <int KIND, typename OutT>
 static int launch_reduce_cols(tfhip_ctx* ctx, int op, const Buf* bx, const Buf* bo, int64_t outer,
                               int64_t red, int64_t inner, float divisor) {
   const bool vec = bx->dtype == TFHIP_FLOAT32 && inner % 4 == 0 &&
                    (reinterpret_cast<uintptr_t>(bx->ptr) & 15) == 0;
-  const int64_t lanes = vec ? inner / 4 : inner;  // column lanes of a row
-  // One launch while a row lane of a tall workgroup (512 lanes) has few elements to walk, or where
-  // there are workgroups for every CU anyway: a second launch costs about 4 us.  A trip of eight
-  // loads takes about 2.5 us whatever it reads, so the workgroup is made as tall as it takes to
-  // have one or two trips, down to four column lanes (runs of 64 bytes): [1000, 512] 14.1 us with
-  // sixteen column lanes, 9.5 with four (12 for the transposition and the row sum before).
-  // Beyond 2048 elements the reduced axis is cut instead.
-  auto shift_for = [&](int most) {
-    int s = 0;
-    while ((1 << s) < most && (int64_t)(1 << s) < lanes) s++;
-    return s;
-  };
-  int tall = shift_for(16);
-  while (tall > 2 && red > 8 * (int64_t)(512 >> tall)) tall--;
-  const int64_t tall_groups = outer * ceil_div(lanes, 1 << tall);
-  const bool single = red <= 16 * (int64_t)(512 >> tall) || tall_groups >= 2 * ctx->num_cus || ctx->no_alloc;
-  if (single) {
-    const int64_t col_blocks = ceil_div(lanes, 1 << tall), grid = outer * col_blocks;
-    if (grid > 0x7fffffffLL || col_blocks > 0x7fffffffLL)
-      return ctx->fail(TFHIP_ENOTSUP, "reduce: too many columns");
-    if (vec)
-      tfhip::launch(ctx, (reduce_cols_kernel<KIND, OutT, 4, 512>), dim3((unsigned)grid), dim3(512), 0, op,
-                    bx->ptr, bx->dtype, (OutT*)bo->ptr, nullptr, nullptr, red, inner, tall, (int)col_blocks,
-                    1, red, divisor);
-    else
-      tfhip::launch(ctx, (reduce_cols_kernel<KIND, OutT, 1, 512>), dim3((unsigned)grid), dim3(512), 0, op,
-                    bx->ptr, bx->dtype, (OutT*)bo->ptr, nullptr, nullptr, red, inner, tall, (int)col_blocks,
-                    1, red, divisor);
-    TFHIP_LAUNCH_CHECK_NAMED(ctx, "reduce_cols");
-    return TFHIP_OK;
-  }
-  // Slices of at least 16 elements a row lane, about eight workgroups of 256 lanes per CU.
-  const int wide = shift_for(64);
-  const int64_t col_blocks = ceil_div(lanes, 1 << wide), rl = 256 >> wide;
-  int64_t parts = std::min<int64_t>(ceil_div(8 * (int64_t)ctx->num_cus, outer * col_blocks),
-                                    ceil_div(red, 16 * rl));
-  const int64_t seg = ceil_div(ceil_div(red, parts), rl) * rl;
-  parts = ceil_div(red, seg);
-  const int64_t cells = outer * inner * parts, grid = outer * col_blocks * parts;
-  if (grid > 0x7fffffffLL) return ctx->fail(TFHIP_ENOTSUP, "reduce: too many columns");
+  const int64_t lanes = vec ? inner / 4 : inner, cells = outer * lanes;
+  if (cells > INDEX32) return ctx->fail(TFHIP_ENOTSUP, "reduce: too many columns");
+  const ColPlan pl = plan_reduce_cols(cells, lanes, red, ctx->num_cus);
+  const int64_t grid = pl.cell_blocks * pl.parts;
   Temp partial(ctx);
-  if (!partial.get((size_t)cells * 16)) return TFHIP_EDEVICE;
-  double* pval = static_cast<double*>(partial.ptr);
-  long long* pidx = reinterpret_cast<long long*>(pval + cells);
-  if (vec)
-    tfhip::launch(ctx, (reduce_cols_kernel<KIND, OutT, 4, 256>), dim3((unsigned)grid), dim3(256), 0, op,
-                  bx->ptr, bx->dtype, (OutT*)bo->ptr, pval, pidx, red, inner, wide, (int)col_blocks,
-                  (int)parts, seg, divisor);
-  else
-    tfhip::launch(ctx, (reduce_cols_kernel<KIND, OutT, 1, 256>), dim3((unsigned)grid), dim3(256), 0, op,
-                  bx->ptr, bx->dtype, (OutT*)bo->ptr, pval, pidx, red, inner, wide, (int)col_blocks,
-                  (int)parts, seg, divisor);
+  double* pval = nullptr;
+  long long* pidx = nullptr;
+  if (pl.parts > 1) {
+    const int64_t slots = outer * inner * pl.parts;
+    if (!partial.get((size_t)slots * 16)) return TFHIP_EDEVICE;
+    pval = static_cast<double*>(partial.ptr);
+    pidx = reinterpret_cast<long long*>(pval + slots);
+  }
+  const unsigned threads = pl.parts > 1 ? 256 : 512;
+  auto kernel = pl.parts > 1 ? (vec ? reduce_cols_kernel<KIND, OutT, 4, 256> : reduce_cols_kernel<KIND, OutT, 1, 256>)
+                             : (vec ? reduce_cols_kernel<KIND, OutT, 4, 512> : reduce_cols_kernel<KIND, OutT, 1, 512>);
+  tfhip::launch(ctx, kernel, dim3((unsigned)grid), dim3(threads), 0, op, bx->ptr, bx->dtype, (OutT*)bo->ptr, pval,
+                pidx, red, inner, (uint32_t)cells, Divisor(lanes), pl.shift, (uint32_t)pl.cell_blocks, pl.parts,
+                pl.seg, divisor);
   TFHIP_LAUNCH_CHECK_NAMED(ctx, "reduce_cols");
-  if (parts == 1) return ctx->fail(TFHIP_EDEVICE, "reduce: bad plan");
-  return launch_reduce_finish(ctx, op, pval, pidx, bo, outer * inner, (int)parts);
+  return pl.parts > 1 ? launch_reduce_finish(ctx, op, pval, pidx, bo, outer * inner, pl.parts) : TFHIP_OK;
 }
 
 extern "C" int tfhip_reduce_axis(tfhip_ctx* ctx, int op, int64_t x, int64_t out, int64_t outer,
