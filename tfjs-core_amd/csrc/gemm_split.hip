@@ -66,7 +66,7 @@ __device__ __forceinline__ int row_of(int s) {
 // exactly.  Integer operations and byte permutes (v_dot2_f32_bf16, which would subtract without
 // unpacking, is slower).  What l leaves are bits below the upper half of the last rest: `lost`
 // collects that word of every value, at one instruction for two: 3 x [1280, 1600] x [1600, 2240]
-// takes 205 us without and 216 with it (243 with a running minimum of the magnitudes, three
+// takes 220 us without and 224 with it (243 with a running minimum of the magnitudes, three
 // instructions for two).
 __device__ __forceinline__ void split2(float x0, float x1, unsigned& h, unsigned& m, unsigned& l, unsigned& lost) {
   constexpr unsigned TOP = 0x07060302u;  // the upper halves of two words as one
@@ -78,7 +78,9 @@ __device__ __forceinline__ void split2(float x0, float x1, unsigned& h, unsigned
   m = __builtin_amdgcn_perm(v1, v0, TOP);
   const unsigned w0 = __builtin_bit_cast(unsigned, r0 - top(v0)), w1 = __builtin_bit_cast(unsigned, r1 - top(v1));
   l = __builtin_amdgcn_perm(w1, w0, TOP);
-  lost = lost | w0 | w1;
+  // (as one instruction here and now: as an expression the compiler keeps the words and joins them
+  // later, which took up to 17 registers)
+  asm("v_or3_b32 %0, %1, %2, %0" : "+v"(lost) : "v"(w0), "v"(w1));
 }
 
 template <int WM_, int WN_, int TM_>
