@@ -216,3 +216,32 @@ def test_small_operands_against_large_ones_in_gathers(tf, n, h, w, cin, cout):
     d64 = dy.astype(np.float64)
     want, magnitude = _conv64(d64, back, 1, 1, (1, 1), h, w), _conv64(np.abs(d64), np.abs(back), 1, 1, (1, 1), h, w)
     assert np.all(np.abs(dx - want) <= _float32_bound(9 * cout, magnitude))
+
+
+@pytest.mark.parametrize("batch,m,k,n,ta,tb", [
+    (24, 1813, 33, 251, False, False), (96, 201, 67, 201, False, True), (1, 3001, 65, 3001, True, True),
+    (6, 2051, 130, 259, True, False), (60, 301, 66, 302, False, True),
+])
+def test_rows_that_are_not_whole_vectors(tf, batch, m, k, n, ta, tb):
+    """A vector read at a row's end holds the next row's first values, one stored there would pass the
+    row: infinities and NaN in those places stay in their own rows and columns."""
+    print("unaligned rows", batch, m, k, n, ta, tb, flush=True)
+    rng = np.random.default_rng(m + k + n)
+    a = rng.uniform(0.5, 1, (batch, m, k)).astype(np.float32)
+    b = rng.uniform(-1, 1, (batch, k, n)).astype(np.float32)
+    # (1e38: a sum of two such products is below the largest float32, 3.4e38)
+    a[0, 17, 0], a[-1, 100, 0], a[0, 0, k - 1], a[-1, m - 1, k - 1] = np.inf, np.nan, 1e38, -np.inf
+    b[0, 0, 9], b[-1, k - 1, 0], b[0, 1, 0], b[-1, 2, n - 1] = -np.inf, np.nan, np.inf, 1e38
+    with tf.tidy():
+        got = tf.matmul(tf.tensor(a.transpose(0, 2, 1).copy() if ta else a),
+                        tf.tensor(b.transpose(0, 2, 1).copy() if tb else b), ta, tb).data_sync()
+        assert _kernel(tf).startswith("gemm_split_"), _kernel(tf)
+    a64, b64 = a.astype(np.float64), b.astype(np.float64)
+    with np.errstate(invalid="ignore"):
+        want = a64 @ b64
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    assert np.array_equal(np.isposinf(got), np.isposinf(want)) and np.array_equal(np.isneginf(got), np.isneginf(want))
+    fin = np.isfinite(want)
+    magnitude = np.abs(np.nan_to_num(a64, posinf=0, neginf=0)) @ np.abs(np.nan_to_num(b64, posinf=0, neginf=0))
+    error = np.abs(np.where(fin, got, 0).astype(np.float64) - np.where(fin, want, 0))
+    assert np.all(error <= _float32_bound(k, magnitude))

@@ -210,19 +210,23 @@ __global__ __launch_bounds__(T::THREADS, 2) void gemm_split_kernel(const GemmArg
     }
   };
 
-  auto load4 = [&](const __amdgpu_buffer_rsrc_t& r, unsigned at, int base, int left) {
-    // 4 consecutive elements, `left` of them inside (VEC: all or none, which `at` says).  `base` is
-    // the same for all lanes; the range check is on the sum.
-    if (VEC) return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(r, (int)at, base, 0));
-    f32x4 v;
-#pragma unroll
-    for (int e = 0; e < 4; e++)
-      v[e] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(
-                 r, (int)(e < left ? at + 4u * e : OOB_OFFSET), base, 0));
-    return v;
+  // 4 consecutive elements, at 4-byte alignment where rows are not whole vectors: the hardware takes
+  // that, and checks the range of each of the four (four loads of 4 bytes: [3001, 1000] x [1000, 3001],
+  // both turned, 363 us, 158 like this, 250 in float32).  `base` is the same for all lanes; the
+  // range check is on the sum.
+  auto load4 = [&](const __amdgpu_buffer_rsrc_t& r, unsigned at, int base) {
+    return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(r, (int)at, base, 0));
   };
   struct Raw {
     f32x4 a[SA::REGS], b[SB::REGS];
+    int a_left, b_left;  // unaligned rows along k: how many of a vector's k there are
+  };
+  // What follows the last k of a row in memory is another row.  (Rows or columns past the last in a
+  // vector along them are harmless: their products are not stored.)
+  auto trim = [&](f32x4 v, int left) {
+#pragma unroll
+    for (int e = 1; e < 4; e++) v[e] = e < left ? v[e] : 0.f;
+    return v;
   };
   // From one output pixel to the next row's first, and from an image's last to the next image.
   const unsigned to_row = AMODE == A_IM2COL ? (unsigned)(p.dh * p.W - p.KW * p.dw) * p.Cin * 4u
@@ -235,10 +239,9 @@ __global__ __launch_bounds__(T::THREADS, 2) void gemm_split_kernel(const GemmArg
   auto load = [&](Raw& o) {
     const int k0 = __builtin_amdgcn_readfirstlane(k_next);
     if (AMODE == A_ROWMAJOR) {
-      const int left = p.K - k0 - SA::k(tid, 0);  // (the same for all items of a thread)
+      o.a_left = p.K - k0 - SA::k(tid, 0);  // (the same for all items of a thread)
 #pragma unroll
-      for (int i = 0; i < SA::PER; i++)
-        o.a[i] = load4(ra, left > 0 ? a_at[i] : OOB_OFFSET, k0 * 4, left);
+      for (int i = 0; i < SA::PER; i++) o.a[i] = load4(ra, o.a_left > 0 ? a_at[i] : OOB_OFFSET, k0 * 4);
     } else if (AMODE == A_IM2COL) {
       // (the 4 channels of an item share a filter tap: Cin is a multiple of 4)
       const bool in_k = k0 + SA::k(tid, 0) < p.K;
@@ -250,11 +253,9 @@ __global__ __launch_bounds__(T::THREADS, 2) void gemm_split_kernel(const GemmArg
       }
     } else if (AMODE == A_TRANSPOSED) {
 #pragma unroll
-      for (int i = 0; i < SA::PER; i++) {
-        const int left = p.M - bm0 - SA::row(tid, i);
+      for (int i = 0; i < SA::PER; i++)
 #pragma unroll
-        for (int e = 0; e < 2; e++) o.a[2 * i + e] = load4(ra, a_at[i], (k0 + e) * p.lda * 4, left);
-      }
+        for (int e = 0; e < 2; e++) o.a[2 * i + e] = load4(ra, a_at[i], (k0 + e) * p.lda * 4);
     } else {
       static_assert(AMODE != A_IM2COL_T || SA::PER == 1, "one pixel position per thread");
       const int k = k0 + SA::k(tid, 0);
@@ -269,17 +270,14 @@ __global__ __launch_bounds__(T::THREADS, 2) void gemm_split_kernel(const GemmArg
       }
     }
     if (B_KC) {
-      const int left = p.K - k0 - SB::k(tid, 0);
+      o.b_left = p.K - k0 - SB::k(tid, 0);
 #pragma unroll
-      for (int i = 0; i < SB::PER; i++)
-        o.b[i] = load4(rb, left > 0 ? b_at[i] : OOB_OFFSET, k0 * 4, left);
+      for (int i = 0; i < SB::PER; i++) o.b[i] = load4(rb, o.b_left > 0 ? b_at[i] : OOB_OFFSET, k0 * 4);
     } else {
 #pragma unroll
-      for (int i = 0; i < SB::PER; i++) {
-        const int left = p.N - bn0 - SB::row(tid, i);
+      for (int i = 0; i < SB::PER; i++)
 #pragma unroll
-        for (int e = 0; e < 2; e++) o.b[2 * i + e] = load4(rb, b_at[i], (k0 + e) * p.ldb * 4, left);
-      }
+        for (int e = 0; e < 2; e++) o.b[2 * i + e] = load4(rb, b_at[i], (k0 + e) * p.ldb * 4);
     }
   };
   auto advance = [&]() {
@@ -322,12 +320,13 @@ __global__ __launch_bounds__(T::THREADS, 2) void gemm_split_kernel(const GemmArg
   // An operand's items go into its planes at `base` in pieces of one split each: piece 2i + j is
   // the j-th pair of k of item i (k contiguous; the second writes both), piece 4i + e the pair of
   // k of row e of item i.
-  auto put_piece = [&](auto staging_tag, char* base, const f32x4* v, unsigned (&half)[3], int n) {
+  auto put_piece = [&](auto staging_tag, char* base, const f32x4* v, int left, unsigned (&half)[3], int n) {
     using S = decltype(staging_tag);
     unsigned part[3];
     if (S::KC) {
       const int i = n / 2, row = S::row(tid, i), k = S::k(tid, i);
-      split2(v[i][2 * (n & 1)], v[i][2 * (n & 1) + 1], part[0], part[1], part[2], lost);
+      const f32x4 x = VEC ? v[i] : trim(v[i], left);
+      split2(x[2 * (n & 1)], x[2 * (n & 1) + 1], part[0], part[1], part[2], lost);
       char* at = base + (k >> 3) * S::GROUP + row * 16 + (k & 4) * 2;
 #pragma unroll
       for (int s = 0; s < 3; s++) {
@@ -346,17 +345,17 @@ __global__ __launch_bounds__(T::THREADS, 2) void gemm_split_kernel(const GemmArg
   constexpr int A_PIECES = SA::REGS * 2, B_PIECES = SB::REGS * 2;
   unsigned half[3];
   auto stage_piece = [&](char* buf, const Raw& o, int n) {
-    if (n < A_PIECES) put_piece(SA(), buf, o.a, half, n);
-    else put_piece(SB(), buf + 3 * SA::PLANE, o.b, half, n - A_PIECES);
+    if (n < A_PIECES) put_piece(SA(), buf, o.a, o.a_left, half, n);
+    else put_piece(SB(), buf + 3 * SA::PLANE, o.b, o.b_left, half, n - A_PIECES);
   };
   // The same as float32 [k / 4][slot][4].
-  auto put_exact = [&](auto staging_tag, char* base, const f32x4* v) {
+  auto put_exact = [&](auto staging_tag, char* base, const f32x4* v, int left) {
     using S = decltype(staging_tag);
 #pragma unroll
     for (int i = 0; i < S::PER; i++) {
       const int row = S::row(tid, i), k = S::k(tid, i);
       if (S::KC) {
-        *reinterpret_cast<f32x4*>(base + (k >> 2) * (S::GROUP - 64) + row * 16) = v[i];
+        *reinterpret_cast<f32x4*>(base + (k >> 2) * (S::GROUP - 64) + row * 16) = VEC ? v[i] : trim(v[i], left);
       } else {
 #pragma unroll
         for (int e = 0; e < 4; e++)
@@ -482,8 +481,8 @@ __global__ __launch_bounds__(T::THREADS, 2) void gemm_split_kernel(const GemmArg
       for (int kt = cur.kt0; kt < cur.kt1; kt++) {
         load(raw);
         advance();
-        put_exact(SA(), lds, raw.a);
-        put_exact(SB(), lds + BM * 64, raw.b);
+        put_exact(SA(), lds, raw.a, raw.a_left);
+        put_exact(SB(), lds + BM * 64, raw.b, raw.b_left);
         __syncthreads();
 #pragma unroll
         for (int q = 0; q < SK / 8; q++) {
@@ -559,25 +558,30 @@ __global__ __launch_bounds__(T::THREADS, 2) void gemm_split_kernel(const GemmArg
   // STORE_WRITE_THROUGH.)
   const Clamp cl = clamp_of(p.act);
   const __amdgpu_buffer_rsrc_t rc = make_rsrc(p.C + tile_at, 0x7fffffffu);
-  const bool pairs = (p.N & 1) == 0;
+  auto store = [&](auto put) {
 #pragma unroll
-  for (int i = 0; i < TM; i++)
+    for (int i = 0; i < TM; i++)
 #pragma unroll
-    for (int r = 0; r < 16; r++) {
-      const int row = local_row(i, r);
-      const bool in = bm0 + row < p.M && col < p.N;
-      const unsigned at = in ? (unsigned)(row * p.N + lcol) * 4u : OOB_OFFSET;
-      const float v0 = clamp(hi[i][0][r] + bias_c[0], cl), v1 = clamp(hi[i][1][r] + bias_c[1], cl);
-      if (pairs) {
-        __builtin_amdgcn_raw_buffer_store_b64(
-            u32x2{__builtin_bit_cast(unsigned, v0), __builtin_bit_cast(unsigned, v1)}, rc, (int)at, 0,
-            STORE_WRITE_THROUGH);
-      } else {
-        __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, v0), rc, (int)at, 0, STORE_WRITE_THROUGH);
-        __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, v1), rc,
-                                              (int)(in && col + 1 < p.N ? at + 4u : OOB_OFFSET), 0, STORE_WRITE_THROUGH);
+      for (int r = 0; r < 16; r++) {
+        const int row = local_row(i, r);
+        const bool in = bm0 + row < p.M && col < p.N;
+        const float v0 = clamp(hi[i][0][r] + bias_c[0], cl), v1 = clamp(hi[i][1][r] + bias_c[1], cl);
+        put(in ? (unsigned)(row * p.N + lcol) * 4u : OOB_OFFSET,
+            u32x2{__builtin_bit_cast(unsigned, v0), __builtin_bit_cast(unsigned, v1)});
       }
-    }
+  };
+  if ((p.N & 1) == 0) {
+    store([&](unsigned at, u32x2 v) { __builtin_amdgcn_raw_buffer_store_b64(v, rc, (int)at, 0, STORE_WRITE_THROUGH); });
+    return;
+  }
+  // N odd: pairs of columns at 4-byte alignment, and the last column by itself.  Rows share their
+  // cache lines with their neighbours, so these stores wait in the L2 to be put together.  (Two
+  // 4-byte stores written through: 22 x [491, 16] x [16, 805] 24.4 us, 15.8 like this.)
+  const bool last = col + 1 == p.N, has_last = bn0 + BN >= p.N;
+  store([&](unsigned at, u32x2 v) {
+    __builtin_amdgcn_raw_buffer_store_b64(v, rc, (int)(last ? OOB_OFFSET : at), 0, 0);
+    if (has_last) __builtin_amdgcn_raw_buffer_store_b32(v[0], rc, (int)(last ? at : OOB_OFFSET), 0, 0);
+  });
 }
 
 // ---------------------------------------------------------------------------------------
@@ -719,7 +723,7 @@ static int launch_mode(tfhip_ctx* ctx, const GemmArgs& p, int batch, int amode32
 // convolutions, because relu and max pooling behind them decide by the last bit, and a training
 // step's gradients would move by whole elements against what they were.  Measured on MI355X,
 // float32 kernels against these: [3000, 1000]^T-shaped x [1000, 3000] 200 -> 146 us, [1500, 3000]
-// x [3000, 900]^T 101 -> 70, 96 x [201, 67] x [67, 201] 23.9 -> 20.4, 3 x 3 filter gradient of
+// x [3000, 900]^T 101 -> 70, 96 x [201, 67] x [67, 201] 24.8 -> 13.0, 3 x 3 filter gradient of
 // [32, 56, 56, 64] -> 128 158 -> 109, its input gradient 204 -> 137.  Small products are quicker
 // there (16 x [128, 128] x [128, 128] 5.8 against 8.2, [1000, 256] x [256, 100] 10.6 against 12.5):
 // the two estimates above are compared.
