@@ -135,3 +135,27 @@ def test_noalloc_under_both_stream_indices_takes_turns_on_the_array(tf):
         be.select_stream(0)
         for i, out in enumerate(outs):
             assert np.array_equal(out.data_sync(), want[i % 2 if i < 12 else 0]), i
+
+
+@pytest.mark.parametrize("m,k,n,ta,tb", [
+    (3136, 3072, 64, 0, 1), (64, 20000, 256, 1, 0), (128, 8000, 70, 1, 1),   # cut along K
+    (256, 512, 256, 0, 1), (2048, 1024, 1024, 1, 0),
+    (784, 2000, 512, 1, 0),                                                 # partial tiles beyond the array
+])
+def test_noalloc_takes_the_same_kernels_for_transposed_operands(tf, m, k, n, ta, tb):
+    be = tf.backend()
+    rng = np.random.default_rng(m + k)
+    a = rng.uniform(-1, 1, (1, k, m) if ta else (1, m, k)).astype(np.float32)
+    b = rng.uniform(-1, 1, (1, n, k) if tb else (1, k, n)).astype(np.float32)
+    with tf.tidy():
+        tf.matmul(tf.tensor(a), tf.tensor(b), bool(ta), bool(tb))
+        want = be.lib.tfhip_last_kernel(be.ctx).decode()
+    r1, r2, kernel, mem = _both(tf, a, b, ta=ta, tb=tb)
+    print("noalloc transposed", m, k, n, ta, tb, want, kernel if r1 is not None else r2, flush=True)
+    if m == 784:
+        assert r1 is None and "static scratch" in r2
+        return
+    assert r1 is not None, r2
+    assert kernel == want
+    assert np.array_equal(r1, r2)
+    assert mem[0] == mem[1], "the pool changed during a no-alloc call: %s" % (mem,)

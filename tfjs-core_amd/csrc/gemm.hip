@@ -1510,7 +1510,6 @@ static int choose_col_groups(const GemmArgs& p, const Plan& pl, double b_elem_by
 // the place of the pool block in which a product cut along K keeps its partial tiles.  Host
 // code reaches it only through the address hipGetSymbolAddress returns for the current
 // device (the array's name is not a device address on the host), asked once per device.
-constexpr size_t kScratchBytes = 8u << 20;
 constexpr int kMaxDevices = 64;
 static __device__ __align__(256) unsigned char scratch[kScratchBytes];
 static void* g_scratch_ptr[kMaxDevices];
@@ -1537,6 +1536,27 @@ int scratch_init(tfhip_ctx* ctx) {
 static void* scratch_address(tfhip_ctx* ctx) {
   if (!ctx->scratch) ctx->fail(TFHIP_EDEVICE, "static scratch memory was not set up");
   return ctx->scratch;
+}
+
+int partial_tiles(tfhip_ctx* ctx, size_t need, Temp* block, float** out) {
+  if (!ctx->no_alloc) {
+    if (!block->get(need)) return TFHIP_EDEVICE;
+    *out = static_cast<float*>(block->ptr);
+    return TFHIP_OK;
+  }
+  // the partial tiles go into the library's static device array instead of a pool block
+  if (need > kScratchBytes)
+    return ctx->fail(TFHIP_ENOTSUP,
+                     "matmul_noalloc: this product is cut along K and its partial tiles take "
+                     "%zu bytes, more than the %zu bytes of static scratch memory; use "
+                     "tfhip_matmul", need, kScratchBytes);
+  *out = static_cast<float*>(scratch_address(ctx));
+  if (!*out) return TFHIP_EDEVICE;
+  // one array per device, two compute streams: behind the other stream's last use of it
+  if (ctx->scratch_sidx >= 0 && ctx->scratch_sidx != ctx->cur) ctx->order(ctx->scratch_sidx, ctx->cur);
+  ctx->scratch_sidx = ctx->cur;
+  if (ctx->capturing) ctx->capture_used_scratch = true;
+  return TFHIP_OK;
 }
 
 template <class T, int AMODE, int BMODE, bool KBLOCKED, bool FAST>
@@ -1596,23 +1616,7 @@ static int launch_cfg(tfhip_ctx* ctx, GemmArgs& p, const Plan& pl) {
   p.partials = nullptr;
   if (pl.splits > 1) {
     const size_t need = (size_t)pl.tail_tiles * pl.splits * T::BM * T::BN * sizeof(float);
-    if (ctx->no_alloc) {
-      // the partial tiles go into the library's static device array instead of a pool block
-      if (need > kScratchBytes)
-        return ctx->fail(TFHIP_ENOTSUP,
-                         "matmul_noalloc: this product is cut along K and its partial tiles take "
-                         "%zu bytes, more than the %zu bytes of static scratch memory; use "
-                         "tfhip_matmul", need, kScratchBytes);
-      p.partials = static_cast<float*>(scratch_address(ctx));
-      if (!p.partials) return TFHIP_EDEVICE;
-      // one array per device, two compute streams: behind the other stream's last use of it
-      if (ctx->scratch_sidx >= 0 && ctx->scratch_sidx != ctx->cur) ctx->order(ctx->scratch_sidx, ctx->cur);
-      ctx->scratch_sidx = ctx->cur;
-      if (ctx->capturing) ctx->capture_used_scratch = true;
-    } else {
-      if (!partials.get(need)) return TFHIP_EDEVICE;
-      p.partials = static_cast<float*>(partials.ptr);
-    }
+    if (int rc = partial_tiles(ctx, need, &partials, &p.partials)) return rc;
   }
   tfhip::launch(ctx, (gemm_kernel<T::WM, T::WN, T::TM, T::TN, AMODE, BMODE, KBLOCKED, FAST>),
                      dim3(pl.grid), dim3(T::WM * T::WN * 64), 0, p);

@@ -679,8 +679,8 @@ static int launch_cfg(tfhip_ctx* ctx, GemmArgs p, const SplitPlan& pl) {
   p.partials = nullptr;
   Temp partials(ctx);
   if (pl.splits > 1) {
-    if (!partials.get((size_t)pl.tail * pl.splits * T::BM * T::BN * sizeof(float))) return TFHIP_EDEVICE;
-    p.partials = static_cast<float*>(partials.ptr);
+    const size_t need = (size_t)pl.tail * pl.splits * T::BM * T::BN * sizeof(float);
+    if (int rc = partial_tiles(ctx, need, &partials, &p.partials)) return rc;
   }
   tfhip::launch(ctx, (gemm_split_kernel<T, AMODE, BMODE, BLOCKED, VEC>),
                 dim3((unsigned)(pl.full + (long long)pl.tail * pl.splits)), dim3(T::THREADS), 0, p);
@@ -702,8 +702,10 @@ static int launch_mode(tfhip_ctx* ctx, const GemmArgs& p, int batch, int amode32
   plan_cfg(pl, 1, Wide::BM, Wide::BN, 0.56 * wait, 0.48, any, p, batch, cus);
   plan_cfg(pl, 2, Tall::BM, Tall::BN, 0.60 * wait, 0.58, any, p, batch, cus);
   if (pl.cfg < 0 || pl.cost > float32_cost(p, batch, cus, amode32, BMODE)) return -1;
-  // (the scratch array of the call that allocates nothing is sized for the float32 kernels' cuts)
-  if (ctx->no_alloc && pl.splits > 1) return -1;
+  // tfhip_matmul_noalloc takes the same plan where its array holds the partial tiles, and float32
+  // where not: the split kernels' cuts are larger than those it has always taken.
+  const size_t tile = pl.cfg == 0 ? Big::BM * Big::BN : pl.cfg == 1 ? Wide::BM * Wide::BN : Tall::BM * Tall::BN;
+  if (ctx->no_alloc && pl.splits > 1 && (size_t)pl.tail * pl.splits * tile * sizeof(float) > kScratchBytes) return -1;
   const int longest = pl.full ? (int)ceil_div(p.K, SK) : pl.kt_per;
   const bool blocked = KBLOCKED && longest * SK > SPLIT_PLAIN_K;
 #define TFHIP_LAUNCH(T)                                                            \

@@ -90,6 +90,11 @@ __device__ __forceinline__ void tile_row_col(const GemmArgs& p, int t, int& tm, 
   }
 }
 
+// gemm.hip: memory for the partial tiles of a product cut along K: a pool block that `block` holds,
+// or (tfhip_matmul_noalloc) the static array of kScratchBytes.
+constexpr size_t kScratchBytes = 8u << 20;
+int partial_tiles(tfhip_ctx* ctx, size_t need, Temp* block, float** out);
+
 // gemm.hip: adds the partial tiles [tail_tiles * splits][bm * bn] of a product cut along K.
 int launch_splitk_finish(tfhip_ctx* ctx, const GemmArgs& p, int bm, int bn);
 
