@@ -217,33 +217,45 @@ __global__ __launch_bounds__(256) void scatter_groups_kernel(const int64_t* __re
   }
 }
 
+// log2 of the groups: enough that a group's sums fit, and four workgroups per CU where there are rows
+// for them.
+static constexpr int scatter_group_shift(int64_t rows, int64_t col_blocks, int most_local, int cus) {
+  int shift = 0;
+  while ((rows + ((int64_t)1 << shift) - 1) >> shift > most_local ||
+         (((int64_t)1 << shift) * col_blocks < 4 * cus && ((int64_t)2 << shift) <= rows))
+    shift++;
+  return shift;
+}
+// A launch counts its lanes along a dimension in 32 bits: 2^23 groups of 256.  (168 million rows of 129
+// columns in double, 87 GB, are the first that need more.)
+constexpr int SCATTER_MOST_SHIFT = 23;
+static_assert(scatter_group_shift(20ll << 23, 1, 20, 256) == SCATTER_MOST_SHIFT &&
+              scatter_group_shift((20ll << 23) + 1, 1, 20, 256) > SCATTER_MOST_SHIFT, "");
+static_assert(scatter_group_shift(20000, 1, 80, 256) == 10 && scatter_group_shift(1, 1, 80, 256) == 0, "");
+
+// False: too many rows for this kernel.
 template <typename T, typename Acc, int CW>
-static void launch_scatter_groups(tfhip_ctx* ctx, const int64_t* flat, const T* updates, T* out, int rows,
+static bool launch_scatter_groups(tfhip_ctx* ctx, const int64_t* flat, const T* updates, T* out, int rows,
                                   int64_t slice, int64_t n_updates, T start, int sum_dupes, int scalar_update) {
   constexpr int CB = 64 * CW, MOST_LOCAL = (40 << 10) / (CB * (int)sizeof(Acc));  // 40 KB of sums
   const int64_t col_blocks = ceil_div(slice, CB);
-  // enough groups that a group's sums fit, and four workgroups per CU where there are rows for them
-  int shift = 0;
-  while (ceil_div(rows, (int64_t)1 << shift) > MOST_LOCAL ||
-         (((int64_t)1 << shift) * col_blocks < 4 * ctx->num_cus && ((int64_t)2 << shift) <= rows))
-    shift++;
+  const int shift = scatter_group_shift(rows, col_blocks, MOST_LOCAL, ctx->num_cus);
+  if (shift > SCATTER_MOST_SHIFT) return false;
   const int local_rows = (int)ceil_div(rows, (int64_t)1 << shift);
   tfhip::launch(ctx, (scatter_groups_kernel<T, Acc, CW>), dim3(1u << shift, (unsigned)col_blocks), dim3(256),
                 (size_t)local_rows * CB * sizeof(Acc), flat, updates, out, rows, slice, n_updates, start,
                 sum_dupes, scalar_update, shift, local_rows);
+  return true;
 }
 template <typename T, typename Acc>
 static void launch_scatter(tfhip_ctx* ctx, const int64_t* flat, const T* updates, T* out, int64_t rows,
                            int64_t slice, int64_t n_updates, T start, int sum_dupes, int scalar_update) {
   // (half a wavefront of columns, and column blocks that a grid's second dimension holds)
   if (slice >= 32 && n_updates > 0 && slice <= 65535 * 256) {
-    if (slice <= 64)
-      launch_scatter_groups<T, Acc, 1>(ctx, flat, updates, out, (int)rows, slice, n_updates, start, sum_dupes, scalar_update);
-    else if (slice <= 128)
-      launch_scatter_groups<T, Acc, 2>(ctx, flat, updates, out, (int)rows, slice, n_updates, start, sum_dupes, scalar_update);
-    else
-      launch_scatter_groups<T, Acc, 4>(ctx, flat, updates, out, (int)rows, slice, n_updates, start, sum_dupes, scalar_update);
-    return;
+    auto launch = slice <= 64    ? launch_scatter_groups<T, Acc, 1>
+                  : slice <= 128 ? launch_scatter_groups<T, Acc, 2>
+                                 : launch_scatter_groups<T, Acc, 4>;
+    if (launch(ctx, flat, updates, out, (int)rows, slice, n_updates, start, sum_dupes, scalar_update)) return;
   }
   tfhip::launch(ctx, (scatter_rows_kernel<T, Acc>), dim3(blocks_for(ctx, rows * slice)), dim3(256), 0, flat,
                 updates, out, rows, slice, n_updates, start, sum_dupes, scalar_update);
