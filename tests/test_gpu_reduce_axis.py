@@ -75,3 +75,74 @@ def test_more_outer_indices_than_a_launch_has_workgroups(tf):
         got, top = tf.sum(t, 1).data_sync(), tf.arg_max(t, 1).data_sync()
     np.testing.assert_array_equal(got, x.astype(np.float64).sum(1).astype(np.float32))
     np.testing.assert_array_equal(top, x.argmax(1))
+
+
+def _plan(tf, shape, parts):
+    """The number of kernels such a reduction takes: the axis cut over workgroups needs a second one."""
+    x = tf.tensor(np.ones(shape, np.float32))
+    with tf.tidy():
+        names = [k[0] if isinstance(k, tuple) else k["name"] for k in tf.time(lambda: tf.sum(x, 0))["kernelTimes"]]
+    x.dispose()
+    assert ("reduce_finish" in names) == (parts > 1), names
+
+
+@pytest.mark.parametrize("rows,parts", [(900, 1), (20000, 2)])
+def test_logical_outcomes_in_one_launch_and_two(tf, rows, parts):
+    """Columns of every outcome, decided in the first, a middle and the last slice of the axis."""
+    cols = 12
+    _plan(tf, (rows, cols), parts)
+    flags = np.ones((rows, cols), bool)
+    flags[:, 1] = False                                       # all false
+    for col, row in ((2, 0), (3, rows // 2), (4, rows - 1)):  # one false
+        flags[row, col] = False
+    flags[:, 5:8] = False
+    for col, row in ((5, 0), (6, rows // 2), (7, rows - 1)):  # one true
+        flags[row, col] = True
+    flags[:, 8:] = np.random.default_rng(rows).random((rows, cols - 8)) < 0.5
+    with tf.tidy():
+        t = tf.tensor(flags)
+        got_all, got_any = tf.all(t, 0).data_sync(), tf.any(t, 0).data_sync()
+    np.testing.assert_array_equal(got_all, flags.all(0))
+    np.testing.assert_array_equal(got_any, flags.any(0))
+    assert flags.all(0).any() and not flags.any(0).all()
+
+
+@pytest.mark.parametrize("rows,parts", [(900, 1), (20000, 2)])
+def test_products_over_leading_axes(tf, rows, parts):
+    rng = np.random.default_rng(rows)
+    x = (1 + rng.uniform(-1, 1, (rows, 12)) / 64).astype(np.float32)
+    x[rows // 3, 5] = 0
+    x[:, 6] = -x[:, 6]
+    ints = np.ones((rows, 8), np.int32)
+    ints[0], ints[rows // 2, :4], ints[-1, 2:6] = 3, -7, 2
+    _plan(tf, x.shape, parts)
+    with tf.tidy():
+        got, goti = tf.prod(tf.tensor(x), 0).data_sync(), tf.prod(tf.tensor(ints), 0).data_sync()
+    want = x.astype(np.float64).prod(0)
+    # products in double, one rounding each, and one to float32
+    assert np.all(np.abs(got - want) <= (2.0 ** -24 + rows * 2.0 ** -52) * np.abs(want))
+    np.testing.assert_array_equal(goti, ints.prod(0))
+
+
+def test_ties_and_nan_across_slices(tf):
+    """As in test_reduce_axis_ties_and_nan, with the axis cut: equal values in different slices, NaN in
+    element 0 (which stays) and in others (which never win), infinities at the ends."""
+    rows = 20000
+    _plan(tf, (rows, 8), 2)
+    x = np.zeros((rows, 8), np.float32)
+    x[11000, 0] = x[19999, 0] = x[400, 0] = 5
+    x[19999, 1] = 7
+    x[0, 2] = np.nan
+    x[9000:9100, 3] = np.nan
+    x[15000, 3] = 2
+    x[0, 4], x[rows - 1, 4] = -np.inf, np.inf
+    x[:, 5] = -np.inf
+    x[:, 6] = np.arange(rows, 0, -1)
+    with tf.tidy():
+        t, turned = tf.tensor(x), tf.tensor(np.ascontiguousarray(x.T))
+        for name in ("arg_max", "arg_min", "max", "min"):
+            got, want = getattr(tf, name)(t, 0).data_sync(), getattr(tf, name)(turned, 1).data_sync()
+            np.testing.assert_array_equal(got, want, err_msg=name)
+        idx, top = tf.arg_max(t, 0).data_sync(), tf.max(t, 0).data_sync()
+    assert list(idx[:2]) == [400, 19999] and np.isnan(top[2]) and idx[2] == 0
+    assert idx[3] == 15000 and top[3] == 2 and idx[4] == rows - 1 and idx[5] == 0 and idx[6] == 0

@@ -245,3 +245,68 @@ def test_rows_that_are_not_whole_vectors(tf, batch, m, k, n, ta, tb):
     magnitude = np.abs(np.nan_to_num(a64, posinf=0, neginf=0)) @ np.abs(np.nan_to_num(b64, posinf=0, neginf=0))
     error = np.abs(np.where(fin, got, 0).astype(np.float64) - np.where(fin, want, 0))
     assert np.all(error <= _float32_bound(k, magnitude))
+
+
+@pytest.mark.parametrize("m,k,n,ta,tb,kernel", [
+    (4096, 64, 4096, True, False, "128x128"), (3136, 3072, 64, False, True, "128x64"),
+    (64, 20000, 256, True, False, "_splitk"), (2048, 1024, 1028, True, True, "64x128"),
+])
+def test_special_values_in_every_tile_shape(tf, m, k, n, ta, tb, kernel):
+    """Infinities and NaN reach the float32 pass of each tile shape and of tiles cut along K."""
+    print("special values", m, k, n, ta, tb, flush=True)
+    rng = np.random.default_rng(m)
+    a, b = rng.uniform(0.5, 1, (m, k)).astype(np.float32), rng.uniform(-1, 1, (k, n)).astype(np.float32)
+    a[1, k // 2], a[m // 2, 3], a[m - 1, k - 1] = np.inf, np.nan, -np.inf
+    b[k - 1, n - 1], b[0, n // 2] = np.inf, np.nan
+    with tf.tidy():
+        got = tf.matmul(tf.tensor(a.T.copy() if ta else a), tf.tensor(b.T.copy() if tb else b), ta, tb).data_sync()
+        name = _kernel(tf)
+    assert name.startswith("gemm_split_") and kernel in name, name
+    a64, b64 = a.astype(np.float64), b.astype(np.float64)
+    with np.errstate(invalid="ignore"):
+        want = a64 @ b64
+    _same_specials(got, want)
+    fin = np.isfinite(want)
+    magnitude = np.abs(np.nan_to_num(a64, posinf=0, neginf=0)) @ np.abs(np.nan_to_num(b64, posinf=0, neginf=0))
+    assert np.all(np.abs(np.where(fin, got, 0) - np.where(fin, want, 0)) <= _float32_bound(k, magnitude))
+
+
+def _same_specials(got, want):
+    for test in (np.isnan, np.isposinf, np.isneginf):
+        assert np.array_equal(test(got), test(want)), test.__name__
+
+
+@pytest.mark.parametrize("n,h,w,cin,cout", [(8, 33, 47, 64, 136), (320, 7, 9, 96, 128)])
+def test_special_values_in_gathers(tf, n, h, w, cin, cout):
+    print("special values, gradients", n, h, w, cin, cout, flush=True)
+    rng = np.random.default_rng(n + cout)
+    x, dy = (rng.standard_normal((n, h, w, c)).astype(np.float32) for c in (cin, cout))
+    wt = rng.standard_normal((3, 3, cin, cout)).astype(np.float32)
+    x[0, 3, 4, 1], x[-1, -1, -1, 2], dy[1, 0, 0, 5] = np.inf, np.nan, -np.inf
+    with tf.tidy():
+        dw = tf.conv2d_der_filter(tf.tensor(x), tf.tensor(dy), wt.shape, 1, "same").data_sync()
+        assert _kernel(tf).startswith("gemm_split_"), _kernel(tf)
+    clean = lambda v: np.abs(np.nan_to_num(v.astype(np.float64), posinf=0, neginf=0))
+    pad = lambda v: np.pad(v, ((0, 0), (1, 1), (1, 1), (0, 0)))
+    p, flat = pad(x.astype(np.float64)), dy.reshape(-1, cout).astype(np.float64)
+    for i in range(3):
+        for j in range(3):
+            part = p[:, i:i + h, j:j + w].reshape(-1, cin).T
+            with np.errstate(invalid="ignore"):
+                want = part @ flat
+            # (the padding of x is zeros, which the infinite dy in a corner makes NaN: in the kernel too)
+            _same_specials(dw[i, j], want)
+            fin = np.isfinite(want)
+            bound = _float32_bound(n * h * w, clean(part) @ clean(flat))
+            assert np.all(np.abs(np.where(fin, dw[i, j], 0) - np.where(fin, want, 0)) <= bound)
+    dy[0, 2, 2, 7] = np.nan
+    with tf.tidy():
+        dx = tf.conv2d_der_input(x.shape, tf.tensor(dy), tf.tensor(wt), 1, "same").data_sync()
+        assert _kernel(tf).startswith("gemm_split_"), _kernel(tf)
+    back = np.ascontiguousarray(wt[::-1, ::-1].transpose(0, 1, 3, 2)).astype(np.float64)
+    with np.errstate(invalid="ignore"):
+        want = _conv64(dy.astype(np.float64), back, 1, 1, (1, 1), h, w)
+    _same_specials(dx, want)
+    fin = np.isfinite(want)
+    bound = _float32_bound(9 * cout, _conv64(clean(dy), clean(back), 1, 1, (1, 1), h, w))
+    assert np.all(np.abs(np.where(fin, dx, 0) - np.where(fin, want, 0)) <= bound)

@@ -29,7 +29,8 @@
 // infinity), and of a value below 2^-110 the last bits can lie below 2^-133, the smallest bf16.  So
 // a workgroup that finds a result that is not finite, or that has staged an operand which is not
 // the sum of its parts, computes its tile again with float32 matrix instructions, and the result
-// is what the float32 kernels give.  Small results need nothing of the kind: these instructions take and give
+// is what the float32 kernels give.  Such a tile takes the time of both: [4096, 1024]^T-shaped x
+// [1024, 1024] 78 us, 157 with one infinity or one value of 2^-120 (float32 kernels 93).  Small results need nothing of the kind: these instructions take and give
 // denormal values, and with both operands near 2^-63 the error is 0.7e-7 here and 0.9e-7 there.
 #include <type_traits>
 
