@@ -447,8 +447,8 @@ def _axis_block(axes):
     Backends with `reduce_block` (feature detection) reduce such axes where they are; for the
     others, and for axes that are apart, the axes are brought innermost first, as the reference does."""
     axes = sorted(axes)
-    if axes and axes == list(range(axes[0], axes[0] + len(axes))) and hasattr(ENGINE.backend, "reduce_block"):
-        return axes
+    if len(axes) == 1 or axes and axes == list(range(axes[0], axes[0] + len(axes))):
+        return axes if hasattr(ENGINE.backend, "reduce_block") else None
     return None
 
 
