@@ -14,9 +14,9 @@
 // What bounds it: a 128 x 128 step is 24 matrix instructions per wavefront, 19 ns each with
 // nothing else in the machine and 23.6 with the six vector instructions per matrix instruction
 // that splitting and addressing cost, and takes 34; LDS is busy a quarter of the time, without
-// conflicts.  3 x 3 convolutions reach 140 to 165 TFLOP/s (float32 kernels 95 to 116, and 157 is
-// the float32 matrix peak).  Measured without effect on that: one buffer of 32 k, loads two steps
-// ahead, the leading parts read before the barrier, v_cvt_pk_bf16_f32 for the splits.
+// conflicts.  Gradients of 3 x 3 convolutions run at 93 to 153 TFLOP/s (float32 kernels 63 to 99, and
+// 157 is the float32 matrix peak).  Measured without effect on that: one buffer of 32 k, loads two
+// steps ahead, the leading parts read before the barrier, v_cvt_pk_bf16_f32 for the splits.
 //
 // LDS layout.  Per operand three planes (h, m, l) of [k / 8][slot][8 bf16]: the matrix instruction
 // takes 8 consecutive k of a row per lane, and 32 lanes read 512 consecutive bytes.  A slot is a
@@ -30,8 +30,9 @@
 // a workgroup that finds a result that is not finite, or that has staged an operand which is not
 // the sum of its parts, computes its tile again with float32 matrix instructions, and the result
 // is what the float32 kernels give.  Such a tile takes the time of both: [4096, 1024]^T-shaped x
-// [1024, 1024] 78 us, 157 with one infinity or one value of 2^-120 (float32 kernels 93).  Small results need nothing of the kind: these instructions take and give
-// denormal values, and with both operands near 2^-63 the error is 0.7e-7 here and 0.9e-7 there.
+// [1024, 1024] 78 us, 157 with one infinity or one value of 2^-120 (float32 kernels 93).  Small
+// results need nothing of the kind: these instructions take and give denormal values, and with
+// both operands near 2^-63 the error is 0.7e-7 here and 0.9e-7 there.
 #include <type_traits>
 
 #include "tfhip_gemm.h"
@@ -646,7 +647,7 @@ static void plan_cfg(SplitPlan& best, int cfg, int bm, int bn, double alone, dou
 static double float32_cost(const GemmArgs& p, int batch, int cus, int amode, int bmode) {
   const double tiles = (double)ceil_div(p.M, 64) * (double)ceil_div(p.N, 64) * batch;
   const double steps = (double)ceil_div(p.K, 16);
-  const double slower = amode == A_IM2COL_UP ? 1.35 : amode == A_IM2COL_T ? 1.25 : amode == A_IM2COL ? 1.1
+  const double slower = amode == A_IM2COL_UP ? 1.35 : amode == A_IM2COL_T ? 1.25
                       : amode == A_TRANSPOSED || bmode == B_TRANSPOSED ? 1.08 : 1.0;
   auto price = [&](double items, double n) {
     return 4.0 + slower * n * (items / cus * 0.33 > 0.4 ? items / cus * 0.33 : 0.4);
@@ -720,16 +721,16 @@ static int launch_mode(tfhip_ctx* ctx, const GemmArgs& p, int batch, int amode32
 #undef TFHIP_LAUNCH
 }
 
-// Which products come here: transposed and batched ones and the gradients of convolutions.
-// Row-major products of one batch entry, and with them the pointwise convolutions, stay with the
-// float32 kernels, whose tile for a shape is settled and tested by name; so do forward
-// convolutions, because relu and max pooling behind them decide by the last bit, and a training
-// step's gradients would move by whole elements against what they were.  Measured on MI355X,
-// float32 kernels against these: [3000, 1000]^T-shaped x [1000, 3000] 200 -> 146 us, [1500, 3000]
-// x [3000, 900]^T 101 -> 70, 96 x [201, 67] x [67, 201] 24.8 -> 13.0, 3 x 3 filter gradient of
-// [32, 56, 56, 64] -> 128 158 -> 109, its input gradient 204 -> 137.  Small products are quicker
-// there (16 x [128, 128] x [128, 128] 5.8 against 8.2, [1000, 256] x [256, 100] 10.6 against 12.5):
-// the two estimates above are compared.
+// Which products come here: transposed and batched ones and the gradients of convolutions, where
+// the two estimates above say so.  Measured on MI355X with normal values, float32 kernels against
+// these: [3000, 1000]^T-shaped x [1000, 3000] 203 -> 177 us, [1500, 3000] x [3000, 900]^T 102 -> 84,
+// 3 x [1280, 1600] x [1600, 2240] 289 -> 230, 96 x [201, 67] x [67, 201] 24.1 -> 13.2, 3 x 3 filter
+// gradient of [32, 56, 56, 64] -> 128 159 -> 113, its input gradient 209 -> 144.  Small products are
+// quicker there (16 x [128, 128] x [128, 128] 5.8 against 8.2, [1000, 256] x [256, 100] 10.6 against
+// 12.5).  Row-major products of one batch entry, and with them the pointwise convolutions, and
+// forward convolutions have not been moved: the float32 kernels' tile choice for them is asserted by
+// name at some sizes, and the results of relu and max pooling behind a forward convolution change
+// with its rounding, whichever that is.
 int launch_split(tfhip_ctx* ctx, const GemmArgs& q, int batch, int amode, int bmode, bool kblocked,
                  long long a_bytes, long long b_bytes) {
   if (q.M < 1 || q.N < 1 || q.K < SPLIT_LEAST_K || batch < 1) return -1;
