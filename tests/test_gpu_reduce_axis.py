@@ -146,3 +146,33 @@ def test_ties_and_nan_across_slices(tf):
         idx, top = tf.arg_max(t, 0).data_sync(), tf.max(t, 0).data_sync()
     assert list(idx[:2]) == [400, 19999] and np.isnan(top[2]) and idx[2] == 0
     assert idx[3] == 15000 and top[3] == 2 and idx[4] == rows - 1 and idx[5] == 0 and idx[6] == 0
+
+
+@pytest.mark.parametrize("shape,axis", [
+    ((300001, 5), 0),      # 512 slices, combined by 32 rows of lanes in two trips; fewer columns than a workgroup takes
+    ((70003, 36), 0),      # four columns per lane, a second workgroup of columns that is nearly empty
+    ((4097, 44), 0),       # two slices
+    ((3, 20011, 21), 1),   # outer extents among the columns
+    ((1024, 4), 0),        # one launch: eight elements for every row lane
+    ((1025, 4), 0),        # and one more
+])
+def test_sliced_columns_of_every_operation(tf, shape, axis):
+    print("sliced columns", shape, axis, flush=True)
+    rng = np.random.default_rng(sum(shape))
+    x = rng.integers(-4, 5, shape).astype(np.float32)          # sums exact, extrema tied
+    near = (1 + 1e-4 * rng.standard_normal(shape)).astype(np.float32)
+    flags = rng.random(shape) < 2.0 / shape[axis]
+    with tf.tidy():
+        t, tn, tb = tf.tensor(x), tf.tensor(near), tf.tensor(flags)
+        for op in ("sum", "max", "min"):
+            np.testing.assert_array_equal(getattr(tf, op)(t, axis).data_sync(), getattr(np, op)(x, axis))
+        for op, want in (("arg_max", np.argmax), ("arg_min", np.argmin)):
+            np.testing.assert_array_equal(getattr(tf, op)(t, axis).data_sync(), want(x, axis))
+        np.testing.assert_array_equal(tf.any(tb, axis).data_sync(), flags.any(axis))
+        np.testing.assert_array_equal(tf.all(tf.logical_not(tb), axis).data_sync(), (~flags).all(axis))
+        mean, prod = tf.mean(tn, axis).data_sync(), tf.prod(tn, axis).data_sync()
+    # the quotients are rounded to float32 before they are added, the sum once more
+    want = near.astype(np.float64).mean(axis)
+    assert np.all(np.abs(mean - want) <= 2 * 2.0 ** -24 * np.abs(want) + 2.0 ** -24)
+    want = near.astype(np.float64).prod(axis)
+    assert np.all(np.abs(prod - want) <= 2 * 2.0 ** -24 * np.abs(want))

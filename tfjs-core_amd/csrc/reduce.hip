@@ -286,25 +286,53 @@ __global__ __launch_bounds__(WAVE* ROWS_PER_BLOCK) void reduce_finish_kernel(
 // index reduced (a bias gradient, batch-norm statistics: [pixels, channels] over the pixels).
 // Bound by the one read of x.  A cell is VEC neighbouring columns of one outer index; all cells are
 // counted through, so that a workgroup takes 1 << cl_shift of them whatever the extents are, one
-// per cell lane (neighbouring lanes read one contiguous run), by THREADS >> cl_shift row lanes.  The
+// per cell lane (neighbouring lanes read one contiguous run), by COL_THREADS >> cl_shift row lanes.  The
 // row lanes stride over the slice of `red` the workgroup owns with UNROLL loads in flight, and meet
 // in LDS in a fixed order, so the result does not depend on scheduling.  parts > 1: `red` is cut
-// into that many slices over workgroups, whose partial results reduce_finish_kernel combines.
+// into that many slices over workgroups, whose partial results (a row of all columns per slice, so
+// that they are written and read in whole lines) reduce_cols_finish_kernel combines.
 // The rules are those of reduce_rows_kernel: sums and products in double, an extremum starts from
 // element 0 and is replaced only by a strictly better value, equal values keep the lower index.
-// Before, such an axis was first transposed to the inside: [100352, 128] summed over its rows took
-// 84 us for the transposition and 15 for the sum, and a mean 34 more for the division.
-enum { COL_SUM = 0, COL_EXTREMUM = 1, COL_LOGICAL = 2 };
-template <int KIND, typename OutT, int VEC, int THREADS>
-__global__ __launch_bounds__(THREADS) void reduce_cols_kernel(
+// What is reduced is known at compile time: a short sum is a chain of a load, a few additions and
+// the meeting in LDS, and fetching the instructions of the operations it does not do is part of it: [1000, 512] 7.1 -> 4.4 us,
+// [4096, 1024] 8.5 -> 4.3, [100352, 128] 13.4 -> 9.8 (5.2 TB/s; with the combining launch 19.5 -> 15.0).
+enum { COL_SUM = 0, COL_MEAN, COL_PROD, COL_EXTREMUM, COL_LOGICAL };
+constexpr int COL_THREADS = 512;
+
+template <int KIND>
+__device__ __forceinline__ void merge_cols(bool want_max, double& v, int64_t& i, double ov, int64_t oi) {
+  if (KIND == COL_EXTREMUM) {
+    if ((want_max ? ov > v : ov < v) || (ov == v && oi < i)) {
+      v = ov;
+      i = oi;
+    }
+  } else if (KIND == COL_LOGICAL) {
+    v = v != 0.0 || ov != 0.0 ? 1.0 : 0.0;
+  } else {
+    v = KIND == COL_PROD ? v * ov : v + ov;
+  }
+}
+template <int KIND, typename OutT>
+__device__ __forceinline__ OutT col_result(int op, double v, int64_t i) {
+  if (KIND == COL_EXTREMUM) {
+    if (op == TFHIP_ARGMAX || op == TFHIP_ARGMIN) return (OutT)i;
+    return std::is_same<OutT, float>::value ? (OutT)v : (OutT)(int32_t)(float)v;
+  }
+  if (KIND == COL_LOGICAL) return (OutT)((v != 0.0) == (op == TFHIP_ANY));
+  return std::is_same<OutT, float>::value ? (OutT)(float)v : (OutT)(int32_t)(uint32_t)(int64_t)v;
+}
+
+template <int KIND, typename OutT, int VEC>
+__global__ __launch_bounds__(COL_THREADS) void reduce_cols_kernel(
     int op, const void* x, int x_dt, OutT* out, double* pval, long long* pidx, int64_t red,
     int64_t inner, uint32_t cells, Divisor lanes, int cl_shift, uint32_t cell_blocks, int parts,
     int64_t seg, float divisor) {
-  constexpr int UNROLL = 8, TAIL = 4;
+  constexpr int UNROLL = 8;
+  constexpr bool INDEXED = KIND == COL_EXTREMUM;
   // partial results, [row lane][column] with a row of one spare element (bank conflicts)
-  __shared__ double s_val[THREADS * VEC + THREADS];
-  __shared__ int64_t s_idx[KIND == COL_EXTREMUM ? THREADS * VEC + THREADS : 1];
-  const int cl = 1 << cl_shift, rl = THREADS >> cl_shift;
+  __shared__ double s_val[COL_THREADS * VEC + COL_THREADS];
+  __shared__ int64_t s_idx[INDEXED ? COL_THREADS * VEC + COL_THREADS : 1];
+  const int cl = 1 << cl_shift, rl = COL_THREADS >> cl_shift;
   const int lc = threadIdx.x & (cl - 1), lr = threadIdx.x >> cl_shift;
   // workgroup -> (slice, block of cells), the blocks of a slice next to each other
   const int part = (int)(blockIdx.x / cell_blocks);
@@ -317,16 +345,12 @@ __global__ __launch_bounds__(THREADS) void reduce_cols_kernel(
   const int64_t r0 = part * seg, r1 = min(red, r0 + seg);
   const bool want_max = op == TFHIP_MAX || op == TFHIP_ARGMAX;
 
-  double acc[VEC];
-  float best[VEC];
+  double acc[VEC];  // the sum, the product, the extremum, whether an element decided (1) or not (0)
   int64_t idx[VEC];
-  int hit[VEC];
 #pragma unroll
   for (int e = 0; e < VEC; e++) {
-    acc[e] = op == TFHIP_PROD ? 1.0 : 0.0;
-    best[e] = KIND == COL_EXTREMUM && in ? ld(x, x_dt, base + e) : 0.f;
+    acc[e] = KIND == COL_PROD ? 1.0 : INDEXED && in ? (double)ld(x, x_dt, base + e) : 0.0;
     idx[e] = 0;
-    hit[e] = 0;
   }
   auto load = [&](int64_t r, float (&v)[VEC]) {
     if (VEC == 4) {
@@ -341,16 +365,13 @@ __global__ __launch_bounds__(THREADS) void reduce_cols_kernel(
   auto take = [&](int64_t r, const float (&v)[VEC]) {
 #pragma unroll
     for (int e = 0; e < VEC; e++) {
-      if (KIND == COL_SUM) {
-        if (op == TFHIP_SUM) acc[e] += (double)quotient(v[e], divisor);
-        else acc[e] *= (double)v[e];
-      } else if (KIND == COL_EXTREMUM) {
-        if (want_max ? v[e] > best[e] : v[e] < best[e]) {
-          best[e] = v[e];
-          idx[e] = r;
-        }
-      } else {
-        hit[e] |= (v[e] != 0.f) == (op == TFHIP_ANY);
+      if (KIND == COL_SUM) acc[e] += (double)v[e];
+      else if (KIND == COL_MEAN) acc[e] += (double)(v[e] / divisor);
+      else if (KIND == COL_PROD) acc[e] *= (double)v[e];
+      else if (KIND == COL_LOGICAL) acc[e] = (v[e] != 0.f) == (op == TFHIP_ANY) ? 1.0 : acc[e];
+      else if (want_max ? (double)v[e] > acc[e] : (double)v[e] < acc[e]) {
+        acc[e] = (double)v[e];
+        idx[e] = r;
       }
     }
   };
@@ -363,77 +384,109 @@ __global__ __launch_bounds__(THREADS) void reduce_cols_kernel(
 #pragma unroll
       for (int u = 0; u < UNROLL; u++) take(r + (int64_t)u * rl, v[u]);
     }
-    // (what is left, or all of a short axis: in flight together too, past the end the first again)
-    for (; r < r1; r += (int64_t)TAIL * rl) {
-      float v[TAIL][VEC];
+    // what is left, or all of a short axis, in flight together too: past the end the first again
+    if (r < r1) {
+      float v[UNROLL][VEC];
 #pragma unroll
-      for (int u = 0; u < TAIL; u++) load(r + (int64_t)u * rl < r1 ? r + (int64_t)u * rl : r, v[u]);
+      for (int u = 0; u < UNROLL; u++) load(r + (int64_t)u * rl < r1 ? r + (int64_t)u * rl : r, v[u]);
 #pragma unroll
-      for (int u = 0; u < TAIL; u++)
+      for (int u = 0; u < UNROLL; u++)
         if (r + (int64_t)u * rl < r1) take(r + (int64_t)u * rl, v[u]);
     }
   }
+  const int64_t columns = (int64_t)cells * VEC;
   // a column's result, or that of this slice of it
   auto put = [&](int64_t at, double v, int64_t vi) {
     if (parts > 1) {
-      pval[at * parts + part] = v;
-      if (KIND == COL_EXTREMUM) pidx[at * parts + part] = vi;
-    } else if (KIND == COL_SUM) {
-      if (std::is_same<OutT, float>::value) out[at] = (OutT)(float)v;
-      else out[at] = (OutT)(int32_t)(uint32_t)(int64_t)v;
-    } else if (KIND == COL_EXTREMUM) {
-      if (op == TFHIP_ARGMAX || op == TFHIP_ARGMIN) out[at] = (OutT)vi;
-      else if (std::is_same<OutT, float>::value) out[at] = (OutT)(float)v;
-      else out[at] = (OutT)(int32_t)(float)v;
+      pval[part * columns + at] = v;
+      if (INDEXED) pidx[part * columns + at] = vi;
     } else {
-      const bool any = v != 0.0;
-      out[at] = (OutT)(op == TFHIP_ANY ? any : !any);
+      out[at] = col_result<KIND, OutT>(op, v, vi);
     }
   };
-  auto mine = [&](int e) { return KIND == COL_SUM ? acc[e] : KIND == COL_EXTREMUM ? (double)best[e] : (double)hit[e]; };
   if (rl == 1) {
     if (!in) return;
 #pragma unroll
-    for (int e = 0; e < VEC; e++) put((int64_t)cell * VEC + e, mine(e), idx[e]);
+    for (int e = 0; e < VEC; e++) put((int64_t)cell * VEC + e, acc[e], idx[e]);
     return;
   }
   const int cols = cl * VEC, pitch = cols + 1;
 #pragma unroll
   for (int e = 0; e < VEC; e++) {
     const int at = lr * pitch + lc * VEC + e;
-    s_val[at] = mine(e);
-    if (KIND == COL_EXTREMUM) s_idx[at] = idx[e];
+    s_val[at] = acc[e];
+    if (INDEXED) s_idx[at] = idx[e];
   }
   __syncthreads();
   // `share` neighbouring lanes of one wavefront finish a column together
-  auto merge = [&](double& v, int64_t& i, double ov, int64_t oi) {
-    if (KIND == COL_SUM) {
-      v = op == TFHIP_SUM ? v + ov : v * ov;
-    } else if (KIND == COL_EXTREMUM) {
-      if ((want_max ? ov > v : ov < v) || (ov == v && oi < i)) {
-        v = ov;
-        i = oi;
-      }
-    } else {
-      v = v != 0.0 || ov != 0.0 ? 1.0 : 0.0;
-    }
-  };
   const int share = min(WAVE, max(1, rl / VEC));
   const int j = threadIdx.x & (share - 1);
   // (the same number of trips for all lanes: both are powers of two)
-  for (int c = threadIdx.x / share; c < cols; c += THREADS / share) {
+  for (int c = threadIdx.x / share; c < cols; c += COL_THREADS / share) {
     double v = s_val[j * pitch + c];
-    int64_t vi = KIND == COL_EXTREMUM ? s_idx[j * pitch + c] : 0;
+    int64_t vi = INDEXED ? s_idx[j * pitch + c] : 0;
     for (int r = j + share; r < rl; r += share)
-      merge(v, vi, s_val[r * pitch + c], KIND == COL_EXTREMUM ? s_idx[r * pitch + c] : 0);
+      merge_cols<KIND>(want_max, v, vi, s_val[r * pitch + c], INDEXED ? s_idx[r * pitch + c] : 0);
     for (int off = share >> 1; off > 0; off >>= 1) {
       const double ov = __shfl_down(v, off, WAVE);
-      const int64_t oi = KIND == COL_EXTREMUM ? __shfl_down(vi, off, WAVE) : 0;
-      merge(v, vi, ov, oi);
+      const int64_t oi = INDEXED ? __shfl_down(vi, off, WAVE) : 0;
+      merge_cols<KIND>(want_max, v, vi, ov, oi);
     }
     const int64_t at = (int64_t)cb * cols + c;
-    if (j == 0 && at < (int64_t)cells * VEC) put(at, v, vi);
+    if (j == 0 && at < columns) put(at, v, vi);
   }
+}
+
+// Combines the slices' partial results: a workgroup takes 32 columns, its 32 rows of lanes every
+// 32nd slice with 8 loads in flight, and the 32 results meet in LDS in ascending order.
+template <int KIND, typename OutT>
+__global__ __launch_bounds__(1024) void reduce_cols_finish_kernel(int op, const double* pval, const long long* pidx,
+                                                                  OutT* out, int64_t columns, int parts) {
+  constexpr bool INDEXED = KIND == COL_EXTREMUM;
+  constexpr int ROWS = 32, UNROLL = 8;
+  __shared__ double s_val[ROWS][32];
+  __shared__ int64_t s_idx[INDEXED ? ROWS : 1][32];
+  const int lane = threadIdx.x & 31, row = threadIdx.x >> 5;
+  const int64_t col = (int64_t)blockIdx.x * 32 + lane;
+  const bool want_max = op == TFHIP_MAX || op == TFHIP_ARGMAX;
+  // (a row without a slice repeats slice 0 of an extremum, and is neutral otherwise)
+  double v = KIND == COL_PROD ? 1.0 : 0.0;
+  int64_t vi = 0;
+  if (col < columns) {
+    if (INDEXED) {
+      v = pval[col];
+      vi = pidx[col];
+    }
+    for (int p = row; p < parts; p += ROWS * UNROLL) {
+      double b[UNROLL];
+      int64_t bi[UNROLL];
+#pragma unroll
+      for (int u = 0; u < UNROLL; u++) {
+        const int64_t at = (int64_t)min(p + u * ROWS, parts - 1) * columns + col;
+        b[u] = pval[at];
+        bi[u] = INDEXED ? pidx[at] : 0;
+      }
+#pragma unroll
+      for (int u = 0; u < UNROLL; u++)
+        if (p + u * ROWS < parts) merge_cols<KIND>(want_max, v, vi, b[u], bi[u]);
+    }
+  }
+  s_val[row][lane] = v;
+  if (INDEXED) s_idx[row][lane] = vi;
+  __syncthreads();
+  // sixteen lanes per column halve the 32 rows, then meet by shuffles
+  const int c = threadIdx.x >> 4, j = threadIdx.x & 15;
+  if (c >= 32) return;
+  double w = s_val[j][c];
+  int64_t wi = INDEXED ? s_idx[j][c] : 0;
+  merge_cols<KIND>(want_max, w, wi, s_val[j + 16][c], INDEXED ? s_idx[j + 16][c] : 0);
+  for (int off = 8; off > 0; off >>= 1) {
+    const double ov = __shfl_down(w, off, WAVE);
+    const int64_t oi = INDEXED ? __shfl_down(wi, off, WAVE) : 0;
+    merge_cols<KIND>(want_max, w, wi, ov, oi);
+  }
+  const int64_t at = (int64_t)blockIdx.x * 32 + c;
+  if (j == 0 && at < columns) out[at] = col_result<KIND, OutT>(op, w, wi);
 }
 
 // softmax over the last axis with the rounding points of the reference composite:
@@ -731,29 +784,28 @@ static ColPlan plan_reduce_cols(int64_t cells, int64_t lanes, int64_t red, int c
   // One launch while a row lane of a tall workgroup (512 lanes) has few elements to walk, or where
   // there are workgroups for every CU anyway: a second launch costs about 4 us.  A trip of eight
   // loads takes about 2.5 us whatever it reads, so the workgroup is made as tall as it takes to
-  // have one or two trips, down to four cell lanes (runs of 64 bytes): [1000, 512] 14.1 us with
-  // sixteen cell lanes, 9.5 with four (12 for the transposition and the row sum before).
+  // have one or two trips, down to four cell lanes (runs of 64 bytes): [1000, 512] 4.4 us with four
+  // (sixteen took half as long again; 12 for the transposition and the row sum before).
   // Beyond 2048 elements the reduced axis is cut instead.
   pl.shift = shift_for(16);
-  while (pl.shift > 2 && red > 8 * (int64_t)(512 >> pl.shift)) pl.shift--;
+  while (pl.shift > 2 && red > 8 * (int64_t)(COL_THREADS >> pl.shift)) pl.shift--;
   // And as wide as leaves every row lane eight elements while two workgroups per CU remain: with
   // many cells and a short axis most row lanes would have nothing.  A workgroup per outer index and
   // 16 lanes of it against this: [100352, 4, 8] 266 -> 6.4 us, [4000000, 2, 2] 7540 -> 37,
   // [100000, 10, 32] 272 -> 25, [4096, 64, 16] 14.4 -> 5.6.
   // (A launch counts its lanes in 32 bits: no more than 2^22 workgroups and a few.)
-  while (pl.shift < 9 && ((8 * (int64_t)(512 >> pl.shift) > red && cells >> (pl.shift + 1) >= 2 * cus) ||
+  while (pl.shift < 9 && ((8 * (int64_t)(COL_THREADS >> pl.shift) > red && cells >> (pl.shift + 1) >= 2 * cus) ||
                           cells >> pl.shift >= 1 << 22))
     pl.shift++;
   pl.cell_blocks = ceil_div(cells, (int64_t)1 << pl.shift);
   pl.seg = red;
-  if (red <= 16 * (int64_t)(512 >> pl.shift) || pl.cell_blocks >= 2 * cus) return pl;
-  // Slices of at least 16 elements a row lane, about eight workgroups of 256 lanes per CU.  (At
-  // least two of them: red is more than 16 times the row lanes, and there are fewer than 2 cus
+  if (red <= 16 * (int64_t)(COL_THREADS >> pl.shift) || pl.cell_blocks >= 2 * cus) return pl;
+  // Slices of at least 8 elements a row lane, about two workgroups per CU.  (At least two of them: red is more than 16 times the row lanes, and there are fewer than 2 cus
   // blocks of at most as many cells.)
   pl.shift = shift_for(64);
   pl.cell_blocks = ceil_div(cells, (int64_t)1 << pl.shift);
-  const int64_t rl = 256 >> pl.shift;
-  const int64_t parts = std::min<int64_t>(ceil_div(8 * (int64_t)cus, pl.cell_blocks), ceil_div(red, 16 * rl));
+  const int64_t rl = COL_THREADS >> pl.shift;
+  const int64_t parts = std::min<int64_t>(ceil_div(2 * (int64_t)cus, pl.cell_blocks), ceil_div(red, 8 * rl));
   pl.seg = ceil_div(ceil_div(red, parts), rl) * rl;
   pl.parts = (int)ceil_div(red, pl.seg);
   return pl;
@@ -764,7 +816,7 @@ static int launch_reduce_cols(tfhip_ctx* ctx, int op, const Buf* bx, const Buf* 
                               int64_t red, int64_t inner, float divisor) {
   const bool vec = bx->dtype == TFHIP_FLOAT32 && inner % 4 == 0 &&
                    (reinterpret_cast<uintptr_t>(bx->ptr) & 15) == 0;
-  const int64_t lanes = vec ? inner / 4 : inner, cells = outer * lanes;
+  const int64_t lanes = vec ? inner / 4 : inner, cells = outer * lanes, columns = outer * inner;
   if (cells > INDEX32) return ctx->fail(TFHIP_ENOTSUP, "reduce: too many columns");
   const ColPlan pl = plan_reduce_cols(cells, lanes, red, ctx->num_cus);
   const int64_t grid = pl.cell_blocks * pl.parts;
@@ -772,19 +824,20 @@ static int launch_reduce_cols(tfhip_ctx* ctx, int op, const Buf* bx, const Buf* 
   double* pval = nullptr;
   long long* pidx = nullptr;
   if (pl.parts > 1) {
-    const int64_t slots = outer * inner * pl.parts;
-    if (!partial.get((size_t)slots * 16)) return TFHIP_EDEVICE;
+    if (!partial.get((size_t)(columns * pl.parts) * 16)) return TFHIP_EDEVICE;
     pval = static_cast<double*>(partial.ptr);
-    pidx = reinterpret_cast<long long*>(pval + slots);
+    pidx = reinterpret_cast<long long*>(pval + columns * pl.parts);
   }
-  const unsigned threads = pl.parts > 1 ? 256 : 512;
-  auto kernel = pl.parts > 1 ? (vec ? reduce_cols_kernel<KIND, OutT, 4, 256> : reduce_cols_kernel<KIND, OutT, 1, 256>)
-                             : (vec ? reduce_cols_kernel<KIND, OutT, 4, 512> : reduce_cols_kernel<KIND, OutT, 1, 512>);
-  tfhip::launch(ctx, kernel, dim3((unsigned)grid), dim3(threads), 0, op, bx->ptr, bx->dtype, (OutT*)bo->ptr, pval,
+  auto kernel = vec ? reduce_cols_kernel<KIND, OutT, 4> : reduce_cols_kernel<KIND, OutT, 1>;
+  tfhip::launch(ctx, kernel, dim3((unsigned)grid), dim3(COL_THREADS), 0, op, bx->ptr, bx->dtype, (OutT*)bo->ptr, pval,
                 pidx, red, inner, (uint32_t)cells, Divisor(lanes), pl.shift, (uint32_t)pl.cell_blocks, pl.parts,
                 pl.seg, divisor);
   TFHIP_LAUNCH_CHECK_NAMED(ctx, "reduce_cols");
-  return pl.parts > 1 ? launch_reduce_finish(ctx, op, pval, pidx, bo, outer * inner, pl.parts) : TFHIP_OK;
+  if (pl.parts == 1) return TFHIP_OK;
+  tfhip::launch(ctx, reduce_cols_finish_kernel<KIND, OutT>, dim3((unsigned)ceil_div(columns, 32)), dim3(1024), 0, op,
+                pval, pidx, (OutT*)bo->ptr, columns, pl.parts);
+  TFHIP_LAUNCH_CHECK_NAMED(ctx, "reduce_finish");
+  return TFHIP_OK;
 }
 
 extern "C" int tfhip_reduce_axis(tfhip_ctx* ctx, int op, int64_t x, int64_t out, int64_t outer,
@@ -801,10 +854,15 @@ extern "C" int tfhip_reduce_axis(tfhip_ctx* ctx, int op, int64_t x, int64_t out,
   if (inner == 1) return reduce_rows(ctx, op, bx, bo, outer, red, (float)divisor);
   switch (op) {
     case TFHIP_SUM:
+      if (divisor != 1.0)
+        return launch_reduce_cols<COL_MEAN, float>(ctx, op, bx, bo, outer, red, inner, (float)divisor);
+      return bo->dtype == TFHIP_FLOAT32
+                 ? launch_reduce_cols<COL_SUM, float>(ctx, op, bx, bo, outer, red, inner, 1.f)
+                 : launch_reduce_cols<COL_SUM, int32_t>(ctx, op, bx, bo, outer, red, inner, 1.f);
     case TFHIP_PROD:
       return bo->dtype == TFHIP_FLOAT32
-                 ? launch_reduce_cols<COL_SUM, float>(ctx, op, bx, bo, outer, red, inner, (float)divisor)
-                 : launch_reduce_cols<COL_SUM, int32_t>(ctx, op, bx, bo, outer, red, inner, 1.f);
+                 ? launch_reduce_cols<COL_PROD, float>(ctx, op, bx, bo, outer, red, inner, 1.f)
+                 : launch_reduce_cols<COL_PROD, int32_t>(ctx, op, bx, bo, outer, red, inner, 1.f);
     case TFHIP_ALL:
     case TFHIP_ANY:
       return launch_reduce_cols<COL_LOGICAL, uint8_t>(ctx, op, bx, bo, outer, red, inner, 1.f);
