@@ -8,6 +8,7 @@
 // respect to the depthwise filter is a reduction over every output pixel: lanes run along
 // the channels, workgroups split the pixels, and a second kernel adds the partial sums in a
 // fixed order, so the result does not depend on scheduling.
+#include <algorithm>
 #include <cstring>
 
 #include "tfhip_internal.h"
@@ -86,31 +87,29 @@ __global__ __launch_bounds__(256) void depthwise_der_filter_partial_kernel(
         ((red[0][lane] + red[1][lane]) + red[2][lane]) + red[3][lane];
 }
 
-// dW[tap][d1][dm] = sum of the slices' partial sums: a workgroup takes 32 elements, its 8 rows of
-// lanes every 8th slice with 8 loads in flight, and the 8 sums are added in ascending order.  One
+// dW[tap][d1][dm] = sum of the slices' partial sums: a workgroup takes 32 elements, its 32 rows of
+// lanes every 32nd slice with 8 loads in flight, and the 32 sums are added in ascending order.  One
 // lane per element walking its slices alone was a chain of loads: 1152 elements of 512 slices took
-// 94 us, 4 here.
-__global__ __launch_bounds__(256) void depthwise_der_filter_finish_kernel(const double* partial, float* dw,
-                                                                          int64_t w_n, int slices) {
-  __shared__ double sums[8][32];
+// 94 us, 4 here; 896 slices take 5.8.
+__global__ __launch_bounds__(1024) void depthwise_der_filter_finish_kernel(const double* partial, float* dw,
+                                                                           int64_t w_n, int slices) {
+  constexpr int ROWS = 32, UNROLL = 8;
+  __shared__ double sums[ROWS][32];
   const int lane = threadIdx.x & 31, row = threadIdx.x >> 5;
   const int64_t g = (int64_t)blockIdx.x * 32 + lane;
   double s = 0.0;
-  if (g < w_n) {
-    int i = row;
-    for (; i + 56 < slices; i += 64) {
-      double v[8];
+  if (g < w_n)
+    for (int i = row; i < slices; i += ROWS * UNROLL) {
+      double v[UNROLL];
 #pragma unroll
-      for (int u = 0; u < 8; u++) v[u] = partial[(int64_t)(i + 8 * u) * w_n + g];
+      for (int u = 0; u < UNROLL; u++) v[u] = partial[(int64_t)min(i + u * ROWS, slices - 1) * w_n + g];
 #pragma unroll
-      for (int u = 0; u < 8; u++) s += v[u];
+      for (int u = 0; u < UNROLL; u++) s += i + u * ROWS < slices ? v[u] : 0.0;
     }
-    for (; i < slices; i += 8) s += partial[(int64_t)i * w_n + g];
-  }
   sums[row][lane] = s;
   __syncthreads();
   if (row == 0 && g < w_n) {
-    for (int r = 1; r < 8; r++) s += sums[r][lane];
+    for (int r = 1; r < ROWS; r++) s += sums[r][lane];
     dw[g] = (float)s;
   }
 }
@@ -159,7 +158,104 @@ __global__ __launch_bounds__(256) void depthwise_der_input_vec_kernel(
   *reinterpret_cast<f32x4*>(dx + (int64_t)g * 4) = acc;
 }
 
-// dW of a 3x3 depthwise filter (multiplier 1): one pass over the output pixels of a slice;
+// dW of a 3x3 depthwise filter (multiplier 1) at stride S.  A lane owns a channel quad and walks the
+// output rows of a column segment (a unit) with the nine taps' sums in registers: the window's rows
+// stay in registers from one output pixel to the next, so a pixel costs 3 S loads of x and one of dy
+// (those of the next row are in flight while a row is added), and neighbouring lanes share them in
+// L1.  Rows and columns beyond the image read 0 through the buffer descriptor.  The lanes of
+// a workgroup that share a quad are then added in a fixed order through LDS.
+// partial[slice][tap][c] in double.  Bound by the one read of x and dy from memory:
+// [32,56,56,128] 21.4 us (4.8 TB/s), at stride 2 13.8; ten loads a pixel, as below, 32.0 and 15.4.
+template <int S>
+__global__ __launch_bounds__(256) void depthwise3x3_der_filter_rows_kernel(
+    const float* __restrict__ x, const float* __restrict__ dy, double* __restrict__ partial,
+    const tfhip_conv2d_info ci, unsigned x_bytes, unsigned y_bytes, int quads_per_wave, int rows, uint32_t units,
+    Divisor by_w, Divisor by_segs) {
+  extern __shared__ __attribute__((aligned(16))) float red[];  // [256 lanes][9 taps][4]
+  constexpr int NB = S + 3;             // row buffers: three in use, S on their way
+  constexpr unsigned OOB = 0x80000000u;  // beyond any extent below 2 GiB
+  const int tid = threadIdx.x;
+  const int q_local = tid & (quads_per_wave - 1);       // quad within the channel block (a power of two)
+  const int subs = 256 / quads_per_wave, sub = tid / quads_per_wave;
+  const int c = (blockIdx.x * quads_per_wave + q_local) * 4;
+  const __amdgpu_buffer_rsrc_t rx =
+      __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(x), (short)0, (int)x_bytes, 0x00020000);
+  const __amdgpu_buffer_rsrc_t ry =
+      __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(dy), (short)0, (int)y_bytes, 0x00020000);
+  const unsigned x_row = (unsigned)ci.in_w * ci.in_c * 4u, y_row = (unsigned)ci.out_w * ci.out_c * 4u;
+  f32x4 acc[9];
+#pragma unroll
+  for (int k = 0; k < 9; k++) acc[k] = f32x4{0.f, 0.f, 0.f, 0.f};
+  if (c < ci.in_c)
+    for (uint32_t unit = blockIdx.y * subs + sub; unit < units; unit += gridDim.y * subs) {
+      uint32_t t = unit;
+      const int yc = (int)by_w.divmod(t), seg = (int)by_segs.divmod(t), n = (int)t;
+      const int y0 = seg * rows, y1 = min(y0 + rows, ci.out_h);
+      unsigned col[3];
+#pragma unroll
+      for (int j = 0; j < 3; j++) {
+        const int xc = yc * S - ci.pad_left + j;
+        col[j] = (unsigned)xc < (unsigned)ci.in_w ? ((unsigned)(n * ci.in_h * ci.in_w + xc) * ci.in_c + c) * 4u : OOB;
+      }
+      const unsigned y_at = ((unsigned)(n * ci.out_h * ci.out_w + yc) * ci.out_c + c) * 4u;
+      f32x4 v[NB][3], d[NB];
+      auto load_row = [&](int r, f32x4 (&to)[3]) {
+        const bool ok = (unsigned)r < (unsigned)ci.in_h && r <= (y1 - 1) * S - ci.pad_top + 2;
+#pragma unroll
+        for (int j = 0; j < 3; j++)
+          to[j] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                                                rx, (int)(ok && col[j] != OOB ? (unsigned)r * x_row + col[j] : OOB), 0, 0));
+      };
+      auto load_dy = [&](int y) {
+        return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                                             ry, (int)(y < y1 ? (unsigned)y * y_row + y_at : OOB), 0, 0));
+      };
+      const int first = y0 * S - ci.pad_top;
+#pragma unroll
+      for (int k = 0; k < 3; k++) load_row(first + k, v[k]);
+      d[0] = load_dy(y0);
+      for (int y = y0; y < y1; y += NB) {
+#pragma unroll
+        for (int u = 0; u < NB; u++) {
+          if (y + u < y1) {
+            const int r = (y + u) * S - ci.pad_top;
+#pragma unroll
+            for (int k = 0; k < S; k++) load_row(r + 3 + k, v[(u * S + 3 + k) % NB]);
+            d[(u + 1) % NB] = load_dy(y + u + 1);
+            __builtin_amdgcn_sched_barrier(0);  // loads first
+#pragma unroll
+            for (int i = 0; i < 3; i++)
+#pragma unroll
+              for (int j = 0; j < 3; j++) acc[i * 3 + j] += v[(u * S + i) % NB][j] * d[u];
+          }
+        }
+      }
+    }
+#pragma unroll
+  for (int k = 0; k < 9; k++) *reinterpret_cast<f32x4*>(red + (tid * 9 + k) * 4) = acc[k];
+  __syncthreads();
+  // thread -> (tap, quad): add the `subs` lanes of that quad in ascending order, in double
+  for (int item = tid; item < 9 * quads_per_wave; item += 256) {
+    const int k = item / quads_per_wave, q = item & (quads_per_wave - 1);
+    const int oc = (blockIdx.x * quads_per_wave + q) * 4;
+    if (oc >= ci.in_c) continue;
+    double s0 = 0.0, s1 = 0.0, s2 = 0.0, s3 = 0.0;
+    for (int r = 0; r < subs; r++) {
+      const float* p = red + ((r * quads_per_wave + q) * 9 + k) * 4;
+      s0 += (double)p[0];
+      s1 += (double)p[1];
+      s2 += (double)p[2];
+      s3 += (double)p[3];
+    }
+    double* out = partial + ((int64_t)blockIdx.y * 9 + k) * ci.in_c + oc;
+    out[0] = s0;
+    out[1] = s1;
+    out[2] = s2;
+    out[3] = s3;
+  }
+}
+
+// The same at any other stride, and for operands of 2 GiB and more: a pass over the output pixels of a slice;
 // a lane owns a channel quad and keeps the nine taps' sums, so dy is read once and the nine
 // x vectors of a pixel come from neighbouring rows that stay in cache.  The lanes of a
 // workgroup that share a quad (several pixels per wavefront when C / 4 < 64, and the four
@@ -445,6 +541,13 @@ static int check_geometry(tfhip_ctx* ctx, const char* op, const tfhip_conv2d_inf
   return TFHIP_OK;
 }
 
+static int der_filter_finish(tfhip_ctx* ctx, const void* partial, const Buf* bdw, int64_t w_n, int64_t slices) {
+  tfhip::launch(ctx, depthwise_der_filter_finish_kernel, dim3((unsigned)ceil_div(w_n, 32)), dim3(1024), 0,
+                static_cast<const double*>(partial), static_cast<float*>(bdw->ptr), w_n, (int)slices);
+  TFHIP_LAUNCH_CHECK_NAMED(ctx, "depthwise_der_filter_finish");
+  return TFHIP_OK;
+}
+
 static bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 
 static unsigned grid_for(tfhip_ctx* ctx, int64_t elements) {
@@ -553,6 +656,33 @@ extern "C" int tfhip_depthwise_conv2d_der_filter(tfhip_ctx* ctx, int64_t x, int6
   if ((rc = as_f32(ctx, bx, &tx, &xf))) return rc;
   if ((rc = as_f32(ctx, bdy, &tdy, &dyf))) return rc;
   const int64_t pixels = (int64_t)ci->batch * ci->out_h * ci->out_w;
+  // (buffer descriptors: both operands below 2 GiB)
+  if (ch_mul == 1 && ci->filter_h == 3 && ci->filter_w == 3 && ci->in_c % 4 == 0 && aligned16(xf) &&
+      aligned16(dyf) && pixels > 0 && x_n > 0 && x_n < (1 << 29) && y_n < (1 << 29) &&
+      ci->stride_h == ci->stride_w && ci->stride_h <= 2) {
+    const int c4 = ci->in_c / 4;
+    int qpw = 1;                       // channel quads per workgroup: a power of two <= 64
+    while (qpw < 64 && qpw < c4) qpw *= 2;
+    const int64_t blocks_c = ceil_div(c4, qpw);
+    const int subs = 256 / qpw;
+    // The columns of the output are cut into segments of at least 8 rows (a segment reads two rows of
+    // x more than it has) until four workgroups per CU, which is what their LDS allows, have
+    // one each.
+    const int64_t columns = (int64_t)ci->batch * ci->out_w, most = ceil_div((int64_t)ctx->num_cus * 4, blocks_c);
+    int64_t segs = std::max<int64_t>(1, std::min<int64_t>(most * subs / columns, ci->out_h / 8));
+    const int64_t rows = ceil_div(ci->out_h, segs);
+    segs = ceil_div(ci->out_h, rows);
+    const int64_t units = columns * segs, per_lane = ceil_div(units, most * subs);
+    const int64_t slices = ceil_div(units, per_lane * subs);
+    if (!tpart.get((size_t)(slices * w_n) * sizeof(double))) return TFHIP_EDEVICE;
+    ctx->name_kernel("depthwise3x3_der_filter");
+    tfhip::launch(ctx, ci->stride_h == 1 ? depthwise3x3_der_filter_rows_kernel<1> : depthwise3x3_der_filter_rows_kernel<2>,
+                  dim3((unsigned)blocks_c, (unsigned)slices), dim3(256), (size_t)(256 * 9 * 4 * sizeof(float)), xf, dyf,
+                  static_cast<double*>(tpart.ptr), *ci, (unsigned)(x_n * 4), (unsigned)(y_n * 4), qpw, (int)rows,
+                  (uint32_t)units, Divisor(ci->out_w), Divisor(segs));
+    TFHIP_LAUNCH_CHECK(ctx);
+    return der_filter_finish(ctx, tpart.ptr, bdw, w_n, slices);
+  }
   if (ch_mul == 1 && ci->filter_h == 3 && ci->filter_w == 3 && ci->in_c % 4 == 0 && aligned16(xf) &&
       aligned16(dyf) && pixels > 0 && pixels <= INDEX32) {
     const int c4 = ci->in_c / 4;
@@ -575,11 +705,7 @@ extern "C" int tfhip_depthwise_conv2d_der_filter(tfhip_ctx* ctx, int64_t x, int6
                        dim3(256), (size_t)(256 * 9 * 4 * sizeof(float)), xf, dyf,
                        static_cast<double*>(tpart.ptr), *ci, qpw, per_slice, Divisor(ci->out_w), Divisor(ci->out_h));
     TFHIP_LAUNCH_CHECK(ctx);
-    tfhip::launch(ctx, depthwise_der_filter_finish_kernel, dim3((unsigned)ceil_div(w_n, 32)), dim3(256),
-                       0, static_cast<const double*>(tpart.ptr),
-                       static_cast<float*>(bdw->ptr), w_n, (int)slices);
-    TFHIP_LAUNCH_CHECK(ctx);
-    return TFHIP_OK;
+    return der_filter_finish(ctx, tpart.ptr, bdw, w_n, slices);
   }
   // enough pixel slices to fill the machine, at least 64 pixels each
   const int64_t channel_blocks = ceil_div(ci->out_c, 64);
@@ -593,11 +719,7 @@ extern "C" int tfhip_depthwise_conv2d_der_filter(tfhip_ctx* ctx, int64_t x, int6
   tfhip::launch(ctx, depthwise_der_filter_partial_kernel,
                      dim3((unsigned)channel_blocks, (unsigned)taps, (unsigned)slices), dim3(256), 0, xf, dyf, static_cast<double*>(tpart.ptr), *ci, ch_mul, per_slice);
   TFHIP_LAUNCH_CHECK(ctx);
-  tfhip::launch(ctx, depthwise_der_filter_finish_kernel, dim3((unsigned)ceil_div(w_n, 32)), dim3(256),
-                     0, static_cast<const double*>(tpart.ptr),
-                     static_cast<float*>(bdw->ptr), w_n, (int)slices);
-  TFHIP_LAUNCH_CHECK(ctx);
-  return TFHIP_OK;
+  return der_filter_finish(ctx, tpart.ptr, bdw, w_n, slices);
 }
 
 extern "C" int tfhip_pool2d_backprop(tfhip_ctx* ctx, int64_t dy, int64_t x, int64_t dx,
