@@ -1,0 +1,141 @@
+"""The extension module of the Python host: tensor records, reference counts and scopes behave as the
+interpreted ones did, with backends written in Python, and hold nothing that was let go.  No GPU needed."""
+import gc
+import weakref
+
+import numpy as np
+import pytest
+
+from test_host_logic import FakeBackend
+
+
+@pytest.fixture
+def fake():
+    import tfhip
+    from tfhip.engine import ENGINE
+    be = FakeBackend()
+    tfhip.register_backend("fake-native", lambda: be, 0)
+    prev = ENGINE.backend_name
+    tfhip.set_backend("fake-native")
+    yield be
+    tfhip.remove_backend("fake-native")
+    if prev:
+        ENGINE.set_backend(prev)
+
+
+def counts():
+    import tfhip
+    m = tfhip.memory()
+    return m["numTensors"], m["numDataBuffers"], m["numBytes"]
+
+
+@pytest.mark.parametrize("kept", [0, 1, 3, 40])
+def test_scopes_keep_what_is_returned(fake, kept):
+    import tfhip as tf
+    base = counts()
+
+    def body():
+        made = [tf.tensor(np.zeros(i + 1, np.float32)) for i in range(50)]
+        inner = tf.tidy(lambda: {"a": made[:kept], "b": (tf.tensor(1.5),)})
+        return [inner, made[:kept]]
+    got = tf.tidy(body)
+    assert counts() == (base[0] + kept + 1, base[1] + kept + 1, base[2] + 4 * (sum(range(1, kept + 1)) + 1))
+    assert len(fake.live) == kept + 1
+    tf.dispose(got[1] + list(got[0]["b"]))
+    tf.dispose(got[1])                      # a second time is no error
+    assert counts() == base and not fake.live
+
+
+def test_errors_end_their_scopes(fake):
+    import tfhip as tf
+    from tfhip.engine import ENGINE
+    base = counts()
+
+    def body():
+        tf.tensor(np.ones(3, np.float32))
+        ENGINE.run_kernel(lambda be: tf.tensor(2.0) and be.nothing)
+    with pytest.raises(AttributeError, match="nothing"):
+        tf.tidy(body)
+    with pytest.raises(ZeroDivisionError):
+        with tf.tidy():
+            tf.tensor(np.ones(3, np.float32))
+            1 / 0
+    assert counts() == base and ENGINE.scopes == [] and not fake.live
+    with pytest.raises(IndexError):
+        ENGINE.end_scope()
+    fake.register = lambda *a: 1 / 0
+    with pytest.raises(ZeroDivisionError):
+        tf.tidy(lambda: tf.tensor(1.0))
+    del fake.register
+    assert ENGINE.scopes == []
+
+
+def test_records(fake):
+    from tfhip.engine import DataId, Tensor
+    t = Tensor([2.0, np.int64(3)], None, None, None, fake)
+    assert t.shape == (2, 3) and t.size == 6 and t.rank == 2 and t.dtype == "float32" and t.quant is None
+    assert type(t.shape[0]) is int and isinstance(t.data_id, DataId) and not t.is_disposed
+    other = Tensor((6,), "int32", t.data_id, backend=fake)
+    assert other.data_id is t.data_id and other.id == t.id + 1 and len(fake.live) == 1
+    t.note = "tensors take attributes"
+    t.dispose()
+    assert t.is_disposed and len(fake.live) == 1
+    other.dispose()
+    assert not fake.live
+    big = Tensor((2 ** 40, 2 ** 30, 0), "bool", backend=fake)
+    assert big.size == 0
+    big.dispose()
+    q = Tensor((4,), "float32", None, np.zeros(4, np.uint8), fake, (0.5, 1.0))
+    q.dispose()
+    with pytest.raises((TypeError, ValueError)):
+        Tensor(("a",), "float32", backend=fake)
+    with pytest.raises((AttributeError, RuntimeError)):
+        Tensor.__new__(Tensor).dispose()
+
+
+def test_nothing_is_held(fake):
+    import tfhip as tf
+    value = np.zeros(7, np.float32)
+    t = tf.tensor(value)
+    r = tf.reshape(t, (7, 1))
+    refs = [weakref.ref(t), weakref.ref(r), weakref.ref(t.data_id)]
+    tf.dispose([t, r])
+    del t, r
+    gc.collect()
+    assert [x() for x in refs] == [None] * 3
+
+    def step():
+        tf.tidy(lambda: [tf.reshape(tf.tensor(value), (1, 7)) for _ in range(4)][-1]).dispose()
+    for _ in range(10):
+        step()
+    gc.collect()
+    before = len(gc.get_objects())
+    for _ in range(200):
+        step()
+    gc.collect()
+    assert len(gc.get_objects()) <= before + 20
+
+
+def test_geometry_is_remembered_by_value_only():
+    from tfhip import shape_util as su
+    a = su.compute_conv2d_info((1, 9, 9, 4), (3, 3, 4, 8), 2, 1, "same")
+    want = dict(a, padInfo=dict(a["padInfo"]))
+    a["padInfo"]["top"] = a["inHeight"] = 77
+    assert su.compute_conv2d_info((1, 9, 9, 4), (3, 3, 4, 8), 2, 1, "same") == want
+    for strides in (2.0, (2.0, 2), [2, 2]):        # equal numbers of other types are computed anew
+        b = su.compute_conv2d_info((1, 9, 9, 4), (3, 3, 4, 8), strides, 1, "same")
+        assert b == want and type(b["strideHeight"]) is type(strides if type(strides) is float else strides[0])
+    c = su.compute_conv2d_info((1, 9, 9, 4), (3, 3, 4, 8), 2, 1, 0)
+    assert type(su.compute_conv2d_info((1, 9, 9, 4), (3, 3, 4, 8), 2, 1, 0.0)["padInfo"]["top"]) is float
+    assert type(c["padInfo"]["top"]) is int
+    for _ in range(2):
+        with pytest.raises(ValueError):
+            su.compute_conv2d_info((1, 9, 9, 4), (3, 3, 4, 8), 2, 1, "other")
+
+
+def test_the_entry_points_need_the_library():
+    from tfhip import _native
+    with pytest.raises(RuntimeError):
+        _native.load("/nonexistent.so")
+    with pytest.raises((TypeError, ValueError)):
+        _native.set_backend_class(dict)

@@ -3,6 +3,7 @@
 
   libtfjs_hip.so   HIP kernels + C ABI (include/tfjs_hip.h), gfx950 only
   tfjs_hip.node    N-API addon that exposes the C ABI to Node.js (needs node headers)
+  _native.*.so     CPython extension of the Python host (csrc/py_native.c)
 
 Usage: python tfjs-core_amd/build.py [--force] [--no-node]
 """
@@ -10,6 +11,7 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(HERE)
@@ -18,6 +20,7 @@ INCLUDE = os.path.join(ROOT, "include")
 LIB = os.path.join(HERE, "libtfjs_hip.so")
 ADDON = os.path.join(HERE, "js", "tfjs_hip.node")
 NODE_INCLUDE = "/usr/include/node"
+NATIVE = os.path.join(HERE, "python", "tfhip", "_native" + sysconfig.get_config_var("EXT_SUFFIX"))
 
 HIP_SOURCES = ["context.hip", "gemm.hip", "gemm_split.hip", "image.hip", "elementwise.hip", "reduce.hip",
                "shape_ops.hip", "backward.hip", "indexing.hip", "spectral.hip", "separable.hip"]
@@ -62,6 +65,18 @@ def build_lib(force=False, verbose=False):
     return LIB
 
 
+def build_native(force=False, verbose=False):
+    src = os.path.join(CSRC, "py_native.c")
+    if not force and not _stale(NATIVE, [src, os.path.join(INCLUDE, "tfjs_hip.h")]):
+        return NATIVE
+    cmd = [shutil.which("gcc") or "gcc", "-O2", "-Wall", "-shared", "-fPIC", "-I" + INCLUDE,
+           "-I" + sysconfig.get_paths()["include"], src, "-o", NATIVE, "-ldl"]
+    if verbose:
+        print(" ".join(cmd))
+    subprocess.check_call(cmd)
+    return NATIVE
+
+
 def build_addon(force=False, verbose=False):
     src = os.path.join(CSRC, "napi_addon.c")
     if not os.path.exists(src) or not os.path.isdir(NODE_INCLUDE):
@@ -82,6 +97,7 @@ def build_addon(force=False, verbose=False):
 def main(argv):
     force = "--force" in argv
     print(build_lib(force, verbose=True))
+    print(build_native(force, verbose=True))
     if "--no-node" not in argv:
         print(build_addon(force, verbose=True))
 

@@ -3,6 +3,8 @@ missing or no gfx950 device answers, callers get an exception."""
 import ctypes as C
 import os
 
+from . import _native
+
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.normpath(os.path.join(_HERE, "..", "..", "libtfjs_hip.so"))
 
@@ -127,5 +129,6 @@ def lib():
             fn.argtypes = args
             fn.restype = None if name == "tfhip_destroy" else (
                 C.c_char_p if name in ("tfhip_last_error", "tfhip_last_kernel") else C.c_int)
+        _native.load(LIB_PATH)
         _lib = l
     return _lib

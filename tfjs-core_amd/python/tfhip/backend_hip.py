@@ -1,13 +1,17 @@
 """MathBackendHIP: the KernelBackend of tfjs-core (tfjs-core/src/backends/backend.ts:91-649)
-on libtfjs_hip.so, Python twin of js/backend_hip.js.  Method names are the reference's in
+on libtfjs_hip.so, Python twin of js/backend_hip.js.  The table of buffers and the most frequent
+entry points (`_out`, `_h`, `_..._out`) are those of the extension module (csrc/py_native.c), the others
+go through ctypes.  Method names are the reference's in
 snake_case; every kernel returns a device-resident Tensor at once (work is queued on the
 context's stream), only read_sync / time wait for the device."""
 import ctypes as C
-import itertools
+import operator
+import struct
 
 import numpy as np
 
 from . import _capi as capi
+from . import _native
 from . import shape_util as su
 from .engine import ENGINE, NP_DTYPE, Tensor
 
@@ -37,6 +41,23 @@ def _info_c(ci):
         ci["outWidth"], ci["outChannels"], ci["strideHeight"], ci["strideWidth"],
         ci["dilationHeight"], ci["dilationWidth"], ci["filterHeight"], ci["filterWidth"],
         int(p["top"]), int(p["left"]), int(p["bottom"]), int(p["right"]))
+
+
+_GEOMETRY = operator.itemgetter(
+    "batchSize", "inHeight", "inWidth", "inChannels", "outHeight", "outWidth", "outChannels",
+    "strideHeight", "strideWidth", "dilationHeight", "dilationWidth", "filterHeight", "filterWidth")
+_PADS = operator.itemgetter("top", "left", "bottom", "right")
+_PACK = struct.Struct("=17i").pack
+
+
+def _packed(ci):
+    """A tfhip_conv2d_info as bytes; what is not whole numbers goes the checked way."""
+    if ci.get("dataFormat", "channelsLast") == "channelsLast":
+        try:
+            return _PACK(*_GEOMETRY(ci), *_PADS(ci["padInfo"]))
+        except struct.error:
+            pass
+    return bytes(_info_c(ci))
 
 
 class _CapturedGraph(object):
@@ -95,7 +116,12 @@ class _PendingRead:
             b.lib.tfhip_read_finish(b.ctx if b.ctx else None, self._ticket, None, 0)
 
 
-class MathBackendHIP(object):
+class MathBackendHIP(_native.BackendCore):
+    # data: DataId -> (handle, storage dtype code, numel)
+    def __new__(cls, *args, **kwargs):
+        capi.lib()  # (the extension module needs its entry points)
+        return super().__new__(cls)
+
     def __init__(self, device=0):
         self.lib = capi.lib()
         ctx = C.c_void_p()
@@ -103,8 +129,7 @@ class MathBackendHIP(object):
         if rc != 0:
             raise RuntimeError("hip backend: %s" % self.lib.tfhip_last_error(None).decode())
         self.ctx = ctx
-        self.data = {}      # DataId -> (handle, storage dtype code, numel)
-        self._ids = itertools.count(1)
+        self._bind(ctx.value)
 
     # ---- errors ----
     def _ck(self, rc):
@@ -112,14 +137,6 @@ class MathBackendHIP(object):
             raise RuntimeError(self.lib.tfhip_last_error(self.ctx).decode())
 
     # ---- TensorStorage (backend.ts:33-44) ----
-    def register(self, data_id, shape, dtype):
-        if data_id in self.data:
-            raise RuntimeError("Data buffer is already registered")
-        code = _DTYPE_CODE[dtype]
-        h = next(self._ids)
-        self._ck(self.lib.tfhip_register(self.ctx, h, _shape_arr(shape), len(shape), code))
-        self.data[data_id] = (h, code, su.size_from_shape(shape))
-
     def write(self, data_id, values):
         if values is None:
             raise ValueError("MathBackendHIP.write(): values can not be null")
@@ -127,7 +144,7 @@ class MathBackendHIP(object):
         arr = np.ascontiguousarray(values, dtype=_NP_OF_CODE[code]).ravel()
         if arr.size != numel:
             raise ValueError("write: %d values for a buffer of %d" % (arr.size, numel))
-        self._ck(self.lib.tfhip_write(self.ctx, h, arr.ctypes.data_as(C.c_void_p), arr.nbytes))
+        self._write(data_id, arr)
 
     def read_sync(self, data_id):
         h, code, numel = self.data[data_id]
@@ -156,11 +173,6 @@ class MathBackendHIP(object):
         owner = _PinnedBlock(self.lib, p.value, numel * np_dtype.itemsize)
         arr = np.frombuffer(owner.view, dtype=np_dtype, count=numel).reshape(shape)
         return arr
-
-    def dispose_data(self, data_id):
-        rec = self.data.pop(data_id, None)
-        if rec is not None:
-            self._ck(self.lib.tfhip_dispose(self.ctx, rec[0]))
 
     def memory(self):
         a, b, c = C.c_size_t(), C.c_size_t(), C.c_size_t()
@@ -231,24 +243,19 @@ class MathBackendHIP(object):
         if self.ctx is not None:
             self.lib.tfhip_destroy(self.ctx)
             self.ctx = None
+            self._bind(0)
             self.data.clear()
 
     # ---- helpers ----
-    def _h(self, t):
-        rec = self.data.get(t.data_id)
-        if rec is None:
-            # data living on another backend: moveData (backend.ts:52-57, engine.ts:361-363)
-            src = ENGINE.ref[t.data_id]
-            values = src[1].read_sync(t.data_id)
-            src[1].dispose_data(t.data_id)
-            self.register(t.data_id, t.shape, t.dtype)
-            self.write(t.data_id, values)
-            src[1] = self
-            rec = self.data[t.data_id]
-        return rec[0]
-
-    def _out(self, shape, dtype="float32"):
-        return Tensor.make(shape, {}, dtype, self)
+    def _move_here(self, t):
+        """Data living on another backend: moveData (backend.ts:52-57, engine.ts:361-363)."""
+        src = ENGINE.ref[t.data_id]
+        values = src[1].read_sync(t.data_id)
+        src[1].dispose_data(t.data_id)
+        self.register(t.data_id, t.shape, t.dtype)
+        self.write(t.data_id, values)
+        src[1] = self
+        return self.data[t.data_id][0]
 
     def _from_host(self, values):
         """A tensor of this backend holding a host array (float32 or int32)."""
@@ -324,13 +331,26 @@ class MathBackendHIP(object):
         return self._matmul(a, b, batch, m, n, k, transpose_a, transpose_b, bias, bk, activation,
                             prelu_activation_weights, pk)
 
-    def _matmul(self, a, b, batch, m, n, k, ta, tb, bias, bk, activation, prelu, pk):
-        out = self._out((batch, m, n))
-        self._ck(self.lib.tfhip_matmul(
-            self.ctx, self._h(a), self._h(b), self._h(out), batch, m, n, k, int(bool(ta)),
-            int(bool(tb)), self._h(bias) if bk else -1, bk, capi.ACT[activation],
-            self._h(prelu) if pk else -1, pk, self._q(b)))
-        return out
+    def _matmul(self, a, b, batch, m, n, k, ta, tb, bias, bk, activation, prelu, pk, out_shape=None):
+        return self._matmul_out(a, b, out_shape or (batch, m, n), batch, m, n, k, 1 if ta else 0,
+                                1 if tb else 0, bias, bk, capi.ACT[activation], prelu, pk)
+
+    def mat_mul_as(self, a, b, out_shape, batch, m, n, k, transpose_a, transpose_b, bias=None,
+                   activation="linear", prelu_activation_weights=None):
+        """Extension of the plug-in API: the batched product straight from operands of any rank into
+        `out_shape`, without a reshape before and after it.  None when the epilogue is one that
+        fused_batch_mat_mul does in separate passes."""
+        if activation not in capi.ACT or a.dtype != "float32":
+            return None
+        bk = pk = 0
+        if bias is not None:
+            bk = self._epilogue_kind(bias, (batch, m, n))
+        if activation == "prelu":
+            pk = self._epilogue_kind(prelu_activation_weights, (batch, m, n))
+        if bk is None or pk is None:
+            return None
+        return self._matmul(a, b, batch, m, n, k, transpose_a, transpose_b, bias, bk, activation,
+                            prelu_activation_weights, pk, out_shape)
 
     # channelsFirst (NCHW, backend_cpu.ts:1565-1572, 1698-1706, 1857-1865 walk the same loops
     # through other strides): the images are turned to NHWC, which the kernels stream with
@@ -364,13 +384,8 @@ class MathBackendHIP(object):
             if bias is not None:
                 r = self.add(r, bias)
             return self._map_activation(r, activation, prelu_activation_weights)
-        out = self._out(out_shape)
-        info = _info_c(conv_info)
-        self._ck(self.lib.tfhip_conv2d(
-            self.ctx, self._h(x), self._h(filter), self._h(out), C.byref(info),
-            self._h(bias) if bk else -1, bk, capi.ACT[activation],
-            self._h(prelu_activation_weights) if pk else -1, pk, self._q(filter)))
-        return out
+        return self._conv2d_out(x, filter, out_shape, _packed(conv_info), bias, bk, capi.ACT[activation],
+                                prelu_activation_weights, pk)
 
     # ---- memory-bound image kernels ----
     def depthwise_conv2d(self, x, filter, conv_info):
@@ -386,12 +401,7 @@ class MathBackendHIP(object):
             if bias is not None:
                 r = self.add(r, bias)
             return self._map_activation(r, activation, None)
-        out = self._out(out_shape)
-        info = _info_c(conv_info)
-        self._ck(self.lib.tfhip_depthwise_conv2d(
-            self.ctx, self._h(x), self._h(filter), self._h(out), C.byref(info),
-            self._h(bias) if bk else -1, bk, capi.ACT[activation], self._q(filter)))
-        return out
+        return self._depthwise_out(x, filter, out_shape, _packed(conv_info), bias, bk, capi.ACT[activation])
 
     def fused_separable_conv2d(self, x, depthwise_filter, pointwise_filter, conv_info,
                                depthwise_bias=None, depthwise_activation=None, bias=None,
@@ -409,21 +419,12 @@ class MathBackendHIP(object):
         if dk in (None, capi.BCAST_FULL) or pk in (None, capi.BCAST_FULL) or \
                 depthwise_activation not in acts or activation not in acts:
             return None
-        out = self._out(out_shape)
-        info = _info_c(conv_info)
-        self._ck(self.lib.tfhip_separable_conv2d(
-            self.ctx, self._h(x), self._h(depthwise_filter), self._h(pointwise_filter),
-            self._h(out), C.byref(info), self._h(depthwise_bias) if dk else -1, dk,
-            capi.ACT[depthwise_activation], self._h(bias) if pk else -1, pk, capi.ACT[activation],
-            self._q(depthwise_filter), self._q(pointwise_filter)))
-        return out
+        return self._separable_out(x, depthwise_filter, pointwise_filter, out_shape, _packed(conv_info),
+                                   depthwise_bias, dk, capi.ACT[depthwise_activation], bias, pk,
+                                   capi.ACT[activation])
 
     def _pool(self, x, conv_info, kind):
-        out = self._out(conv_info["outShape"])
-        info = _info_c(conv_info)
-        self._ck(self.lib.tfhip_pool2d(self.ctx, self._h(x), self._h(out), C.byref(info),
-                                       capi.POOL[kind]))
-        return out
+        return self._pool_out(x, conv_info["outShape"], _packed(conv_info), capi.POOL[kind])
 
     def avg_pool(self, x, conv_info):
         return self._pool(x, conv_info, "avg")
@@ -435,8 +436,8 @@ class MathBackendHIP(object):
     # ---- backward kernels (backend.ts:423-441, 456-465); conv_info is the forward op's ----
     def _backward(self, fn, a, b, out_shape, conv_info, *extra):
         out = self._out(out_shape)
-        info = _info_c(conv_info)
-        self._ck(fn(self.ctx, self._h(a), self._h(b), self._h(out), C.byref(info), *extra))
+        self._ck(fn(self.ctx, self._h(a), self._h(b), self._h(out),
+                    C.byref(capi.Conv2DInfoC.from_buffer_copy(_packed(conv_info))), *extra))
         return out
 
     def conv2d_der_input(self, dy, filter, conv_info):
@@ -475,17 +476,18 @@ class MathBackendHIP(object):
                               capi.POOL["avg"])
 
     # ---- elementwise ----
+    refuses_unfit_shapes = True  # binary operations check the broadcast themselves
+
     def _binary(self, op, a, b, out_dtype):
-        out_shape = su.broadcast_shape(a.shape, b.shape)
-        out = self._out(out_shape, out_dtype)
-        self._ck(self.lib.tfhip_binary(self.ctx, capi.BINARY[op], self._h(a), _shape_arr(a.shape),
-                                       a.rank, self._h(b), _shape_arr(b.shape), b.rank,
-                                       self._h(out)))
+        out = self._binary_out(capi.BINARY[op], a, b, out_dtype)
+        if out is None:
+            su.broadcast_shape(a.shape, b.shape)  # (says what does not fit)
+            raise ValueError("hip backend: rank above 64")
         return out
 
     @staticmethod
     def _arith_dtype(a, b):
-        dt = su.upcast_type(a.dtype, b.dtype)
+        dt = a.dtype if a.dtype == b.dtype else su.upcast_type(a.dtype, b.dtype)
         return "int32" if dt == "bool" else dt
 
     def add(self, a, b):
@@ -510,9 +512,7 @@ class MathBackendHIP(object):
         return self._binary("minimum", a, b, self._arith_dtype(a, b))
 
     def _unary(self, op, x, out_dtype="float32", p0=0.0, p1=0.0):
-        out = self._out(x.shape, out_dtype)
-        self._ck(self.lib.tfhip_unary(self.ctx, capi.UNARY[op], self._h(x), self._h(out), p0, p1))
-        return out
+        return self._unary_out(capi.UNARY[op], x, out_dtype, p0, p1)
 
     def relu(self, x):  # keeps the input dtype (backend_cpu.ts:1194)
         return self._unary("relu", x, "int32" if x.dtype != "float32" else "float32")
@@ -608,9 +608,7 @@ class MathBackendHIP(object):
             shape[shape.index(-1)] = x.size // known if known else 0
         if su.size_from_shape(shape) != x.size:
             raise ValueError("Size(%d) must match the product of shape %s" % (x.size, shape))
-        t = Tensor(shape, x.dtype, x.data_id, None, self)
-        t.quant = x.quant
-        return t
+        return self._alias(x, shape)
 
     # ---- reductions (innermost axes) ----
     def _reduce(self, op, x, axes, out_dtype):
@@ -618,11 +616,8 @@ class MathBackendHIP(object):
             raise ValueError("%s must be called with innermost axes, got %s for rank %d"
                              % (op, axes, x.rank))
         out_shape, red_shape = su.compute_out_and_reduce_shapes(x.shape, axes)
-        out = self._out(out_shape, out_dtype)
-        self._ck(self.lib.tfhip_reduce(self.ctx, capi.REDUCE[op], self._h(x), self._h(out),
-                                       su.size_from_shape(out_shape),
-                                       su.size_from_shape(red_shape)))
-        return out
+        return self._reduce_out(capi.REDUCE[op], x, out_shape, out_dtype, su.size_from_shape(out_shape),
+                                su.size_from_shape(red_shape))
 
     def reduce_block(self, op, x, axes, divisor=1.0):
         """Extension of the plug-in API: `op` ("sum", "prod", "max", "min", "all", "any", "arg_max",
@@ -633,12 +628,11 @@ class MathBackendHIP(object):
             dtype = su.upcast_type(x.dtype, "int32") if op in ("sum", "prod") else \
                 "float32" if x.dtype == "float32" else "int32"
         first, last = axes[0], axes[-1]
-        out = self._out(x.shape[:first] + x.shape[last + 1:], dtype)
-        self._ck(self.lib.tfhip_reduce_axis(
-            self.ctx, capi.REDUCE[op.replace("_", "")], self._h(x), self._h(out),
-            su.size_from_shape(x.shape[:first]), su.size_from_shape(x.shape[first:last + 1]),
-            su.size_from_shape(x.shape[last + 1:]), float(divisor)))
-        return out
+        shape = x.shape
+        before, after = shape[:first], shape[last + 1:]
+        return self._reduce_axis_out(
+            capi.REDUCE[op.replace("_", "")], x, before + after, dtype, su.size_from_shape(before),
+            su.size_from_shape(shape[first:last + 1]), su.size_from_shape(after), float(divisor))
 
     def sum(self, x, axes):
         return self._reduce("sum", x, axes, su.upcast_type(x.dtype, "int32"))
@@ -705,9 +699,7 @@ class MathBackendHIP(object):
         (ops/softmax.ts:45-79)."""
         cols = logits.shape[-1]
         rows = logits.size // cols if cols else 0
-        out = self._out(logits.shape)
-        self._ck(self.lib.tfhip_softmax_rows(self.ctx, self._h(logits), self._h(out), rows, cols))
-        return out
+        return self._softmax_out(logits, rows, cols)
 
     # ---- data movement ----
     def gather(self, x, indices, axis):
@@ -1015,3 +1007,6 @@ class MathBackendHIP(object):
         self._ck(self.lib.tfhip_transpose(self.ctx, self._h(x), _shape_arr(x.shape), x.rank,
                                           _shape_arr(perm), self._h(out)))
         return out
+
+
+_native.set_backend_class(MathBackendHIP)

@@ -1,41 +1,28 @@
 """Minimal engine of the Node-free driver: backend registry, data-id reference counts and
 tidy scopes, after tfjs-core/src/engine.ts:149-359 (registry / init / fallback),
-:502-572 (registerTensor / disposeTensor) and :365-411, 675-718 (tidy, scopes)."""
+:502-572 (registerTensor / disposeTensor) and :365-411, 675-718 (tidy, scopes).  The tensor
+record, the counts and the scopes are in the extension module (csrc/py_native.c)."""
 import contextlib
 import warnings
 
 import numpy as np
 
-from . import shape_util as su
+try:
+    from . import _native
+except ImportError as err:
+    raise ImportError("tfhip._native is not built: run `python tfjs-core_amd/build.py` (%s)" % err)
 
 NP_DTYPE = {"float32": np.float32, "int32": np.int32, "bool": np.uint8}
 
-
-class DataId(object):
-    """Opaque key of one backend buffer (tensor.ts:416)."""
-    __slots__ = ("__weakref__",)
+DataId = _native.DataId
 
 
-class Tensor(object):
-    _next_id = 0
-
-    def __init__(self, shape, dtype, data_id=None, values=None, backend=None, quant=None,
-                 storage_dtype=None):
-        self.shape = tuple(map(int, shape))
-        self.dtype = dtype or "float32"
-        self.size = su.size_from_shape(self.shape)
-        self.rank = len(self.shape)
-        self.data_id = data_id if data_id is not None else DataId()
-        self.quant = quant  # (scale, min) when the buffer holds uint8 affine-quantised weights
-        self.is_disposed = False
-        self.id = Tensor._next_id
-        Tensor._next_id += 1
-        # storage_dtype: element type of the buffer when it differs from the tensor's dtype
-        # (a float32 tensor over int32 data after a widening cast, quantised weights)
-        ENGINE.register_tensor(self, backend,
-                               storage_dtype or ("uint8q" if quant else self.dtype))
-        if values is not None:
-            ENGINE.write(backend, self.data_id, values)
+class Tensor(_native.TensorBase):
+    """Tensor(shape, dtype, data_id=None, values=None, backend=None, quant=None, storage_dtype=None):
+    a view of the buffer `data_id` stands for, a new one of `values` when it is None.  quant:
+    (scale, min) when the buffer holds uint8 affine-quantised weights.  storage_dtype: element type
+    of the buffer when it differs from the tensor's dtype (a float32 tensor over int32 data
+    after a widening cast, quantised weights)."""
 
     @staticmethod
     def make(shape, data, dtype=None, backend=None):
@@ -67,11 +54,6 @@ class Tensor(object):
                 return (vals.astype(np.uint8) if as_bool else vals).reshape(shape)
         return _Data()
 
-    def dispose(self):
-        if not self.is_disposed:
-            ENGINE.dispose_tensor(self)
-            self.is_disposed = True
-
     def reshape(self, shape):
         self._check()
         return ENGINE.backend.reshape(self, shape)
@@ -80,17 +62,11 @@ class Tensor(object):
         return "Tensor(shape=%s, dtype=%s)" % (self.shape, self.dtype)
 
 
-class Engine(object):
+class Engine(_native.EngineCore):
     def __init__(self):
         self.registry = {}        # name -> backend instance
         self.factories = {}       # name -> (factory, priority)
         self.backend_name = None
-        self._backend = None
-        self.ref = {}             # data_id -> [refcount, backend, nbytes]
-        self.scopes = []
-        self.num_tensors = 0
-        self.num_bytes = 0
-        self.num_data_buffers = 0
 
     # ---- registry (engine.ts:220-359) ----
     def register_backend(self, name, factory, priority=1):
@@ -151,20 +127,6 @@ class Engine(object):
             self._backend = None
 
     # ---- tensors (engine.ts:502-572, 833-865) ----
-    def register_tensor(self, t, backend, storage_dtype):
-        backend = backend or self.backend
-        rec = self.ref.get(t.data_id)
-        if rec is None:
-            nbytes = t.size * (1 if storage_dtype in ("bool", "uint8q") else 4)
-            rec = self.ref[t.data_id] = [0, backend, nbytes]
-            self.num_data_buffers += 1
-            self.num_bytes += nbytes
-            backend.register(t.data_id, t.shape, storage_dtype)
-        rec[0] += 1
-        self.num_tensors += 1
-        if self.scopes:
-            self.scopes[-1].append(t)
-
     def write(self, backend, data_id, values):
         rec = self.ref[data_id]
         (backend or rec[1]).write(data_id, values)
@@ -175,19 +137,6 @@ class Engine(object):
     def read(self, data_id):
         return self.ref[data_id][1].read(data_id)
 
-    def dispose_tensor(self, t):
-        rec = self.ref.get(t.data_id)
-        if rec is None:
-            return
-        self.num_tensors -= 1
-        if rec[0] <= 1:
-            rec[1].dispose_data(t.data_id)
-            self.num_data_buffers -= 1
-            self.num_bytes -= rec[2]
-            del self.ref[t.data_id]
-        else:
-            rec[0] -= 1
-
     def memory(self):
         info = dict(numTensors=self.num_tensors, numDataBuffers=self.num_data_buffers,
                     numBytes=self.num_bytes, unreliable=False)
@@ -195,34 +144,8 @@ class Engine(object):
         return info
 
     # ---- scopes (engine.ts:365-411, 675-718) ----
-    def start_scope(self):
-        self.scopes.append([])
-
-    def end_scope(self, result=None):
-        scope = self.scopes.pop()
-        if not scope:
-            return
-        # (one tensor is what nearly every operation returns)
-        keep = (result,) if isinstance(result, Tensor) else _flatten_tensors(result)
-        keep = {id(t) for t in keep}
-        outer = self.scopes[-1] if self.scopes else None
-        for t in scope:
-            if id(t) in keep:
-                if outer is not None:
-                    outer.append(t)
-            elif not t.is_disposed:
-                t.dispose()
-
     def tidy(self, fn=None):
-        if fn is None:
-            return self._tidy_ctx()
-        self.start_scope()
-        result = None
-        try:
-            result = fn()
-            return result
-        finally:
-            self.end_scope(result)
+        return self._tidy_ctx() if fn is None else self.scoped(fn)
 
     @contextlib.contextmanager
     def _tidy_ctx(self):
@@ -231,17 +154,6 @@ class Engine(object):
             yield
         finally:
             self.end_scope(None)
-
-    def run_kernel(self, forward):
-        """ENGINE.runKernel without a tape (engine.ts:435-498): the forward function gets the
-        active backend; intermediates made inside are released when it returns."""
-        self.scopes.append([])
-        result = None
-        try:
-            result = forward(self._backend or self.backend)
-            return result
-        finally:
-            self.end_scope(result)
 
 
 def _flatten_tensors(r):
@@ -258,3 +170,4 @@ def _flatten_tensors(r):
 
 
 ENGINE = Engine()
+_native.set_engine(ENGINE, Tensor, _flatten_tensors)

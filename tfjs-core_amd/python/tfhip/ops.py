@@ -23,6 +23,8 @@ def tensor(values, shape=None, dtype=None):
     """tf.tensor (ops/tensor_ops.ts:55-59, 108-112)."""
     if isinstance(values, Tensor):
         return values
+    if type(values) is float and shape is None and dtype is None:
+        return Tensor((), "float32", None, np.array((values,), np.float32))
     arr = np.asarray(values)
     if dtype is None:
         dtype = _dtype_of(arr)
@@ -100,37 +102,43 @@ def _matmul_prep(a, b, transpose_a, transpose_b, name):
         raise ValueError("Error in %s: inner shapes (%d) and (%d) of Tensors with shapes %s and "
                          "%s and transposeA=%s and transposeB=%s must match."
                          % (name, inner_a, inner_b, a.shape, b.shape, transpose_a, transpose_b))
-    batch = su.size_from_shape(dims_a)
-    out_shape = tuple(dims_a) + (outer_a, outer_b)
-    a3 = (batch, inner_a, outer_a) if transpose_a else (batch, outer_a, inner_a)
-    b3 = (batch, outer_b, inner_b) if transpose_b else (batch, inner_b, outer_b)
-    return a, b, a3, b3, out_shape
+    return a, b, su.size_from_shape(dims_a), outer_a, outer_b, inner_a, dims_a + (outer_a, outer_b)
 
 
-def matmul(a, b, transpose_a=False, transpose_b=False):
-    a, b, a3, b3, out_shape = _matmul_prep(a, b, transpose_a, transpose_b, "matMul")
-
+def _mat_mul(a, b, batch, m, n, k, out_shape, transpose_a, transpose_b, *epilogue):
+    """The product on the active backend: in one call where the backend takes operands of any rank
+    (feature detection), else as rank 3, as the reference does."""
     def fwd(be):
-        r = be.batch_mat_mul(be.reshape(a, a3), be.reshape(b, b3), transpose_a, transpose_b)
+        if hasattr(be, "mat_mul_as"):
+            r = be.mat_mul_as(a, b, out_shape, batch, m, n, k, transpose_a, transpose_b, *epilogue)
+            if r is not None:
+                return r
+        a3 = be.reshape(a, (batch, k, m) if transpose_a else (batch, m, k))
+        b3 = be.reshape(b, (batch, n, k) if transpose_b else (batch, k, n))
+        if epilogue:
+            r = be.fused_batch_mat_mul(a3, b3, transpose_a, transpose_b, *epilogue)
+        else:
+            r = be.batch_mat_mul(a3, b3, transpose_a, transpose_b)
         return be.reshape(r, out_shape)
     return ENGINE.run_kernel(fwd)
 
 
+def matmul(a, b, transpose_a=False, transpose_b=False):
+    a, b, batch, m, n, k, out_shape = _matmul_prep(a, b, transpose_a, transpose_b, "matMul")
+    return _mat_mul(a, b, batch, m, n, k, out_shape, transpose_a, transpose_b)
+
+
 def fused_matmul(a, b, transpose_a=False, transpose_b=False, bias=None, activation="linear",
                  prelu_activation_weights=None):
-    a, b, a3, b3, out_shape = _matmul_prep(a, b, transpose_a, transpose_b, "fused matMul")
+    a, b, batch, m, n, k, out_shape = _matmul_prep(a, b, transpose_a, transpose_b, "fused matMul")
     if bias is not None:
         bias = _conv(bias, "bias", "fused matMul")
         bias, _ = _types_match(bias, a)
         su.broadcast_shape(out_shape, bias.shape)
     if prelu_activation_weights is not None:
         prelu_activation_weights = _conv(prelu_activation_weights, "prelu weights", "fused matMul")
-
-    def fwd(be):
-        r = be.fused_batch_mat_mul(be.reshape(a, a3), be.reshape(b, b3), transpose_a, transpose_b,
-                                   bias, activation, prelu_activation_weights)
-        return be.reshape(r, out_shape)
-    return ENGINE.run_kernel(fwd)
+    return _mat_mul(a, b, batch, m, n, k, out_shape, transpose_a, transpose_b, bias, activation,
+                    prelu_activation_weights)
 
 
 # ---- convolutions (ops/conv.ts:145-217, 470-540; ops/fused_ops.ts:276-425) ----
@@ -302,7 +310,8 @@ def pool(x, window_shape, pooling_type, pad, dilations=None, strides=None):
 # ---- elementwise ----
 def _binary(name, method, a, b):
     a, b = _types_match(_conv(a, "a", name), _conv(b, "b", name))
-    su.broadcast_shape(a.shape, b.shape)
+    if a.shape != b.shape and not hasattr(ENGINE.backend, "refuses_unfit_shapes"):
+        su.broadcast_shape(a.shape, b.shape)
     return ENGINE.run_kernel(lambda be: getattr(be, method)(a, b))
 
 

@@ -1,6 +1,7 @@
 """Host-side shape math of the op wrappers: the Python twin of js/conv_util.js,
 js/broadcast_util.js and js/axis_util.js.  Follows tfjs-core/src/ops/conv_util.ts:66-182,
 296-320, 391-435, ops/broadcast_util.ts:27-87 and ops/axis_util.ts:24-109."""
+import functools
 import math
 
 
@@ -12,7 +13,7 @@ def size_from_shape(shape):
 
 
 def _tuple2(v):
-    if isinstance(v, (int, float)):
+    if type(v) is int or isinstance(v, (int, float)):
         return (v, v)
     return (v[0], v[1])
 
@@ -60,8 +61,36 @@ def _out_shape_2d(in_hw, field, stride, zero_pad, mode):
     return int(rows), int(cols)
 
 
+_ONLY_INT = {int}
+
+
+def _whole(v):
+    """A whole number, or a pair of them, of type int and no other."""
+    return type(v) is int or (type(v) is tuple and len(v) == 2 and type(v[0]) is type(v[1]) is int)
+
+
 def compute_conv2d_info(in_shape, filter_shape, strides, dilations, pad, rounding_mode=None,
                         depthwise=False, data_format="channelsLast"):
+    # The geometry of a layer is computed for the first call and copied for the next ones (4.5 us
+    # against 1); only for arguments whose types leave nothing that compares equal and is not.
+    if type(in_shape) is tuple and type(filter_shape) is tuple and _whole(strides) and \
+            _whole(dilations) and type(pad) in (int, str) and rounding_mode is None and \
+            {*map(type, in_shape), *map(type, filter_shape)} == _ONLY_INT:
+        ci = _remembered_conv2d_info(in_shape, filter_shape, strides, dilations, pad,
+                                     bool(depthwise), data_format)
+        return dict(ci, padInfo=dict(ci["padInfo"]))
+    return _compute_conv2d_info(in_shape, filter_shape, strides, dilations, pad, rounding_mode,
+                                depthwise, data_format)
+
+
+@functools.lru_cache(maxsize=1024)
+def _remembered_conv2d_info(in_shape, filter_shape, strides, dilations, pad, depthwise, data_format):
+    return _compute_conv2d_info(in_shape, filter_shape, strides, dilations, pad, None, depthwise,
+                                data_format)
+
+
+def _compute_conv2d_info(in_shape, filter_shape, strides, dilations, pad, rounding_mode, depthwise,
+                         data_format):
     if data_format == "channelsLast":
         batch, in_h, in_w, in_c = in_shape
     elif data_format == "channelsFirst":
