@@ -222,6 +222,36 @@ static int handle_of(BackendObject* be, PyObject* t, int64_t* handle) {
   return *handle == -1 && PyErr_Occurred() ? -1 : 0;
 }
 
+/* Contiguous values of the stored type straight to the library; 0: not such values (the Python
+ * method converts them, or refuses), 1: written, -1: failed. */
+static int backend_write_plain(BackendObject* be, PyObject* data_id, PyObject* values) {
+  static const char formats[] = {'f', 'i', 'B', 'B'};
+  PyObject* rec = PyDict_GetItemWithError(be->data, data_id);
+  if (!rec) return PyErr_Occurred() ? -1 : 0;
+  const long long handle = PyLong_AsLongLong(PyTuple_GET_ITEM(rec, 0));
+  const long code = PyLong_AsLong(PyTuple_GET_ITEM(rec, 1));
+  const long long count = PyLong_AsLongLong(PyTuple_GET_ITEM(rec, 2));
+  if (PyErr_Occurred()) return -1;
+  Py_buffer view;
+  if (!PyObject_CheckBuffer(values)) return 0;
+  if (PyObject_GetBuffer(values, &view, PyBUF_C_CONTIGUOUS | PyBUF_FORMAT)) {
+    PyErr_Clear();
+    return 0;
+  }
+  int rc = 0;
+  const int fits = code >= 0 && code < 4 && view.format && view.format[0] == formats[code] && !view.format[1] &&
+                   view.itemsize == (code == TFHIP_FLOAT32 || code == TFHIP_INT32 ? 4 : 1) &&
+                   view.len == count * view.itemsize;
+  if (fits) {
+    Py_BEGIN_ALLOW_THREADS
+    rc = api.tfhip_write(be->ctx, handle, view.buf, (size_t)view.len);
+    Py_END_ALLOW_THREADS
+  }
+  PyBuffer_Release(&view);
+  if (!fits) return 0;
+  return check(be, rc) ? -1 : 1;
+}
+
 /* ---- engine -------------------------------------------------------------------------------- */
 static int engine_register(EngineObject* e, TensorObject* t, PyObject* backend, PyObject* storage) {
   PyObject* be = backend && backend != Py_None ? backend : e->backend;
@@ -540,6 +570,11 @@ static int Tensor_init(TensorObject* t, PyObject* args, PyObject* kwds) {
   int rc = tensor_fill(t, dims, dtype, data_id, backend, quant, storage);
   Py_DECREF(dims);
   if (!rc && values != Py_None) {
+    PyObject* to = backend != Py_None ? backend : engine->backend;
+    if (Py_TYPE(to) == backend_class) {
+      const int written = backend_write_plain((BackendObject*)to, t->data_id, values);
+      if (written) return written > 0 ? 0 : -1;
+    }
     PyObject* r = PyObject_CallMethodObjArgs((PyObject*)engine, s_write, backend, t->data_id, values, NULL);
     rc = r ? 0 : -1;
     Py_XDECREF(r);

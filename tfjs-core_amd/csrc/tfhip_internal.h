@@ -12,6 +12,7 @@
 #include <string>
 #include <tuple>
 #include <unordered_map>
+#include <unordered_set>
 #include <utility>
 #include <vector>
 
@@ -128,6 +129,14 @@ struct tfhip_ctx {
   static constexpr unsigned char kAllStreams = (unsigned char)((1u << kStreams) - 1);
   hipStream_t streams[kStreams] = {};
   int cur = 0;  // index of `stream`
+  // Streams on which nothing was queued since the host last waited for them (a bit per stream).  (Asking
+  // the driver costs up to 10 us where there is work.)
+  unsigned char idle = kAllStreams;
+  std::unordered_set<void*> quiet;  // free blocks that came back while every stream was idle: no work left on them
+  // A pinned block per compute stream for a larger write that finds the stream idle: the copy out of it
+  // runs on that stream, so an idle stream also says that the block is free.
+  char* stages[kStreams] = {};
+  char* idle_stage();  // the selected stream's block, or nullptr (work is queued, or no memory)
   // Streams that may hold queued work which a graph replay has not been ordered behind yet (a bit
   // per stream, set when the stream is selected): a replay waits for these, see tfhip_graph_launch.
   unsigned char dirty = 1;
