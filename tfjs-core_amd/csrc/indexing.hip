@@ -4,6 +4,7 @@
 // reference.  Every result element is produced by one lane that visits its contributions in
 // the order the reference's loops do, so sums round the same way and nothing depends on
 // scheduling (no atomics on data).
+#include <algorithm>
 #include <climits>
 #include <type_traits>
 
@@ -72,8 +73,8 @@ __global__ void gather_rows_vec_kernel(const uint4* x, const int64_t* flat, uint
 // whenever an update addresses its row, which is the order backend_cpu.ts:3858-3886 applies
 // them in.  Acc = T rounds every sum to the element type as a typed array does; Acc = double
 // rounds once at the end, as the masked sums of unsortedSegmentSum do.
-template <typename T, typename Acc>
-__global__ __launch_bounds__(256) void scatter_rows_kernel(const int64_t* flat, const T* updates, T* out,
+template <typename T, typename Acc, typename I>
+__global__ __launch_bounds__(256) void scatter_rows_kernel(const I* flat, const T* updates, T* out,
                                                            int64_t rows, int64_t slice, int64_t n_updates,
                                                            T start, int sum_dupes, int scalar_update) {
   // the index list passes through LDS 256 entries at a time: every lane of the workgroup walks
@@ -112,38 +113,44 @@ __global__ __launch_bounds__(256) void scatter_rows_kernel(const int64_t* flat, 
 
 // The same for slices of 32 elements and more (an embedding's gradient).  The kernel above walks
 // the whole index list for every 256 result elements, which is what it is bound by: 10240 updates
-// of 128 into 20000 rows took 1980 us; 64 here.  A workgroup owns the rows f with
+// of 128 into 20000 rows took 1980 us; 25.5 here.  A workgroup of 16 or 4 wavefronts owns the rows f with
 // f % groups = its number (so that the frequent rows of a text, which have neighbouring numbers,
 // go to different workgroups) and 64 columns for each of CW wavefronts side by side: it walks the
-// list once, 4096 entries at a time with 16 loads in flight per lane, and packs the entries of its
-// rows, in order, into LDS.  A wavefront then takes a row, finds its entries by ballot and adds
-// them in ascending order, up to 64 updates in flight: what bounds it is the most frequent row, a
-// chain of hundreds of additions.  The sums lie in LDS between passes; every one is taken in the
-// order of the list, as above.
+// list once, 4096 entries at a time, and packs the entries of its rows, in order, into LDS, counting
+// them per row.  A set of CW wavefronts then takes a row that has any, finds its entries by ballot
+// and adds them in ascending order, up to 64 updates in flight.  What bounds it is the most frequent
+// row, a chain of hundreds of additions: sums that are rounded once at the end (Acc = double) of a
+// row with more than HOT entries in the pass are cut over the sets, 64 list entries in turn each,
+// and their parts added in the order of the sets (one set for the whole chain, four wavefronts: 64 us).
+// The sums lie in LDS between passes; every other one is taken in the order of the list, as above.
 constexpr int SCATTER_PASS = 4096;
-template <typename T, typename Acc, int CW>
-__global__ __launch_bounds__(256) void scatter_groups_kernel(const int64_t* __restrict__ flat,
-                                                             const T* __restrict__ updates, T* __restrict__ out,
-                                                             int rows, int64_t slice, int64_t n_updates,
-                                                             T start, int sum_dupes, int scalar_update,
-                                                             int group_shift, int local_rows) {
-  constexpr int PER = SCATTER_PASS / 256, CB = 64 * CW, ROW_WAVES = 4 / CW;
+template <typename T, typename Acc, int CW, int THREADS, typename I>
+__global__ __launch_bounds__(THREADS) void scatter_groups_kernel(
+    const I* __restrict__ flat, const T* __restrict__ updates, T* __restrict__ out, int rows, int64_t slice,
+    int64_t n_updates, T start, int sum_dupes, int scalar_update, int group_shift, int local_rows) {
+  constexpr int WAVES = THREADS / 64, PER = SCATTER_PASS / THREADS, CB = 64 * CW, SETS = WAVES / CW;
+  static_assert(PER * WAVES == 64, "the counts of a pass are one wavefront's prefix sum");
+  constexpr bool CUT = !std::is_same<T, Acc>::value && SETS > 1;
+  constexpr int HOT = 64;
   extern __shared__ __attribute__((aligned(16))) char scatter_lds[];
-  Acc* sums = reinterpret_cast<Acc*>(scatter_lds);  // [local_rows][CB]
-  __shared__ unsigned list[SCATTER_PASS];           // local row << 12 | entry of the pass
-  __shared__ int first[PER * 4 + 1];                // where a wavefront's entries of a load begin
+  Acc* sums = reinterpret_cast<Acc*>(scatter_lds);               // [local_rows][CB]
+  int* counts = reinterpret_cast<int*>(sums + local_rows * CB);  // entries of the pass per row
+  __shared__ unsigned list[SCATTER_PASS];                        // local row << 12 | entry of the pass
+  __shared__ int first[65];                                      // where a wavefront's entries of a load begin
+  __shared__ Acc parts[CUT ? SETS * CB : 1];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int groups = 1 << group_shift, mine = (int)blockIdx.x;
-  const int own = (wave % CW) * 64 + lane;          // column within the block
+  const int groups = 1 << group_shift, mine = (int)(blockIdx.z * gridDim.x + blockIdx.x);
+  const int set = wave / CW, own = (wave % CW) * 64 + lane;      // column within the block
   const int64_t col = (int64_t)blockIdx.y * CB + own;
   const bool stored = col < slice;
-  const int64_t read_col = stored ? col : 0;        // (a column past the slice: summed, not stored)
-  for (int i = tid; i < local_rows * CB; i += 256) sums[i] = (Acc)start;
+  const int64_t read_col = stored ? col : 0;                     // (a column past the slice: summed, not stored)
+  for (int i = tid; i < local_rows * CB; i += THREADS) sums[i] = (Acc)start;
   for (int64_t i0 = 0; i0 < n_updates; i0 += SCATTER_PASS) {
-    int64_t f[PER];
+    for (int i = tid; i < local_rows; i += THREADS) counts[i] = 0;
+    I f[PER];
 #pragma unroll
     for (int u = 0; u < PER; u++) {
-      const int64_t i = i0 + u * 256 + tid;
+      const int64_t i = i0 + u * THREADS + tid;
       f[u] = i < n_updates ? flat[i] : -1;
     }
     unsigned long long hit[PER];
@@ -151,7 +158,7 @@ __global__ __launch_bounds__(256) void scatter_groups_kernel(const int64_t* __re
     for (int u = 0; u < PER; u++) {
       const bool in = f[u] >= 0 && f[u] < rows && ((int)f[u] & (groups - 1)) == mine;
       hit[u] = __ballot(in);
-      if (lane == 0) first[u * 4 + wave] = __popcll(hit[u]);
+      if (lane == 0) first[u * WAVES + wave] = __popcll(hit[u]);
     }
     __syncthreads();
     if (wave == 0) {  // 64 counts into their prefix sums
@@ -168,96 +175,133 @@ __global__ __launch_bounds__(256) void scatter_groups_kernel(const int64_t* __re
     const int total = __builtin_amdgcn_readfirstlane(first[64]);
 #pragma unroll
     for (int u = 0; u < PER; u++)
-      if (hit[u] >> lane & 1)
-        list[first[u * 4 + wave] + __popcll(hit[u] & ((1ull << lane) - 1))] =
-            (unsigned)((int)f[u] >> group_shift) << 12 | (unsigned)(u * 256 + tid);
+      if (hit[u] >> lane & 1) {
+        const int r = (int)f[u] >> group_shift;
+        list[first[u * WAVES + wave] + __popcll(hit[u] & ((1ull << lane) - 1))] =
+            (unsigned)r << 12 | (unsigned)(u * THREADS + tid);
+        atomicAdd(&counts[r], 1);
+      }
     __syncthreads();
     const T* pass_updates = updates + (scalar_update ? 0 : i0 * slice);
     const int64_t step = scalar_update ? 0 : slice;
     const int64_t at_col = scalar_update ? 0 : read_col;
-    for (int r = wave / CW; r < local_rows && total > 0; r += ROW_WAVES) {
-      Acc acc = sums[r * CB + own];
-      for (int c0 = 0; c0 < total; c0 += 64) {
-        const unsigned e = c0 + lane < total ? list[c0 + lane] : ~0u;
-        unsigned long long left = __ballot((int)(e >> 12) == r);
-        // up to U updates in flight, added in ascending order.  (No branches around the loads, or
-        // each would be waited for: past the last entry the one before is read again.)
-        auto take = [&](auto most) {
-          constexpr int U = decltype(most)::value;
-          T x[U];
-          const int n = min(U, (int)__popcll(left));
-          int at = 0;
+    // the entries of row r among list[c0 .. c0 + 64), added to acc in ascending order
+    auto add_entries = [&](int r, int c0, Acc& acc) {
+      const unsigned e = c0 + lane < total ? list[c0 + lane] : ~0u;
+      unsigned long long left = __ballot((int)(e >> 12) == r);
+      const int found = (int)__popcll(left);
+      // up to U updates in flight.  (No branches around the loads, or each would be waited
+      // for: past the last entry the one before is read again.)
+      auto take = [&](auto most) {
+        constexpr int U = decltype(most)::value;
+        T x[U];
+        const int n = min(U, (int)__popcll(left));
+        int at = 0;
 #pragma unroll
-          for (int u = 0; u < U; u++) {
-            at = left ? __builtin_ctzll(left) : at;
-            left &= left - 1;
-            const int entry = __builtin_amdgcn_readlane((int)e, at) & (SCATTER_PASS - 1);
-            x[u] = (pass_updates + entry * step)[at_col];
+        for (int u = 0; u < U; u++) {
+          at = left ? __builtin_ctzll(left) : at;
+          left &= left - 1;
+          const int entry = __builtin_amdgcn_readlane((int)e, at) & (SCATTER_PASS - 1);
+          x[u] = (pass_updates + entry * step)[at_col];
+        }
+#pragma unroll
+        for (int u = 0; u < U; u++)
+          if (u < n) acc = sum_dupes ? (Acc)(acc + x[u]) : (Acc)x[u];
+      };
+      while (left) {
+        const int n = __popcll(left);
+        if (n > 16) take(std::integral_constant<int, 64>());
+        else if (n > 2) take(std::integral_constant<int, 16>());
+        else take(std::integral_constant<int, 2>());
+      }
+      return found;
+    };
+    for (int r0 = 0; r0 < local_rows && total > 0; r0 += 64) {
+      const int n = r0 + lane < local_rows ? counts[r0 + lane] : 0;
+      // (the same masks in every wavefront)
+      unsigned long long hot = CUT && sum_dupes ? __ballot(n > HOT) : 0ull;
+      unsigned long long mine_left = __ballot(n > 0) & ~hot & (~0ull / ((1ull << SETS) - 1)) << set;
+      for (; mine_left; mine_left &= mine_left - 1) {
+        const int at = __builtin_ctzll(mine_left), r = r0 + at;
+        int due = __builtin_amdgcn_readlane(n, at);
+        Acc acc = sums[r * CB + own];
+        for (int c0 = 0; due > 0; c0 += 64) due -= add_entries(r, c0, acc);
+        sums[r * CB + own] = acc;
+      }
+      if constexpr (CUT) {
+        for (; hot; hot &= hot - 1) {
+          const int r = r0 + __builtin_ctzll(hot);
+          Acc acc = (Acc)0;
+          for (int c0 = set * 64; c0 < total; c0 += 64 * SETS) add_entries(r, c0, acc);
+          parts[set * CB + own] = acc;
+          __syncthreads();
+          if (set == 0) {
+            Acc all = sums[r * CB + own];
+            for (int s = 0; s < SETS; s++) all += parts[s * CB + own];
+            sums[r * CB + own] = all;
           }
-#pragma unroll
-          for (int u = 0; u < U; u++)
-            if (u < n) acc = sum_dupes ? (Acc)(acc + x[u]) : (Acc)x[u];
-        };
-        while (left) {
-          const int n = __popcll(left);
-          if (n > 16) take(std::integral_constant<int, 64>());
-          else if (n > 2) take(std::integral_constant<int, 16>());
-          else take(std::integral_constant<int, 2>());
+          __syncthreads();
         }
       }
-      sums[r * CB + own] = acc;
     }
     __syncthreads();
   }
   __syncthreads();
-  for (int r = wave / CW; r < local_rows; r += ROW_WAVES) {
+  for (int r = set; r < local_rows; r += SETS) {
     const int64_t row = mine + (int64_t)r * groups;
     if (row >= rows) break;
     if (stored) out[row * slice + col] = (T)sums[r * CB + own];
   }
 }
 
-// log2 of the groups: enough that a group's sums fit, and four workgroups per CU where there are rows
-// for them.
-static constexpr int scatter_group_shift(int64_t rows, int64_t col_blocks, int most_local, int cus) {
+// log2 of the groups: enough that a group's sums fit, and `per_cu` workgroups per CU where there are
+// rows for them.
+static constexpr int scatter_group_shift(int64_t rows, int64_t col_blocks, int most_local, int cus, int per_cu = 4) {
   int shift = 0;
   while ((rows + ((int64_t)1 << shift) - 1) >> shift > most_local ||
-         (((int64_t)1 << shift) * col_blocks < 4 * cus && ((int64_t)2 << shift) <= rows))
+         (((int64_t)1 << shift) * col_blocks < per_cu * cus && ((int64_t)2 << shift) <= rows))
     shift++;
   return shift;
 }
-// A launch counts its lanes along a dimension in 32 bits: 2^23 groups of 256.  (168 million rows of 129
-// columns in double, 87 GB, are the first that need more.)
-constexpr int SCATTER_MOST_SHIFT = 23;
+// A launch counts its lanes along a dimension in 32 bits: 2^21 groups of 1024 side by side, four
+// times.  (168 million rows of 129 columns in double, 87 GB, are the first that need more.)
+constexpr int SCATTER_MOST_SHIFT = 23, SCATTER_SHIFT_X = 21;
 static_assert(scatter_group_shift(20ll << 23, 1, 20, 256) == SCATTER_MOST_SHIFT &&
               scatter_group_shift((20ll << 23) + 1, 1, 20, 256) > SCATTER_MOST_SHIFT, "");
 static_assert(scatter_group_shift(20000, 1, 80, 256) == 10 && scatter_group_shift(1, 1, 80, 256) == 0, "");
 
 // False: too many rows for this kernel.
-template <typename T, typename Acc, int CW>
-static bool launch_scatter_groups(tfhip_ctx* ctx, const int64_t* flat, const T* updates, T* out, int rows,
+template <typename T, typename Acc, int CW, typename I>
+static bool launch_scatter_groups(tfhip_ctx* ctx, const I* flat, const T* updates, T* out, int rows,
                                   int64_t slice, int64_t n_updates, T start, int sum_dupes, int scalar_update) {
   constexpr int CB = 64 * CW, MOST_LOCAL = (40 << 10) / (CB * (int)sizeof(Acc));  // 40 KB of sums
   const int64_t col_blocks = ceil_div(slice, CB);
-  const int shift = scatter_group_shift(rows, col_blocks, MOST_LOCAL, ctx->num_cus);
+  // 16 wavefronts where all workgroups are in the machine at once (two a CU) or nearly: one pass over the
+  // list takes as long as its longest chain.  With more of them, what counts is how often the list is walked,
+  // and four wavefronts walk it in fewer steps: 100000 rows of 300, 50000 updates 790 us against 1366 (and
+  // 20000 rows of 128, 10240 updates 25.5 with sixteen, 50 with four).  A short list has no long chains.
+  int shift = scatter_group_shift(rows, col_blocks, MOST_LOCAL, ctx->num_cus, 2);
+  const bool wide = ((int64_t)1 << shift) * col_blocks <= 4 * ctx->num_cus && n_updates > 1024;
+  if (!wide) shift = scatter_group_shift(rows, col_blocks, MOST_LOCAL, ctx->num_cus);
   if (shift > SCATTER_MOST_SHIFT) return false;
-  const int local_rows = (int)ceil_div(rows, (int64_t)1 << shift);
-  tfhip::launch(ctx, (scatter_groups_kernel<T, Acc, CW>), dim3(1u << shift, (unsigned)col_blocks), dim3(256),
-                (size_t)local_rows * CB * sizeof(Acc), flat, updates, out, rows, slice, n_updates, start,
+  const int local_rows = (int)ceil_div(rows, (int64_t)1 << shift), across = std::min(shift, SCATTER_SHIFT_X);
+  tfhip::launch(ctx, wide ? scatter_groups_kernel<T, Acc, CW, 1024, I> : scatter_groups_kernel<T, Acc, CW, 256, I>,
+                dim3(1u << across, (unsigned)col_blocks, 1u << (shift - across)), dim3(wide ? 1024 : 256),
+                (size_t)local_rows * (CB * sizeof(Acc) + sizeof(int)), flat, updates, out, rows, slice, n_updates, start,
                 sum_dupes, scalar_update, shift, local_rows);
   return true;
 }
-template <typename T, typename Acc>
-static void launch_scatter(tfhip_ctx* ctx, const int64_t* flat, const T* updates, T* out, int64_t rows,
+template <typename T, typename Acc, typename I>
+static void launch_scatter(tfhip_ctx* ctx, const I* flat, const T* updates, T* out, int64_t rows,
                            int64_t slice, int64_t n_updates, T start, int sum_dupes, int scalar_update) {
   // (half a wavefront of columns, and column blocks that a grid's second dimension holds)
   if (slice >= 32 && n_updates > 0 && slice <= 65535 * 256) {
-    auto launch = slice <= 64    ? launch_scatter_groups<T, Acc, 1>
-                  : slice <= 128 ? launch_scatter_groups<T, Acc, 2>
-                                 : launch_scatter_groups<T, Acc, 4>;
+    auto launch = slice <= 64    ? launch_scatter_groups<T, Acc, 1, I>
+                  : slice <= 128 ? launch_scatter_groups<T, Acc, 2, I>
+                                 : launch_scatter_groups<T, Acc, 4, I>;
     if (launch(ctx, flat, updates, out, (int)rows, slice, n_updates, start, sum_dupes, scalar_update)) return;
   }
-  tfhip::launch(ctx, (scatter_rows_kernel<T, Acc>), dim3(blocks_for(ctx, rows * slice)), dim3(256), 0, flat,
+  tfhip::launch(ctx, (scatter_rows_kernel<T, Acc, I>), dim3(blocks_for(ctx, rows * slice)), dim3(256), 0, flat,
                 updates, out, rows, slice, n_updates, start, sum_dupes, scalar_update);
 }
 
@@ -412,10 +456,11 @@ __global__ void crop_and_resize_kernel(const float* images, const float* boxes,
 
 // Flat slice indices of `indices` [n, slice_rank] into a tensor of `shape` whose first
 // slice_rank dimensions are indexed; fails with the reference's message when one of them is
-// out of range (backend_cpu.ts:3796-3799, 3870-3873).  Waits for the device.
+// out of range (backend_cpu.ts:3796-3799, 3870-3873).  Waits for the device.  as_they_are: the
+// caller reads the indices themselves, only the shapes are looked at.
 static int flatten_checked(tfhip_ctx* ctx, const char* op, const Buf* bi, const int32_t* shape,
                            int rank, int64_t n, int slice_rank, Temp* flat, int64_t* slice_out,
-                           int64_t* rows_out, bool check = true) {
+                           int64_t* rows_out, bool check = true, bool as_they_are = false) {
   if (check && ctx->capturing)
     return ctx->fail(TFHIP_EINVAL, "%s: checks its indices on the host, which a graph capture cannot do", op);
   if (rank < 0 || rank > MAX_SLICE_RANK || slice_rank < 0 || slice_rank > rank || n < 0)
@@ -433,7 +478,7 @@ static int flatten_checked(tfhip_ctx* ctx, const char* op, const Buf* bi, const 
   }
   *slice_out = slice;
   *rows_out = rows;
-  if (n == 0) return TFHIP_OK;
+  if (n == 0 || as_they_are) return TFHIP_OK;
   Temp flag(ctx);
   if (!flat->get((size_t)n * sizeof(int64_t)) || !flag.get(sizeof(int))) return TFHIP_EDEVICE;
   int* bad = static_cast<int*>(flag.ptr);
@@ -518,8 +563,10 @@ extern "C" int tfhip_scatter_nd(tfhip_ctx* ctx, int64_t indices, int64_t updates
   Temp flat(ctx);
   int64_t slice = 0, rows = 0;
   int rc;
+  // (row numbers that need no check are read as they are: a segment sum, two launches fewer)
+  const bool skip = flags & TFHIP_SCATTER_SKIP_INVALID, as_they_are = skip && slice_rank == 1;
   if ((rc = flatten_checked(ctx, "scatterND", bi, out_shape, rank, num_updates, slice_rank, &flat, &slice, &rows,
-                            !(flags & TFHIP_SCATTER_SKIP_INVALID))))
+                            !skip, as_they_are)))
     return rc;
   const bool scalar_update = bu->numel == 1 && num_updates * slice != 1;
   if (bo->numel != rows * slice || (!scalar_update && bu->numel != num_updates * slice))
@@ -529,16 +576,19 @@ extern "C" int tfhip_scatter_nd(tfhip_ctx* ctx, int64_t indices, int64_t updates
   if (bo->numel == 0) return TFHIP_OK;
   if (rows > INT_MAX) return ctx->fail(TFHIP_ENOTSUP, "scatterND: more than 2^31 - 1 result slices");
   const int sum = flags & TFHIP_SCATTER_SUM ? 1 : 0, one = scalar_update ? 1 : 0;
-  const int64_t* fl = (const int64_t*)flat.ptr;
-  if (bo->dtype == TFHIP_INT32)
-    launch_scatter<int32_t, int32_t>(ctx, fl, (const int32_t*)bu->ptr, (int32_t*)bo->ptr, rows, slice, num_updates,
-                                     (int32_t)default_value, sum, one);
-  else if (flags & TFHIP_SCATTER_WIDE_SUM)
-    launch_scatter<float, double>(ctx, fl, (const float*)bu->ptr, (float*)bo->ptr, rows, slice, num_updates,
-                                  (float)default_value, sum, one);
-  else
-    launch_scatter<float, float>(ctx, fl, (const float*)bu->ptr, (float*)bo->ptr, rows, slice, num_updates,
-                                 (float)default_value, sum, one);
+  auto scatter = [&](const auto* fl) {
+    if (bo->dtype == TFHIP_INT32)
+      launch_scatter<int32_t, int32_t>(ctx, fl, (const int32_t*)bu->ptr, (int32_t*)bo->ptr, rows, slice, num_updates,
+                                       (int32_t)default_value, sum, one);
+    else if (flags & TFHIP_SCATTER_WIDE_SUM)
+      launch_scatter<float, double>(ctx, fl, (const float*)bu->ptr, (float*)bo->ptr, rows, slice, num_updates,
+                                    (float)default_value, sum, one);
+    else
+      launch_scatter<float, float>(ctx, fl, (const float*)bu->ptr, (float*)bo->ptr, rows, slice, num_updates,
+                                   (float)default_value, sum, one);
+  };
+  if (as_they_are) scatter((const int32_t*)bi->ptr);
+  else scatter((const int64_t*)flat.ptr);
   TFHIP_LAUNCH_CHECK(ctx);
   return TFHIP_OK;
 }
