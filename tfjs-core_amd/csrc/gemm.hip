@@ -198,6 +198,7 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N * 64) void gemm_kernel(const GemmA
     long long a_base[A_PER];  // row-major: row*lda ; im2col: n*H*W*Cin
     int a_ih0[A_PER], a_iw0[A_PER];
     bool a_ok[A_PER];
+    unsigned a_taps[A_PER];   // A_IM2COL_TAPS: the filter taps whose pixel lies inside the image, a bit each
     // FAST loaders whose k offset is the same for every lane (row-major A, every B): the byte
     // offset of the item inside a tile that lies wholly below K, and inside the one tile that K
     // cuts (items at or beyond K out of range).  The tile's own offset rides in the scalar
@@ -253,6 +254,16 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N * 64) void gemm_kernel(const GemmA
           L.a_base[i] = (long long)n * p.H * p.W * p.Cin;
           L.a_ih0[i] = oh * p.sh - p.pt;
           L.a_iw0[i] = ow * p.sw - p.pl;
+          if (AMODE == A_IM2COL_TAPS) {
+            unsigned columns = 0, taps = 0;
+            for (int kw = 0; kw < p.KW; kw++)
+              columns |= ((unsigned)(L.a_iw0[i] + kw * p.dw) < (unsigned)p.W ? 1u : 0u) << kw;
+            for (int kh = 0; kh < p.KH; kh++)
+              taps |= ((unsigned)(L.a_ih0[i] + kh * p.dh) < (unsigned)p.H ? columns : 0u) << (kh * p.KW);
+            L.a_taps[i] = L.a_ok[i] ? taps : 0u;
+            // (of the first tap; before the image's first byte where that lies outside)
+            L.a_voff[i] = ((unsigned)((n * p.H + L.a_ih0[i]) * p.W + L.a_iw0[i]) * p.Cin + L.a_kq[i]) * 4u;
+          }
         }
       }
     }
@@ -320,6 +331,19 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N * 64) void gemm_kernel(const GemmA
       for (int i = 0; i < A_PER; i++)
         reg[i] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(
                      r, (int)L.a_voff[i], k0 * 4, 0));
+      return;
+    }
+    if (AMODE == A_IM2COL_TAPS) {
+      // A step lies in one tap, which is the same for all lanes: its place is found with scalar
+      // instructions, and an item costs an addition and a look at its bit.  (With k per lane a step cost
+      // two divisions, some 45 vector instructions, on the pipe of the matrix instructions: 3 x 3 of
+      // [32, 112, 112, 64] -> 128 505 -> 453 us, 131 TFLOP/s; [32, 28, 28, 256] -> 256 262 -> 233.)
+      const unsigned tap = p.by_cin.quotient((unsigned)k0), kh = p.by_kw.quotient(tap);
+      const unsigned at = (((kh * p.dh) * p.W + (tap - kh * p.KW) * p.dw) * p.Cin + (k0 - tap * p.Cin)) * 4u;
+      const unsigned bit = k0 < p.K ? 1u << tap : 0u;
+#pragma unroll
+      for (int i = 0; i < A_PER; i++)
+        reg[i] = buffer_load_f32x4(rsrc_a, L.a_taps[i] & bit ? L.a_voff[i] + at : OOB_OFFSET);
       return;
     }
     if (FAST) {
@@ -1588,7 +1612,7 @@ int launch_splitk_finish(tfhip_ctx* ctx, const GemmArgs& p, int bm, int bn) {
 
 template <class T, int AMODE, int BMODE, bool KBLOCKED, bool FAST>
 static int launch_cfg(tfhip_ctx* ctx, GemmArgs& p, const Plan& pl) {
-  static const char* const a_names[] = {"rowmajor", "transposed", "im2col", "im2col_up", "im2col_t"};
+  static const char* const a_names[] = {"rowmajor", "transposed", "im2col", "im2col_up", "im2col_t", "im2col"};
   static const char* const b_names[] = {"f32", "f32t", "u8"};
   ctx->name_kernel("gemm_%dx%d_%s_%s%s%s", T::BM, T::BN,
            a_names[AMODE], b_names[BMODE], KBLOCKED ? "_kb48" : "",
@@ -1649,17 +1673,19 @@ static int launch_mode(tfhip_ctx* ctx, GemmArgs& p, int batch) {
                   p.ldb == p.N && (p.K & 3) == 0 && (p.lda & 3) == 0 &&
                   (long long)p.M * p.N <= 0x7fffffffLL;
   Plan plans[NCFG];
-  const bool gathered = AMODE == A_IM2COL || AMODE == A_IM2COL_UP || AMODE == A_IM2COL_T;
+  // (planned as the general gather is: the same tiles, cut in the same places, the same sums)
+  constexpr int PLAN_MODE = AMODE == A_IM2COL_TAPS ? A_IM2COL : AMODE;
+  const bool gathered = AMODE == A_IM2COL || AMODE == A_IM2COL_UP || AMODE == A_IM2COL_T || AMODE == A_IM2COL_TAPS;
   const bool huge = (double)p.M * p.N * p.K * batch >= 5e10;
   const double eff_big = gathered ? 0.98 : huge ? 1.00 : 0.95;
   const double eff_mid = gathered ? 0.95 : huge ? 0.93 : 0.91;
   const double eff_wide = gathered ? 1.00 : huge ? 0.94 : 0.99;
   const double eff_small = gathered ? 0.92 : huge ? 0.92 : 1.00;
-  plans[0] = make_plan(p, batch, Big::BM, Big::BN, resident_blocks<Big, AMODE, BMODE, KBLOCKED, FAST>(ctx), cus, eff_big, KBLOCKED, mk);
-  plans[1] = make_plan(p, batch, Mid::BM, Mid::BN, resident_blocks<Mid, AMODE, BMODE, KBLOCKED, FAST>(ctx), cus, eff_mid, KBLOCKED, mk);
-  plans[2] = make_plan(p, batch, Wide::BM, Wide::BN, resident_blocks<Wide, AMODE, BMODE, KBLOCKED, FAST>(ctx), cus, eff_wide, KBLOCKED, mk);
-  plans[3] = make_plan(p, batch, Thin::BM, Thin::BN, resident_blocks<Thin, AMODE, BMODE, KBLOCKED, FAST>(ctx), cus, 0.80, KBLOCKED, mk);
-  plans[4] = make_plan(p, batch, Small::BM, Small::BN, resident_blocks<Small, AMODE, BMODE, KBLOCKED, FAST>(ctx), cus, eff_small, KBLOCKED, mk);
+  plans[0] = make_plan(p, batch, Big::BM, Big::BN, resident_blocks<Big, PLAN_MODE, BMODE, KBLOCKED, FAST>(ctx), cus, eff_big, KBLOCKED, mk);
+  plans[1] = make_plan(p, batch, Mid::BM, Mid::BN, resident_blocks<Mid, PLAN_MODE, BMODE, KBLOCKED, FAST>(ctx), cus, eff_mid, KBLOCKED, mk);
+  plans[2] = make_plan(p, batch, Wide::BM, Wide::BN, resident_blocks<Wide, PLAN_MODE, BMODE, KBLOCKED, FAST>(ctx), cus, eff_wide, KBLOCKED, mk);
+  plans[3] = make_plan(p, batch, Thin::BM, Thin::BN, resident_blocks<Thin, PLAN_MODE, BMODE, KBLOCKED, FAST>(ctx), cus, 0.80, KBLOCKED, mk);
+  plans[4] = make_plan(p, batch, Small::BM, Small::BN, resident_blocks<Small, PLAN_MODE, BMODE, KBLOCKED, FAST>(ctx), cus, eff_small, KBLOCKED, mk);
   // rows and columns beyond M and N are wasted matrix-core work: charge it
   const int bns[NCFG] = {Big::BN, Mid::BN, Wide::BN, Thin::BN, Small::BN};
   const int bms[NCFG] = {Big::BM, Mid::BM, Wide::BM, Thin::BM, Small::BM};
@@ -1792,6 +1818,12 @@ static int launch_gemm(tfhip_ctx* ctx, GemmArgs& p, int batch, int amode, int bm
   }
   p.a_bytes = fast ? (unsigned)a_bytes : 0;
   p.b_bytes = fast ? (unsigned)b_bytes : 0;
+  if (amode == A_IM2COL && fast && p.Cin % BK == 0 && p.KH * p.KW < 32) {
+    p.by_cin = Divisor(p.Cin);
+    p.by_kw = Divisor(p.KW);
+    return bmode == B_UINT8 ? launch_mode<A_IM2COL_TAPS, B_UINT8, false, true>(ctx, p, batch)
+                            : launch_mode<A_IM2COL_TAPS, B_ROWMAJOR, false, true>(ctx, p, batch);
+  }
 #define TFHIP_CASE(AM, BM_, KB)                                \
   if (amode == AM && bmode == BM_ && kblocked == KB)           \
     return fast ? launch_mode<AM, BM_, KB, true>(ctx, p, batch) \

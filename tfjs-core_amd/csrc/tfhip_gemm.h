@@ -9,8 +9,9 @@ namespace tfhip {
 // A_IM2COL_UP: the gather of conv2dDerInput (rows are input pixels, k is (filter row, filter
 // column, output channel) of the flipped filter; the image gathered from is dy, stretched by
 // the forward stride).  A_IM2COL_T: the gather of conv2dDerFilter (rows are (filter row,
-// filter column, input channel), k runs over the output pixels (n, oh, ow)).
-enum { A_ROWMAJOR = 0, A_TRANSPOSED = 1, A_IM2COL = 2, A_IM2COL_UP = 3, A_IM2COL_T = 4 };
+// filter column, input channel), k runs over the output pixels (n, oh, ow)).  A_IM2COL_TAPS: A_IM2COL
+// where the channels of a filter tap are whole k steps, and the taps are fewer than 32.
+enum { A_ROWMAJOR = 0, A_TRANSPOSED = 1, A_IM2COL = 2, A_IM2COL_UP = 3, A_IM2COL_T = 4, A_IM2COL_TAPS = 5 };
 enum { B_ROWMAJOR = 0, B_TRANSPOSED = 1, B_UINT8 = 2 };
 
 struct GemmArgs {
@@ -26,6 +27,7 @@ struct GemmArgs {
   int a_vec, b_vec;  // operands allow aligned 4-element accesses
   // implicit-GEMM geometry (A_IM2COL): rows are (n, oh, ow), k is (kh, kw, c)
   int H, W, Cin, OH, OW, KH, KW, sh, sw, dh, dw, pt, pl;
+  Divisor by_cin, by_kw;  // A_IM2COL_TAPS
   int up_h, up_w;  // A_IM2COL_UP: forward strides (dy is read at row / up_h when divisible)
   double qscale, qmin;
   // schedule (see work_item)
