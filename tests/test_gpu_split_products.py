@@ -310,3 +310,45 @@ def test_special_values_in_gathers(tf, n, h, w, cin, cout):
     fin = np.isfinite(want)
     bound = _float32_bound(9 * cout, _conv64(clean(dy), clean(back), 1, 1, (1, 1), h, w))
     assert np.all(np.abs(np.where(fin, dx, 0) - np.where(fin, want, 0)) <= bound)
+
+
+@pytest.mark.parametrize("n,h,w,cin,cout,f,pad", [
+    (32, 56, 57, 48, 128, 3, "same"),     # taps of whole steps; ragged columns; leftover tiles cut along K
+    (64, 57, 55, 30 * 2, 64, 3, "valid"), # every column count up to the tile's, padding of the gradient
+    (8, 28, 28, 64, 256, 5, "same"),      # every tile cut
+])
+def test_input_gradient_in_tall_tiles(tf, n, h, w, cin, cout, f, pad):
+    print("tall tiles", n, h, w, cin, cout, f, pad, flush=True)
+    rng = np.random.default_rng(cin + cout)
+    oh, ow = (h, w) if pad == "same" else (h - f + 1, w - f + 1)
+    dy = rng.standard_normal((n, oh, ow, cout)).astype(np.float32)
+    k = rng.standard_normal((f, f, cin, cout)).astype(np.float32)
+    with tf.tidy():
+        got = tf.conv2d_der_input((n, h, w, cin), tf.tensor(dy), tf.tensor(k), 1, pad).data_sync().astype(np.float64)
+        assert _kernel(tf).startswith("gemm_split_256x64_im2col"), _kernel(tf)
+    edge = f - 1 - ((f - 1) // 2 if pad == "same" else 0)
+    wide = np.zeros((n, h + f - 1, w + f - 1, cout))
+    wide[:, edge:edge + oh, edge:edge + ow] = dy
+    for img in (0, n // 2, n - 1):
+        want, magnitude = np.zeros((h, w, cin)), np.zeros((h, w, cin))
+        for i in range(f):
+            for j in range(f):
+                part, tap = wide[img, i:i + h, j:j + w], k[f - 1 - i, f - 1 - j].astype(np.float64).T
+                want += part @ tap
+                magnitude += np.abs(part) @ np.abs(tap)
+        _check(got[img], want, magnitude, f * f * cout)
+
+
+@pytest.mark.parametrize("m,k,n", [(100000, 64, 64), (70001, 128, 60)])
+def test_tall_tiles_of_products(tf, m, k, n):
+    print("tall products", m, k, n, flush=True)
+    rng = np.random.default_rng(m)
+    a, b = rng.standard_normal((m, k)).astype(np.float32), rng.standard_normal((n, k)).astype(np.float32)
+    a[7, 3], a[m - 1, k - 1] = np.inf, 2.0 ** -130            # a tile of each kind is summed again
+    with tf.tidy():
+        got = tf.matmul(tf.tensor(a), tf.tensor(b), False, True).data_sync().astype(np.float64)
+        assert _kernel(tf).startswith("gemm_split_256x64"), _kernel(tf)
+    want, magnitude = a.astype(np.float64) @ b.T.astype(np.float64), np.abs(a).astype(np.float64) @ np.abs(b).T
+    fine = np.isfinite(want)
+    assert np.array_equal(np.isfinite(got), fine)
+    _check(got[fine], want[fine], magnitude[fine], k)

@@ -126,7 +126,7 @@ struct Staging {
 template <class T, int AMODE, int BMODE, int BLOCKED, bool VEC>
 __global__ __launch_bounds__(T::THREADS, 2) void gemm_split_kernel(const GemmArgs p) {
   constexpr int BM = T::BM, BN = T::BN, TM = T::TM, TN = T::TN, THREADS = T::THREADS;
-  constexpr bool A_KC = AMODE == A_ROWMAJOR || AMODE == A_IM2COL;
+  constexpr bool A_KC = AMODE == A_ROWMAJOR || AMODE == A_IM2COL || AMODE == A_IM2COL_TAPS;
   constexpr bool B_KC = BMODE == B_TRANSPOSED;
   static_assert(BM % 64 == 0 && BN % 64 == 0, "slots are dealt within 64 rows");
   using SA = Staging<BM, THREADS, A_KC>;
@@ -155,6 +155,7 @@ __global__ __launch_bounds__(T::THREADS, 2) void gemm_split_kernel(const GemmArg
   // ---- what this thread stages ----
   unsigned a_at[SA::PER], b_at[SB::PER];  // byte offset of the item at k = 0; OOB_OFFSET: no such row
   int a_ih[SA::PER], a_iw[SA::PER];       // gathers: image row and column at the first tap (pixel)
+  unsigned a_taps[SA::PER];               // A_IM2COL_TAPS: the taps inside the image, a bit each
   // Position of the thread's next k in a gather: channel and filter column (A_IM2COL), or output
   // column and output row (A_IM2COL_T); the image rows, columns and bytes it lies from where the
   // item starts, kept up by additions (a 32-bit multiply takes four times an addition's time).
@@ -178,6 +179,16 @@ __global__ __launch_bounds__(T::THREADS, 2) void gemm_split_kernel(const GemmArg
         a_ih[i] = ok ? oh * p.sh - p.pt : -0x40000000;  // (a row past the last: no image row)
         a_iw[i] = ow * p.sw - p.pl;
         a_at[i] = (unsigned)((n * p.H + a_ih[i]) * p.W + a_iw[i]) * p.Cin * 4u;
+      } else if (AMODE == A_IM2COL_TAPS) {
+        const int ow = row % p.OW, r = row / p.OW;
+        const int oh = r % p.OH, n = r / p.OH;
+        const int ih = oh * p.sh - p.pt, iw = ow * p.sw - p.pl;
+        unsigned columns = 0, taps = 0;
+        for (int kw = 0; kw < p.KW; kw++) columns |= ((unsigned)(iw + kw * p.dw) < (unsigned)p.W ? 1u : 0u) << kw;
+        for (int kh = 0; kh < p.KH; kh++)
+          taps |= ((unsigned)(ih + kh * p.dh) < (unsigned)p.H ? columns : 0u) << (kh * p.KW);
+        a_taps[i] = ok ? taps : 0u;
+        a_at[i] = ((unsigned)((n * p.H + ih) * p.W + iw) * p.Cin + SA::k(tid, 0)) * 4u;
       } else {
         const int tap = row / p.Cin, c = row - tap * p.Cin;
         const int kh = tap / p.KW, kw = tap - kh * p.KW;
@@ -253,6 +264,13 @@ __global__ __launch_bounds__(T::THREADS, 2) void gemm_split_kernel(const GemmArg
                         ((unsigned)(a_iw[i] + g_col) < (unsigned)p.W);
         o.a[i] = buffer_load_f32x4(ra, ok ? a_at[i] + g_at : OOB_OFFSET);
       }
+    } else if (AMODE == A_IM2COL_TAPS) {
+      // (a step lies in one tap: its place is scalar arithmetic, a look at a bit says whether it is there)
+      const unsigned tap = p.by_cin.quotient((unsigned)k0), kh = p.by_kw.quotient(tap);
+      const unsigned at = (((kh * p.dh) * p.W + (tap - kh * p.KW) * p.dw) * p.Cin + (k0 - tap * p.Cin)) * 4u;
+      const unsigned bit = k0 < p.K ? 1u << tap : 0u;
+#pragma unroll
+      for (int i = 0; i < SA::PER; i++) o.a[i] = buffer_load_f32x4(ra, a_taps[i] & bit ? a_at[i] + at : OOB_OFFSET);
     } else if (AMODE == A_TRANSPOSED) {
 #pragma unroll
       for (int i = 0; i < SA::PER; i++)
@@ -597,7 +615,9 @@ struct SplitPlan {
 // The best plan of one tile shape, against `best`, by an estimate in microseconds: a launch, and
 // the steps of the busiest CU.  A step of a workgroup alone on its CU takes `alone` us and one of
 // several `shared` (measured: [128, 128] tiles 0.80 and 0.80, their wavefronts fill a CU; [64, 128]
-// 0.56 and 0.48; [128, 64] 0.60 and 0.58).  A cut along K costs a second launch and the partial
+// 0.56 and 0.48; [128, 64] 0.60 and 0.58; [256, 64] 1.20 and 0.88, which is a quarter less than two of the
+// former: where there are at most 64 columns a wavefront of 64 x 64 splits and reads from LDS
+// two thirds of what two of 32 x 64 do).  A cut along K costs a second launch and the partial
 // tiles' way through memory.  `most_steps`: longest range of K the shape may be given.
 static void plan_cfg(SplitPlan& best, int cfg, int bm, int bn, double alone, double shared, int most_steps,
                      const GemmArgs& p, int batch, int cus) {
@@ -662,7 +682,7 @@ static double float32_cost(const GemmArgs& p, int batch, int cus, int amode, int
 
 template <class T, int AMODE, int BMODE, int BLOCKED, bool VEC>
 static int launch_cfg(tfhip_ctx* ctx, GemmArgs p, const SplitPlan& pl) {
-  static const char* const a_names[] = {"rowmajor", "transposed", "im2col", "im2col_up", "im2col_t"};
+  static const char* const a_names[] = {"rowmajor", "transposed", "im2col", "im2col_up", "im2col_t", "im2col"};
   static const char* const b_names[] = {"f32", "f32t"};
   ctx->name_kernel("gemm_split_%dx%d_%s_%s%s%s", T::BM, T::BN, a_names[AMODE], b_names[BMODE],
                    VEC ? "" : "_unaligned", pl.splits > 1 ? pl.full ? "_tailk" : "_splitk" : "");
@@ -695,6 +715,7 @@ static int launch_mode(tfhip_ctx* ctx, const GemmArgs& p, int batch, int amode32
   using Big = SplitCfg<2, 2, 2>;   // 128 x 128
   using Wide = SplitCfg<2, 2, 1>;  // 64 x 128
   using Tall = SplitCfg<4, 1, 1>;  // 128 x 64
+  using High = SplitCfg<4, 1, 2>;  // 256 x 64
   const int cus = ctx->num_cus, any = 0x7fffffff;
   SplitPlan pl;
   // (the registers of a 128 x 128 tile hold no third set of sums)
@@ -703,10 +724,16 @@ static int launch_mode(tfhip_ctx* ctx, const GemmArgs& p, int batch, int amode32
   plan_cfg(pl, 0, Big::BM, Big::BN, 0.80 * wait, 0.80, KBLOCKED ? SPLIT_PLAIN_K / SK : any, p, batch, cus);
   plan_cfg(pl, 1, Wide::BM, Wide::BN, 0.56 * wait, 0.48, any, p, batch, cus);
   plan_cfg(pl, 2, Tall::BM, Tall::BN, 0.60 * wait, 0.58, any, p, batch, cus);
+  constexpr bool HIGH = AMODE != A_IM2COL_T && AMODE != A_IM2COL;  // (one pixel position per thread; registers)
+  if constexpr (HIGH)
+    plan_cfg(pl, 3, High::BM, High::BN, 1.20, 0.88, KBLOCKED ? SPLIT_PLAIN_K / SK : any, p, batch, cus);
   if (pl.cfg < 0 || pl.cost > float32_cost(p, batch, cus, amode32, BMODE)) return -1;
   // tfhip_matmul_noalloc takes the same plan where its array holds the partial tiles, and float32
   // where not: the split kernels' cuts are larger than those it has always taken.
-  const size_t tile = pl.cfg == 0 ? Big::BM * Big::BN : pl.cfg == 1 ? Wide::BM * Wide::BN : Tall::BM * Tall::BN;
+  const size_t tile = pl.cfg == 0   ? Big::BM * Big::BN
+                      : pl.cfg == 1 ? Wide::BM * Wide::BN
+                      : pl.cfg == 2 ? Tall::BM * Tall::BN
+                                    : High::BM * High::BN;
   if (ctx->no_alloc && pl.splits > 1 && (size_t)pl.tail * pl.splits * tile * sizeof(float) > kScratchBytes) return -1;
   const int longest = pl.full ? (int)ceil_div(p.K, SK) : pl.kt_per;
   const bool blocked = KBLOCKED && longest * SK > SPLIT_PLAIN_K;
@@ -716,7 +743,10 @@ static int launch_mode(tfhip_ctx* ctx, const GemmArgs& p, int batch, int amode32
   switch (pl.cfg) {
     case 0: return launch_cfg<Big, AMODE, BMODE, 0, VEC>(ctx, p, pl);
     case 1: TFHIP_LAUNCH(Wide);
-    default: TFHIP_LAUNCH(Tall);
+    case 2: TFHIP_LAUNCH(Tall);
+    default:
+      if constexpr (HIGH) return launch_cfg<High, AMODE, BMODE, 0, VEC>(ctx, p, pl);
+      else return -1;
   }
 #undef TFHIP_LAUNCH
 }
@@ -746,10 +776,15 @@ int launch_split(tfhip_ctx* ctx, const GemmArgs& q, int batch, int amode, int bm
     amode = A_IM2COL;
   }
   const bool vec = q.a_vec && q.b_vec;
+  if (amode == A_IM2COL && vec && q.Cin % SK == 0 && q.KH * q.KW < 32) amode = A_IM2COL_TAPS;
   if (bmode == B_UINT8 || (!vec && (amode == A_IM2COL || amode == A_IM2COL_T))) return -1;
   GemmArgs p = q;
   p.a_bytes = (unsigned)a_bytes;
   p.b_bytes = (unsigned)b_bytes;
+  if (amode == A_IM2COL_TAPS) {
+    p.by_cin = Divisor(p.Cin);
+    p.by_kw = Divisor(p.KW);
+  }
 #define TFHIP_CASE(AM, BM_, KB, V)                               \
   if (amode == AM && bmode == BM_ && kblocked == KB && vec == V) \
     return launch_mode<AM, BM_, KB, V>(ctx, p, batch, amode32);
@@ -762,6 +797,7 @@ int launch_split(tfhip_ctx* ctx, const GemmArgs& q, int batch, int amode, int bm
   TFHIP_CASE(A_TRANSPOSED, B_ROWMAJOR, true, false)
   TFHIP_CASE(A_TRANSPOSED, B_TRANSPOSED, true, false)
   TFHIP_CASE(A_IM2COL, B_ROWMAJOR, false, true)
+  TFHIP_CASE(A_IM2COL_TAPS, B_ROWMAJOR, false, true)
   TFHIP_CASE(A_IM2COL_T, B_ROWMAJOR, false, true)
 #undef TFHIP_CASE
   return -1;
