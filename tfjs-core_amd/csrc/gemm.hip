@@ -919,16 +919,22 @@ __global__ void splitk_finish_kernel(const GemmArgs p, int BM, int BN, int first
     if (row >= p.M || col >= p.N) continue;
     f32x4 v = {0.f, 0.f, 0.f, 0.f};
     const float* src = p.partials + ((long long)tt * p.splits) * (BM * BN) + e;
-    // four partial tiles in flight at a time; added in ascending k order
+    // sixteen partial tiles in flight at a time, then four; added in ascending k order.  (A filter gradient
+    // has 100 of them and few elements: its sum is a chain of trips to memory, 11.0 us with four, 8.0.)
     int s = 0;
-    for (; s + 4 <= p.splits; s += 4) {
-      f32x4 t[4];
+    auto add = [&](auto most) {
+      constexpr int U = decltype(most)::value;
+      for (; s + U <= p.splits; s += U) {
+        f32x4 t[U];
 #pragma unroll
-      for (int u = 0; u < 4; u++)
-        t[u] = *reinterpret_cast<const f32x4*>(src + (long long)(s + u) * (BM * BN));
+        for (int u = 0; u < U; u++)
+          t[u] = *reinterpret_cast<const f32x4*>(src + (long long)(s + u) * (BM * BN));
 #pragma unroll
-      for (int u = 0; u < 4; u++) v += t[u];
-    }
+        for (int u = 0; u < U; u++) v += t[u];
+      }
+    };
+    add(std::integral_constant<int, 16>());
+    add(std::integral_constant<int, 4>());
     for (; s < p.splits; s++) v += *reinterpret_cast<const f32x4*>(src + (long long)s * (BM * BN));
     const long long base = (long long)batch * p.strideC + (long long)row * p.N + col;
 #pragma unroll
