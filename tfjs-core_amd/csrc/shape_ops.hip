@@ -43,6 +43,46 @@ struct Box32 {
   Divisor region[MAXBOX];
   int32_t x_stride[MAXBOX], out_stride[MAXBOX];
 };
+// The same for boxes of runs: 4-byte elements that lie side by side on both sides (the innermost
+// dimension, which `outer` does not hold), copied in vectors of 4 at 4-byte alignment, which the
+// hardware takes.  MIRROR = 0: runs of `len` elements.  MIRROR = 1 .. 3: rows of `len` elements in pixels
+// of so many, read backwards pixel by pixel; the four elements of a vector come from one line or two.
+// What the end of a row cuts is copied as a whole vector too, from before the end, the same values
+// twice.  Mirroring [16, 480, 640, 3] left to right 22.2 -> 18.5 us (6.4 TB/s), top to bottom 20.0 -> 18.0;
+// placing [32, 56, 56, 64] in the channels of a larger tensor 10.6 -> 8.8.
+typedef int32_t i32x4 __attribute__((ext_vector_type(4)));
+struct __attribute__((packed, aligned(4))) Loose4 {
+  i32x4 v;
+};
+template <int MIRROR>
+__global__ __launch_bounds__(256) void copy_runs_kernel(const int32_t* __restrict__ x, int32_t* __restrict__ out,
+                                                        uint32_t n, Box32 outer, Divisor groups, int len) {
+  constexpr int W = MIRROR ? MIRROR : 1;  // elements of a pixel
+  uint32_t rem = blockIdx.x * blockDim.x + threadIdx.x;
+  if (rem >= n) return;
+  const int e0 = min((int)groups.divmod(rem) * 4, len - 4);
+  int32_t src = outer.x_offset, dst = outer.out_offset + e0;
+#pragma unroll
+  for (int d = MAXBOX - 1; d >= 0; d--) {
+    if (d < outer.rank) {
+      const int32_t c = (int32_t)outer.region[d].divmod(rem);
+      src += c * outer.x_stride[d];
+      dst += c * outer.out_stride[d];
+    }
+  }
+  i32x4 v;
+  if (MIRROR == 0) {
+    v = reinterpret_cast<const Loose4*>(x + src + e0)->v;
+  } else if (MIRROR == 1) {  // (x_offset is the row's last element)
+    const i32x4 t = reinterpret_cast<const Loose4*>(x + src - e0 - 3)->v;
+    v = i32x4{t[3], t[2], t[1], t[0]};
+  } else {                   // (x_offset is the row's last pixel)
+#pragma unroll
+    for (int e = 0; e < 4; e++) v[e] = x[src - (e0 + e) / W * W + (e0 + e) % W];
+  }
+  reinterpret_cast<Loose4*>(out + dst)->v = v;
+}
+
 template <typename T>
 __global__ void strided_copy32_kernel(const T* __restrict__ x, T* __restrict__ out, uint32_t n, Box32 b) {
   constexpr int U = 4;
@@ -260,9 +300,35 @@ extern "C" int tfhip_strided_copy(tfhip_ctx* ctx, int64_t x, int64_t out, int ra
       c.x_stride[c.rank] = (int32_t)x_strides[d];
       c.out_stride[c.rank++] = (int32_t)out_strides[d];
     }
+    // Runs: the innermost dimension side by side on both sides, or a mirrored row of small pixels.  (Below 8
+    // elements, or 8 pixels, a row's last vector repeats too much of the one before.)
+    const bool words = dtype_size(bx->dtype) == 4;
+    auto inner = [&](int from_end, int64_t xs) {
+      const int d = c.rank - from_end;
+      return d >= 0 && c.x_stride[d] == xs && c.out_stride[d] == (xs < 0 ? -xs : xs) && extent[d] >= 8;
+    };
+    const int64_t pixel = c.rank > 0 && c.x_stride[c.rank - 1] == 1 && c.out_stride[c.rank - 1] == 1 ? extent[c.rank - 1] : 0;
+    int mirror = -1, drop = 1;
+    if (words && inner(1, 1)) mirror = 0;
+    else if (words && inner(1, -1)) mirror = 1;
+    else if (words && (pixel == 2 || pixel == 3) && inner(2, -pixel)) mirror = (int)pixel, drop = 2;
     for (int d = 0; d < c.rank; d++) c.region[d] = Divisor(extent[d]);
+    if (mirror >= 0) {
+      const int64_t len = extent[c.rank - drop] * (mirror > 1 ? mirror : 1), groups = ceil_div(len, 4);
+      c.rank -= drop;
+      int64_t lanes = groups;
+      for (int d = 0; d < c.rank; d++) lanes *= extent[d];
+      auto kernel = mirror == 0   ? copy_runs_kernel<0>
+                    : mirror == 1 ? copy_runs_kernel<1>
+                    : mirror == 2 ? copy_runs_kernel<2>
+                                  : copy_runs_kernel<3>;
+      tfhip::launch(ctx, kernel, dim3((unsigned)ceil_div(lanes, 256)), block, 0, (const int32_t*)bx->ptr,
+                    (int32_t*)bo->ptr, (uint32_t)lanes, c, Divisor(groups), (int)len);
+      TFHIP_LAUNCH_CHECK(ctx);
+      return TFHIP_OK;
+    }
     const dim3 grid4(grid_for(ctx, ceil_div(n, 4), 256));
-    if (dtype_size(bx->dtype) == 4)
+    if (words)
       tfhip::launch(ctx, strided_copy32_kernel<int32_t>, grid4, block, 0, (const int32_t*)bx->ptr,
                     (int32_t*)bo->ptr, (uint32_t)n, c);
     else
