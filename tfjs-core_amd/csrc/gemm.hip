@@ -697,10 +697,14 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N * 64) void gemm_kernel(const GemmA
   // to their LDS stores and every step pays their latency in full.  With FAST loaders the
   // loads past the last tile are range-checked to zero and parked in an unused buffer, so
   // the loop body has no branches.
-  // Staging registers.  Convolutions (not KBLOCKED) keep two sets and run the global loads
-  // three tiles ahead of the matrix cores instead of two: a step of a lone wavefront is
-  // shorter than a trip to HBM.
-  constexpr int AHEAD = KBLOCKED ? 2 : 3;
+  // Staging registers: two sets, and the global loads run three tiles ahead of the matrix cores instead
+  // of two: a step of a lone wavefront is shorter than a trip to HBM.  With matMul's second accumulator
+  // this leaves four 64 x 64 workgroups on a CU instead of six, and is the better trade all the same:
+  // [4096, 784] x [784, 1024] 66.6 -> 62.3 us, [4096, 1024] x [1024, 1024] 83.5 -> 78.2, [2688, 1792] x
+  // [1792, 512] 66.6 -> 58.2, [1000, 784]^T x [1000, 512] 21.3 -> 19.8 (five workgroups, held to 96
+  // registers, give the same).  Only matMul's 256 x 32 tile, which would keep two of three, stays at two
+  // tiles and one set ([2304, 2336] x [2336, 32] 15.2 us, 15.6 with three).
+  constexpr int AHEAD = KBLOCKED && BN == 32 ? 2 : 3;
   f32x4 a_reg[2][A_PER], b_reg[2][B_PER];
   Frag f0, f1;
   load_a(L, cur.kt0 * BK, a_reg[0]);
@@ -753,16 +757,16 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N * 64) void gemm_kernel(const GemmA
   };
 
   if (KBLOCKED) {
-    int buf = 0;
-    for (int i = 0; i < n_steps; i += TILES_PER_KBLOCK) {
-      step(i, buf, a_reg[0], b_reg[0], std::true_type{});
-      buf ^= 1;
-#pragma unroll
-      for (int t = 1; t < TILES_PER_KBLOCK; t++)
-        if (i + t < n_steps) {
-          step(i + t, buf, a_reg[0], b_reg[0], std::false_type{});
-          buf ^= 1;
-        }
+    static_assert(TILES_PER_KBLOCK == 3, "two blocks of k take six steps");
+    for (int i = 0; i < n_steps; i += 6) {
+      step(i, 0, a_reg[SET1], b_reg[SET1], std::true_type{});
+      if (i + 1 < n_steps) step(i + 1, 1, a_reg[0], b_reg[0], std::false_type{});
+      if (i + 2 < n_steps) step(i + 2, 0, a_reg[SET1], b_reg[SET1], std::false_type{});
+      flush();
+      if (i + 3 >= n_steps) break;
+      step(i + 3, 1, a_reg[0], b_reg[0], std::true_type{});
+      if (i + 4 < n_steps) step(i + 4, 0, a_reg[SET1], b_reg[SET1], std::false_type{});
+      if (i + 5 < n_steps) step(i + 5, 1, a_reg[0], b_reg[0], std::false_type{});
       flush();
     }
   } else {
