@@ -116,15 +116,6 @@ __global__ __launch_bounds__(1024) void depthwise_der_filter_finish_kernel(const
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
-// out[kh][kw][c] = w[KH - 1 - kh][KW - 1 - kw][c] (channel multiplier 1).
-__global__ void flip_depthwise_filter_kernel(const float* w, float* out, int KH, int KW, int C) {
-  const int g = blockIdx.x * blockDim.x + threadIdx.x;
-  if (g >= KH * KW * C) return;
-  const int c = g % C, t = g / C;
-  const int kw = t % KW, kh = t / KW;
-  out[g] = w[((KH - 1 - kh) * KW + (KW - 1 - kw)) * C + c];
-}
-
 // Fast variants for channel multiplier 1, C % 4 == 0 and 16-byte aligned buffers: a lane owns
 // 4 consecutive channels (16-byte accesses) and sums in float in the same tap order.
 // S = 1, 2: the forward stride, known at compile time (no integer division); S = 0: any.
@@ -587,11 +578,6 @@ extern "C" int tfhip_depthwise_conv2d_der_input(tfhip_ctx* ctx, int64_t dy, int6
   if (ch_mul == 1 && ci->stride_h == 1 && ci->stride_w == 1 && y_n > 0) {
     // stride 1: dx is the depthwise convolution of dy with the filter flipped in both spatial
     // directions and the padding filter - 1 - pad: the forward kernels do it at their speed
-    Temp tflip(ctx);
-    if (!tflip.get((size_t)w_n * sizeof(float))) return TFHIP_EDEVICE;
-    tfhip::launch(ctx, flip_depthwise_filter_kernel, dim3((unsigned)ceil_div(w_n, 256)), dim3(256), 0, wf, static_cast<float*>(tflip.ptr), ci->filter_h, ci->filter_w,
-                       ci->in_c);
-    TFHIP_LAUNCH_CHECK(ctx);
     tfhip_conv2d_info back = *ci;
     back.in_h = ci->out_h; back.in_w = ci->out_w;
     back.out_h = ci->in_h; back.out_w = ci->in_w;
@@ -599,7 +585,7 @@ extern "C" int tfhip_depthwise_conv2d_der_input(tfhip_ctx* ctx, int64_t dy, int6
     back.pad_top = ci->filter_h - 1 - ci->pad_top;
     back.pad_left = ci->filter_w - 1 - ci->pad_left;
     back.pad_bottom = back.pad_right = 0;   // (not read by the kernels)
-    if ((rc = depthwise_forward_f32(ctx, dyf, static_cast<const float*>(tflip.ptr), dxf, &back))) return rc;
+    if ((rc = depthwise_mirrored_f32(ctx, dyf, wf, dxf, &back))) return rc;
     strncat(ctx->last_kernel, "_as_der_input", sizeof ctx->last_kernel - strlen(ctx->last_kernel) - 1);
     return TFHIP_OK;
   }

@@ -52,6 +52,8 @@ struct DwArgs {
   float* y;
   tfhip_conv2d_info ci;
   int ch_mul;
+  int tap;                   // elements from one filter tap to the next: in_c ch_mul, negative where w is the
+                             // last tap and the filter is taken mirrored in both directions
   int bias_kind, act;
   int quant;
   double qscale, qmin;
@@ -87,14 +89,14 @@ __global__ __launch_bounds__(256) void depthwise3x3_kernel(const DwArgs p) {
     const unsigned char* wq = static_cast<const unsigned char*>(p.w);
 #pragma unroll
     for (int i = 0; i < 9; i++) {
-      const unsigned v = *reinterpret_cast<const unsigned*>(wq + (int64_t)i * C + c);
+      const unsigned v = *reinterpret_cast<const unsigned*>(wq + (int64_t)i * p.tap + c);
 #pragma unroll
       for (int e = 0; e < 4; e++) w[i][e] = dq((v >> (8 * e)) & 0xffu, p.qscale, p.qmin);
     }
   } else {
     const float* wf = static_cast<const float*>(p.w);
 #pragma unroll
-    for (int i = 0; i < 9; i++) w[i] = *reinterpret_cast<const f32x4*>(wf + (int64_t)i * C + c);
+    for (int i = 0; i < 9; i++) w[i] = *reinterpret_cast<const f32x4*>(wf + (int64_t)i * p.tap + c);
   }
 
   const int oh0 = th * TH, ow0 = tw * TW;
@@ -187,14 +189,14 @@ __global__ __launch_bounds__(256) void depthwise3x3_rows_kernel(const DwArgs p, 
     const unsigned char* wq = static_cast<const unsigned char*>(p.w);
 #pragma unroll
     for (int i = 0; i < 9; i++) {
-      const unsigned v = *reinterpret_cast<const unsigned*>(wq + (int64_t)i * C + c);
+      const unsigned v = *reinterpret_cast<const unsigned*>(wq + (int64_t)i * p.tap + c);
 #pragma unroll
       for (int e = 0; e < 4; e++) w[i][e] = dq((v >> (8 * e)) & 0xffu, p.qscale, p.qmin);
     }
   } else {
     const float* wf = static_cast<const float*>(p.w);
 #pragma unroll
-    for (int i = 0; i < 9; i++) w[i] = *reinterpret_cast<const f32x4*>(wf + (int64_t)i * C + c);
+    for (int i = 0; i < 9; i++) w[i] = *reinterpret_cast<const f32x4*>(wf + (int64_t)i * p.tap + c);
   }
   f32x4 b = {0.f, 0.f, 0.f, 0.f};
   if (p.bias_kind == TFHIP_BCAST_COLUMN) b = *reinterpret_cast<const f32x4*>(p.bias + c);
@@ -300,7 +302,7 @@ __global__ void depthwise_generic_kernel(const DwArgs p) {
     t /= ci.out_w;
     const int oh = (int)(t % ci.out_h);
     const int n = (int)(t / ci.out_h);
-    const int c = oc / p.ch_mul, q = oc - c * p.ch_mul;
+    const int c = oc / p.ch_mul;
     float acc = 0.f;
     for (int kh = 0; kh < ci.filter_h; kh++) {
       const int ih = oh * ci.stride_h - ci.pad_top + kh * ci.dilation_h;
@@ -308,7 +310,7 @@ __global__ void depthwise_generic_kernel(const DwArgs p) {
       for (int kw = 0; kw < ci.filter_w; kw++) {
         const int iw = ow * ci.stride_w - ci.pad_left + kw * ci.dilation_w;
         if ((unsigned)iw >= (unsigned)ci.in_w) continue;
-        const int64_t wi = (((int64_t)kh * ci.filter_w + kw) * ci.in_c + c) * p.ch_mul + q;
+        const int64_t wi = ((int64_t)kh * ci.filter_w + kw) * p.tap + oc;
         const float wv = p.quant ? dq(static_cast<const unsigned char*>(p.w)[wi], p.qscale, p.qmin)
                                  : static_cast<const float*>(p.w)[wi];
         acc += p.x[(((int64_t)n * ci.in_h + ih) * ci.in_w + iw) * ci.in_c + c] * wv;
@@ -571,20 +573,22 @@ static int dispatch_depthwise(tfhip_ctx* ctx, DwArgs& p, const tfhip_conv2d_info
   return TFHIP_OK;
 }
 
-// depthwiseConv2D of float32 device buffers without bias or activation: the forward kernels
-// reused by depthwiseConv2DDerInput (stride 1: dx is the depthwise convolution of dy with the
-// spatially flipped filter).
-int depthwise_forward_f32(tfhip_ctx* ctx, const float* x, const float* w, float* y,
-                          const tfhip_conv2d_info* ci) {
+// depthwiseConv2D of float32 device buffers (channel multiplier 1) by the filter mirrored in both
+// directions, without bias or activation: depthwiseConv2DDerInput at stride 1.  The kernels walk the taps
+// from the last to the first; a mirrored copy of the filter was a launch of its own: [32, 56, 56, 128]
+// 20.0 -> 17.7 us, [1, 14, 14, 512] 10.4 -> 7.5.
+int depthwise_mirrored_f32(tfhip_ctx* ctx, const float* x, const float* w, float* y,
+                           const tfhip_conv2d_info* ci) {
   DwArgs p = {};
   p.x = x;
-  p.w = w;
+  p.w = w + (int64_t)(ci->filter_h * ci->filter_w - 1) * ci->in_c;
+  p.tap = -ci->in_c;
   p.y = y;
   p.ci = *ci;
-  p.ch_mul = ci->out_c / ci->in_c;
+  p.ch_mul = 1;
   p.bias_kind = TFHIP_BCAST_NONE;
   p.act = TFHIP_ACT_LINEAR;
-  return dispatch_depthwise(ctx, p, ci, p.ch_mul, TFHIP_BCAST_NONE,
+  return dispatch_depthwise(ctx, p, ci, 1, TFHIP_BCAST_NONE,
                             (int64_t)ci->batch * ci->in_h * ci->in_w * ci->in_c,
                             (int64_t)ci->batch * ci->out_h * ci->out_w * ci->out_c);
 }
@@ -644,6 +648,7 @@ extern "C" int tfhip_depthwise_conv2d(tfhip_ctx* ctx, int64_t x, int64_t filter,
   p.y = static_cast<float*>(bo->ptr);
   p.ci = *ci;
   p.ch_mul = ch_mul;
+  p.tap = ci->out_c;
   p.bias_kind = bias_kind;
   p.act = act;
 

@@ -306,8 +306,8 @@ int launch_convert(tfhip_ctx* ctx, const void* src, int src_dtype, void* dst, in
                    int64_t n);
 
 // image.hip
-int depthwise_forward_f32(tfhip_ctx* ctx, const float* x, const float* w, float* y,
-                          const tfhip_conv2d_info* ci);
+int depthwise_mirrored_f32(tfhip_ctx* ctx, const float* x, const float* w, float* y,
+                           const tfhip_conv2d_info* ci);
 
 inline int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
