@@ -702,9 +702,10 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N * 64) void gemm_kernel(const GemmA
   // this leaves four 64 x 64 workgroups on a CU instead of six, and is the better trade all the same:
   // [4096, 784] x [784, 1024] 66.6 -> 62.3 us, [4096, 1024] x [1024, 1024] 83.5 -> 78.2, [2688, 1792] x
   // [1792, 512] 66.6 -> 58.2, [1000, 784]^T x [1000, 512] 21.3 -> 19.8 (five workgroups, held to 96
-  // registers, give the same).  Only matMul's 256 x 32 tile, which would keep two of three, stays at two
-  // tiles and one set ([2304, 2336] x [2336, 32] 15.2 us, 15.6 with three).
-  constexpr int AHEAD = KBLOCKED && BN == 32 ? 2 : 3;
+  // registers, give the same).  matMul's larger tiles, which have few workgroups on a CU as it is, stay at
+  // two tiles and one set: 128 x 128 on [8192, 4096] x [4096, 4096] 2102 us, 2198 with three; 256 x 32 on
+  // [2304, 2336] x [2336, 32] 15.2 and 15.6.
+  constexpr int AHEAD = KBLOCKED && BM * BN > 64 * 64 ? 2 : 3;
   f32x4 a_reg[2][A_PER], b_reg[2][B_PER];
   Frag f0, f1;
   load_a(L, cur.kt0 * BK, a_reg[0]);
@@ -756,17 +757,30 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N * 64) void gemm_kernel(const GemmA
       for (int j = 0; j < TN; j++) acc[i][j] += blk[i][j];
   };
 
-  if (KBLOCKED) {
+  if (KBLOCKED && AHEAD == 3) {
     static_assert(TILES_PER_KBLOCK == 3, "two blocks of k take six steps");
     for (int i = 0; i < n_steps; i += 6) {
-      step(i, 0, a_reg[SET1], b_reg[SET1], std::true_type{});
+      step(i, 0, a_reg[1], b_reg[1], std::true_type{});
       if (i + 1 < n_steps) step(i + 1, 1, a_reg[0], b_reg[0], std::false_type{});
-      if (i + 2 < n_steps) step(i + 2, 0, a_reg[SET1], b_reg[SET1], std::false_type{});
+      if (i + 2 < n_steps) step(i + 2, 0, a_reg[1], b_reg[1], std::false_type{});
       flush();
       if (i + 3 >= n_steps) break;
       step(i + 3, 1, a_reg[0], b_reg[0], std::true_type{});
-      if (i + 4 < n_steps) step(i + 4, 0, a_reg[SET1], b_reg[SET1], std::false_type{});
+      if (i + 4 < n_steps) step(i + 4, 0, a_reg[1], b_reg[1], std::false_type{});
       if (i + 5 < n_steps) step(i + 5, 1, a_reg[0], b_reg[0], std::false_type{});
+      flush();
+    }
+  } else if (KBLOCKED) {
+    int buf = 0;
+    for (int i = 0; i < n_steps; i += TILES_PER_KBLOCK) {
+      step(i, buf, a_reg[0], b_reg[0], std::true_type{});
+      buf ^= 1;
+#pragma unroll
+      for (int t = 1; t < TILES_PER_KBLOCK; t++)
+        if (i + t < n_steps) {
+          step(i + t, buf, a_reg[0], b_reg[0], std::false_type{});
+          buf ^= 1;
+        }
       flush();
     }
   } else {
@@ -1682,7 +1696,6 @@ static int launch_mode(tfhip_ctx* ctx, GemmArgs& p, int batch) {
   const bool mk = FAST && AMODE == A_ROWMAJOR && BMODE != B_TRANSPOSED && batch == 1 &&
                   p.ldb == p.N && (p.K & 3) == 0 && (p.lda & 3) == 0 &&
                   (long long)p.M * p.N <= 0x7fffffffLL;
-  Plan plans[NCFG];
   // (planned as the general gather is: the same tiles, cut in the same places, the same sums)
   constexpr int PLAN_MODE = AMODE == A_IM2COL_TAPS ? A_IM2COL : AMODE;
   const bool gathered = AMODE == A_IM2COL || AMODE == A_IM2COL_UP || AMODE == A_IM2COL_T || AMODE == A_IM2COL_TAPS;
@@ -1691,20 +1704,39 @@ static int launch_mode(tfhip_ctx* ctx, GemmArgs& p, int batch) {
   const double eff_mid = gathered ? 0.95 : huge ? 0.93 : 0.91;
   const double eff_wide = gathered ? 1.00 : huge ? 0.94 : 0.99;
   const double eff_small = gathered ? 0.92 : huge ? 0.92 : 1.00;
-  plans[0] = make_plan(p, batch, Big::BM, Big::BN, resident_blocks<Big, PLAN_MODE, BMODE, KBLOCKED, FAST>(ctx), cus, eff_big, KBLOCKED, mk);
-  plans[1] = make_plan(p, batch, Mid::BM, Mid::BN, resident_blocks<Mid, PLAN_MODE, BMODE, KBLOCKED, FAST>(ctx), cus, eff_mid, KBLOCKED, mk);
-  plans[2] = make_plan(p, batch, Wide::BM, Wide::BN, resident_blocks<Wide, PLAN_MODE, BMODE, KBLOCKED, FAST>(ctx), cus, eff_wide, KBLOCKED, mk);
-  plans[3] = make_plan(p, batch, Thin::BM, Thin::BN, resident_blocks<Thin, PLAN_MODE, BMODE, KBLOCKED, FAST>(ctx), cus, 0.80, KBLOCKED, mk);
-  plans[4] = make_plan(p, batch, Small::BM, Small::BN, resident_blocks<Small, PLAN_MODE, BMODE, KBLOCKED, FAST>(ctx), cus, eff_small, KBLOCKED, mk);
-  // rows and columns beyond M and N are wasted matrix-core work: charge it
   const int bns[NCFG] = {Big::BN, Mid::BN, Wide::BN, Thin::BN, Small::BN};
   const int bms[NCFG] = {Big::BM, Mid::BM, Wide::BM, Thin::BM, Small::BM};
-  int best = -1;
-  for (int i = 0; i < NCFG; i++) {
-    const double useful = ((double)p.N / (ceil_div(p.N, bns[i]) * bns[i])) *
-                          ((double)p.M / (ceil_div(p.M, bms[i]) * bms[i]));
-    plans[i].cost /= useful;
-    if (best < 0 || plans[i].cost < plans[best].cost) best = i;
+  auto cheapest = [&](Plan (&plans)[NCFG], int small_resident) {
+    plans[0] = make_plan(p, batch, Big::BM, Big::BN, resident_blocks<Big, PLAN_MODE, BMODE, KBLOCKED, FAST>(ctx), cus, eff_big, KBLOCKED, mk);
+    plans[1] = make_plan(p, batch, Mid::BM, Mid::BN, resident_blocks<Mid, PLAN_MODE, BMODE, KBLOCKED, FAST>(ctx), cus, eff_mid, KBLOCKED, mk);
+    plans[2] = make_plan(p, batch, Wide::BM, Wide::BN, resident_blocks<Wide, PLAN_MODE, BMODE, KBLOCKED, FAST>(ctx), cus, eff_wide, KBLOCKED, mk);
+    plans[3] = make_plan(p, batch, Thin::BM, Thin::BN, resident_blocks<Thin, PLAN_MODE, BMODE, KBLOCKED, FAST>(ctx), cus, 0.80, KBLOCKED, mk);
+    plans[4] = make_plan(p, batch, Small::BM, Small::BN, small_resident, cus, eff_small, KBLOCKED, mk);
+    // rows and columns beyond M and N are wasted matrix-core work: charge it
+    int best = -1;
+    for (int i = 0; i < NCFG; i++) {
+      const double useful = ((double)p.N / (ceil_div(p.N, bns[i]) * bns[i])) *
+                            ((double)p.M / (ceil_div(p.M, bms[i]) * bms[i]));
+      plans[i].cost /= useful;
+      if (best < 0 || plans[i].cost < plans[best].cost) best = i;
+    }
+    return best;
+  };
+  Plan plans[NCFG];
+  int best = cheapest(plans, resident_blocks<Small, PLAN_MODE, BMODE, KBLOCKED, FAST>(ctx));
+  if (KBLOCKED && ctx->no_alloc) {
+    // A program that allocates nothing is served where the partial tiles of a plan for six workgroups (five
+    // without FAST or of a transposed A) fit the scratch memory, which does not depend on how the 64 x 64
+    // tile is built; that plan takes over where the one above does not fit.
+    auto fits = [&](const Plan& pl, int i) {
+      return pl.splits <= 1 || (size_t)pl.tail_tiles * pl.splits * bms[i] * bns[i] * sizeof(float) <= kScratchBytes;
+    };
+    Plan six[NCFG];
+    const int which = cheapest(six, AMODE == A_ROWMAJOR && FAST ? 6 : 5);
+    if (!fits(six[which], which) || !fits(plans[best], best)) {
+      best = which;
+      plans[best] = six[best];
+    }
   }
   switch (best) {
     case 0: return launch_cfg<Big, AMODE, BMODE, KBLOCKED, FAST>(ctx, p, plans[0]);
