@@ -1677,12 +1677,12 @@ static int launch_cfg(tfhip_ctx* ctx, GemmArgs& p, const Plan& pl) {
 // shape is measured on MI355X (every tile forced on every shape, interleaved, clocks warm).
 // Row-major operands: [4096, 1024] x [1024, 1024], where every shape fills whole rounds, takes
 // 77.0 us in 128 x 128 tiles, 80.7 in 128 x 64, 74.0 in 64 x 128 and 73.4 in 64 x 64 (four
-// wavefronts of one 32 x 32 accumulator; seven workgroups share a CU, which hides latency better
+// wavefronts of one 32 x 32 accumulator; seven workgroups share a CU, four in matMul, which hides latency better
 // than a deeper pipeline in fewer, larger wavefronts); at [8192, 4096] x [4096, 4096] the large
 // tile, with half the LDS traffic per flop, wins: 2086 / 2233 / 2219 / 2281 us.
 // Implicit GEMM (the A tile is gathered, so reusing it over more columns pays): a 3 x 3
 // convolution of 112 x 112 x 64 -> 128 takes 514 / 536 / 514 / 561 us, 56 x 56 x 128 -> 128
-// 502 / 520 / 494 / 554.
+// 502 / 520 / 494 / 554 (with taps placed per lane; by scalar arithmetic the first takes 453 in its 64 x 128).
 template <int AMODE, int BMODE, bool KBLOCKED, bool FAST>
 static int launch_mode(tfhip_ctx* ctx, GemmArgs& p, int batch) {
   using Big = TileCfg<4, 2, 1, 2>;     // 128 x 128, 8 wavefronts of 32 x 64
