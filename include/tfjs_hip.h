@@ -180,7 +180,10 @@ int tfhip_graph_destroy(tfhip_ctx* ctx, int64_t graph_id);
  * layout), for matching launches to profiler rows.  Not part of the reference interface. */
 const char* tfhip_last_kernel(tfhip_ctx* ctx);
 /* Raw device address of an id's buffer (for callers that share the device, e.g. a
- * harness that generates inputs in HBM).  Not part of the reference interface. */
+ * harness that generates inputs in HBM).  What the caller queues on the address on the default
+ * stream before the id is disposed comes before what the context does with the memory afterwards,
+ * uploads into it among them.  Work on other streams of the caller's is the caller's to finish
+ * first.  Not part of the reference interface. */
 int tfhip_device_ptr(tfhip_ctx* ctx, int64_t id, void** ptr, size_t* nbytes);
 
 /* ---- dense contractions ------------------------------------------------------------ */

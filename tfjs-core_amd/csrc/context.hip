@@ -394,7 +394,7 @@ void tfhip_ctx::park(void* p, size_t cap, hipEvent_t ready, int sidx) {
     return;
   }
   pools[sidx][cap].push_back(p);
-  if (idle == kAllStreams && !capturing) quiet.insert(p);
+  if (idle == kAllStreams && !capturing && !exported.count(p)) quiet.insert(p);
   else quiet.erase(p);
 }
 
@@ -466,6 +466,7 @@ void tfhip_ctx::trim() {
           ev_put(ev->second);
           block_ready.erase(ev);
         }
+        exported.erase(p);
         (void)hipFree(p);
       }
     pool.clear();
@@ -619,7 +620,9 @@ int tfhip_register(tfhip_ctx* ctx, int64_t id, const int32_t* shape, int rank, i
 // The upload stream may overwrite a block only after the compute-stream work that used it:
 // it waits for the event the block's last owner left (release_buf), or, when the history is
 // not known (a live buffer overwritten, a recycled block without an event), for everything
-// queued on the compute stream so far.  A buffer fresh from the driver needs no wait.
+// queued on the compute stream so far.  A buffer fresh from the driver needs no wait, and neither does a
+// block that went back to the pool while every compute stream was idle (tfhip_ctx::quiet), unless
+// its address was ever given out.
 int tfhip_write(tfhip_ctx* ctx, int64_t id, const void* host, size_t nbytes) {
   if (!ctx) return TFHIP_EINVAL;
   if (ctx->capturing)
@@ -1065,9 +1068,12 @@ const char* tfhip_last_kernel(tfhip_ctx* ctx) { return ctx ? ctx->last_kernel : 
 
 int tfhip_device_ptr(tfhip_ctx* ctx, int64_t id, void** ptr, size_t* nbytes) {
   if (!ctx || !ptr) return TFHIP_EINVAL;
-  const unsigned char idle = ctx->idle;  // (nothing is queued here)
+  // (Of this context's own work nothing is queued here, so its streams are as idle as they were.
+  // What the caller queues on the address they cannot see.)
+  const unsigned char idle = ctx->idle;
   TFHIP_GET(ctx, b, id);
   ctx->idle = idle;
+  if (b->ptr) ctx->exported.insert(b->ptr);
   *ptr = b->ptr;
   if (nbytes) *nbytes = b->nbytes;
   return TFHIP_OK;

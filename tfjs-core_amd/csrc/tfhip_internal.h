@@ -132,7 +132,13 @@ struct tfhip_ctx {
   // Streams on which nothing was queued since the host last waited for them (a bit per stream).  (Asking
   // the driver costs up to 10 us where there is work.)
   unsigned char idle = kAllStreams;
-  std::unordered_set<void*> quiet;  // free blocks that came back while every stream was idle: no work left on them
+  // Free blocks that came back while every stream was idle, so that no work is left on them: the next
+  // upload into one starts without a fence, as into a block fresh from the driver.  A block whose address
+  // was given out (tfhip_device_ptr) is never one of them: work that others queued on it is seen by no
+  // stream of this context, and what puts the upload behind it is the fence on a compute
+  // stream, which the default stream's work comes before.  (By block and not by buffer: the next buffer in
+  // it may be let go before anything of its own was queued.)
+  std::unordered_set<void*> quiet, exported;
   // A pinned block per compute stream for a larger write that finds the stream idle: the copy out of it
   // runs on that stream, so an idle stream also says that the block is free.
   char* stages[kStreams] = {};
