@@ -93,6 +93,66 @@ def test_records(fake):
         Tensor.__new__(Tensor).dispose()
 
 
+FIELDS = ["shape", "dtype", "size", "rank", "data_id", "quant", "is_disposed", "id"]
+
+
+@pytest.mark.parametrize("field", FIELDS + ["all"])
+def test_half_made_records_raise(fake, field):
+    """A record without a field (made by __new__ alone, or the field deleted) is an AttributeError."""
+    import tfhip as tf
+    from tfhip import _capi, _native
+    from tfhip.engine import ENGINE, Tensor
+    _capi.lib()
+    core = _native.BackendCore.__new__(_native.BackendCore)     # (no context: what reaches the library fails)
+    base = counts()
+    ENGINE.start_scope()
+    t = tf.tensor(np.zeros((2, 3), np.float32)) if field != "all" else Tensor.__new__(Tensor)
+    kept = {f: getattr(t, f, None) for f in FIELDS}
+    if field == "all":
+        ENGINE.scopes[-1].append(t)
+    else:
+        delattr(t, field)
+    needed = lambda *fields: field == "all" or field in fields
+    calls = [(lambda: ENGINE.dispose_tensor(t), needed("data_id")),
+             (lambda: ENGINE.end_scope(), needed("is_disposed", "data_id")),
+             (lambda: t.dispose(), needed("is_disposed", "data_id")),
+             (lambda: core._alias(t, (6,)), needed("data_id", "dtype", "quant")),
+             (lambda: core._unary_out(0, t, "float32", 0.0, 0.0), needed("shape")),
+             (lambda: core._binary_out(0, t, t, "float32"), needed("shape")),
+             (lambda: core._softmax_out(t, 2, 3), needed("shape")),
+             (lambda: core._matmul_out(t, t, (1, 2, 2), 1, 2, 2, 3, 0, 1, None, 0, 0, None, 0), needed("quant"))]
+    for call, missing in calls:
+        if missing:
+            with pytest.raises(AttributeError):
+                call()
+    if field == "all":
+        while ENGINE.scopes:
+            ENGINE.scopes.pop()
+        return
+    for f in FIELDS:
+        setattr(t, f, kept[f])
+    if not t.is_disposed:
+        t.dispose()
+    while ENGINE.scopes:
+        ENGINE.end_scope()
+    assert counts() == base and not fake.live
+
+
+def test_an_engine_without_its_backend_field_raises(fake):
+    import tfhip as tf
+    from tfhip.engine import ENGINE, Tensor
+    backend = ENGINE._backend
+    del ENGINE._backend
+    try:
+        for call in (lambda: ENGINE.run_kernel(lambda be: be), lambda: ENGINE.tidy(lambda: tf.tensor(1.0)),
+                     lambda: Tensor((1,), "float32", None, np.zeros(1, np.float32))):
+            with pytest.raises(AttributeError):
+                call()
+    finally:
+        ENGINE._backend = backend
+    assert ENGINE.scopes == []
+
+
 def test_nothing_is_held(fake):
     import tfhip as tf
     value = np.zeros(7, np.float32)

@@ -89,9 +89,15 @@ static PyTypeObject Tensor_Type, Engine_Type, Backend_Type;
 static EngineObject* engine;
 static long long next_tensor_id;
 
+/* A field that was never set (a record made by __new__ alone) or was deleted: what Python says then. */
+static int there(PyObject* field, const char* name) {
+  if (!field) PyErr_Format(PyExc_AttributeError, "'%s' is not set", name);
+  return field != NULL;
+}
+
 /* ---- shapes ------------------------------------------------------------------------------------ */
 static PyObject* as_shape(PyObject* shape) {  /* a tuple of ints; new reference */
-  if (!shape) return PyErr_Format(PyExc_AttributeError, "the tensor was never made");
+  if (!there(shape, "shape")) return NULL;
   if (PyTuple_CheckExact(shape)) {
     Py_ssize_t i, n = PyTuple_GET_SIZE(shape);
     for (i = 0; i < n && PyLong_CheckExact(PyTuple_GET_ITEM(shape, i)); i++) {}
@@ -137,7 +143,8 @@ static PyObject* product(PyObject* shape) {
 #define MAX_DIMS 64
 /* Dimensions as the library takes them (it checks the rank itself: 8 at most). */
 static int dims_of(PyObject* shape, int32_t* dims) {
-  if (!shape || !PyTuple_Check(shape)) {
+  if (!there(shape, "shape")) return -1;
+  if (!PyTuple_Check(shape)) {
     PyErr_SetString(PyExc_TypeError, "a tensor's shape is a tuple");
     return -1;
   }
@@ -295,6 +302,7 @@ out:
 }
 
 static int engine_dispose(EngineObject* e, TensorObject* t) {
+  if (!there(t->data_id, "data_id")) return -1;
   PyObject* rec = PyDict_GetItemWithError(e->ref, t->data_id);
   if (!rec) return PyErr_Occurred() ? -1 : 0;
   e->num_tensors--;
@@ -326,6 +334,7 @@ static int engine_dispose(EngineObject* e, TensorObject* t) {
 }
 
 static int tensor_dispose(TensorObject* t) {
+  if (!there(t->is_disposed, "is_disposed") || !there((PyObject*)engine, "engine")) return -1;
   const int gone = PyObject_IsTrue(t->is_disposed);
   if (gone) return gone < 0 ? -1 : 0;
   if (engine_dispose(engine, t)) return -1;
@@ -481,6 +490,7 @@ static PyObject* Engine_end(EngineObject* e, PyObject* const* args, Py_ssize_t n
 static PyObject* Engine_scoped(EngineObject* e, PyObject* fn) { return engine_scoped(e, fn, NULL); }
 static PyObject* Engine_run_kernel(EngineObject* e, PyObject* forward) {
   PyObject* be = e->backend;
+  if (!there(be, "_backend")) return NULL;
   if (be != Py_None) Py_INCREF(be);
   else if (!(be = PyObject_GetAttr((PyObject*)e, s_backend))) return NULL;
   PyObject* r = engine_scoped(e, forward, be);
@@ -571,7 +581,7 @@ static int Tensor_init(TensorObject* t, PyObject* args, PyObject* kwds) {
   Py_DECREF(dims);
   if (!rc && values != Py_None) {
     PyObject* to = backend != Py_None ? backend : engine->backend;
-    if (Py_TYPE(to) == backend_class) {
+    if (to && Py_TYPE(to) == backend_class) {
       const int written = backend_write_plain((BackendObject*)to, t->data_id, values);
       if (written) return written > 0 ? 0 : -1;
     }
@@ -606,7 +616,6 @@ static void Tensor_dealloc(TensorObject* t) {
 }
 static PyObject* Tensor_dispose(TensorObject* t, PyObject* unused) {
   (void)unused;
-  if (!t->is_disposed || !t->data_id) return PyErr_Format(PyExc_AttributeError, "dispose: the tensor was never made");
   if (tensor_dispose(t)) return NULL;
   Py_RETURN_NONE;
 }
@@ -680,9 +689,11 @@ static int optional_handle(BackendObject* be, PyObject* t, long long kind, int64
 }
 /* (scale, min) of quantised weights, or None. */
 static int quant_of(PyObject* t, tfhip_qparams* q, const tfhip_qparams** out) {
-  PyObject* v = PyObject_TypeCheck(t, &Tensor_Type) ? ((TensorObject*)t)->quant : NULL;
   *out = NULL;
-  if (!v || v == Py_None) return 0;
+  if (!PyObject_TypeCheck(t, &Tensor_Type)) return 0;
+  PyObject* v = ((TensorObject*)t)->quant;
+  if (!there(v, "quant")) return -1;
+  if (v == Py_None) return 0;
   if (!PyTuple_Check(v) || PyTuple_GET_SIZE(v) != 2) {
     PyErr_SetString(PyExc_TypeError, "quant is (scale, min)");
     return -1;
@@ -779,7 +790,7 @@ static PyObject* Backend_alias(BackendObject* be, PyObject* const* args, Py_ssiz
   NEED("_alias", 2);
   if (!PyObject_TypeCheck(args[0], &Tensor_Type)) return PyErr_Format(PyExc_TypeError, "_alias: not a tensor");
   TensorObject* x = (TensorObject*)args[0];
-  if (!x->data_id) return PyErr_Format(PyExc_AttributeError, "_alias: the tensor was never made");
+  if (!there(x->data_id, "data_id") || !there(x->dtype, "dtype") || !there(x->quant, "quant")) return NULL;
   return make_tensor(args[1], x->dtype, x->data_id, (PyObject*)be, x->quant, x->dtype);
 }
 /* _binary_out(op, a, b, dtype): None when the shapes do not broadcast. */
