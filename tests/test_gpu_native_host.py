@@ -66,3 +66,21 @@ def test_products_of_any_rank_and_epilogue(tf):
         np.testing.assert_array_equal(r.data_sync(), ints @ ints.T)
         for value in (2.5, -0.0, float("inf"), float("nan"), 1e-45):
             np.testing.assert_array_equal(tf.tensor(value).data_sync(), np.float32(value))
+
+
+@pytest.mark.parametrize("quant", [(0.25, -3.0), [0.25, -3.0], [1, -3]])
+def test_quantised_weights_in_any_sequence(tf, quant):
+    """What the dense kernels take as (scale, min) is what dequantize takes."""
+    from tfhip.engine import Tensor
+    rng = np.random.default_rng(5)
+    a, q = rng.standard_normal((6, 16)).astype(np.float32), rng.integers(0, 256, (16, 8)).astype(np.uint8)
+    want = a.astype(np.float64) @ (q * float(quant[0]) + quant[1])
+    with tf.tidy():
+        w = Tensor((16, 8), "float32", None, q, tf.backend(), quant)
+        got = tf.matmul(tf.tensor(a), w).data_sync()
+        x, f = tf.tensor(a.reshape(1, 2, 3, 16)), tf.reshape(w, (1, 1, 16, 8))
+        conv = tf.fused.conv2d(x, f, 1, "valid").data_sync()
+    # (float32 sums of 16 products: 17 roundings of terms of at most this size)
+    bound = 17 * 2.0 ** -24 * (np.abs(a) @ np.abs(q * float(quant[0]) + quant[1]))
+    assert np.all(np.abs(got - want) <= bound)
+    assert np.all(np.abs(conv.reshape(6, 8) - want) <= bound)

@@ -687,21 +687,24 @@ static int optional_handle(BackendObject* be, PyObject* t, long long kind, int64
   *handle = -1;
   return t == Py_None || !kind ? 0 : handle_of(be, t, handle);
 }
-/* (scale, min) of quantised weights, or None. */
+/* (scale, min) of quantised weights, in any sequence; None, or anything empty, for others. */
 static int quant_of(PyObject* t, tfhip_qparams* q, const tfhip_qparams** out) {
   *out = NULL;
   if (!PyObject_TypeCheck(t, &Tensor_Type)) return 0;
   PyObject* v = ((TensorObject*)t)->quant;
   if (!there(v, "quant")) return -1;
-  if (v == Py_None) return 0;
-  if (!PyTuple_Check(v) || PyTuple_GET_SIZE(v) != 2) {
-    PyErr_SetString(PyExc_TypeError, "quant is (scale, min)");
-    return -1;
+  const int given = PyObject_IsTrue(v);
+  if (given <= 0) return given;
+  double* const values[] = {&q->scale, &q->min};
+  for (int i = 0; i < 2; i++) {
+    PyObject* item = PySequence_GetItem(v, i);
+    if (!item) return -1;
+    *values[i] = PyFloat_AsDouble(item);
+    Py_DECREF(item);
+    if (*values[i] == -1.0 && PyErr_Occurred()) return -1;
   }
-  q->scale = PyFloat_AsDouble(PyTuple_GET_ITEM(v, 0));
-  q->min = PyFloat_AsDouble(PyTuple_GET_ITEM(v, 1));
   *out = q;
-  return PyErr_Occurred() ? -1 : 0;
+  return 0;
 }
 /* The geometry of a convolution or a pool, packed by the caller. */
 static int geometry(PyObject* packed, tfhip_conv2d_info* info) {
