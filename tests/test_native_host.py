@@ -153,6 +153,36 @@ def test_an_engine_without_its_backend_field_raises(fake):
     assert ENGINE.scopes == []
 
 
+def test_arguments_by_name(fake):
+    """The engine's and the backend's methods take their arguments by name, as Python functions do."""
+    import tfhip as tf
+    from tfhip import _native
+    from tfhip.engine import ENGINE, DataId, Tensor
+    base = counts()
+    ENGINE.start_scope()
+    a, b = tf.tensor(1.0), tf.tensor(2.0)
+    ENGINE.end_scope(result=a)
+    assert b.is_disposed and not a.is_disposed
+    assert ENGINE.run_kernel(forward=lambda be: be) is fake
+    t = Tensor.__new__(Tensor)                                   # a record that the program registers itself
+    t.shape, t.size, t.dtype, t.rank, t.data_id, t.is_disposed = (3,), 3, "int32", 1, DataId(), False
+    ENGINE.register_tensor(t=t, backend=None, storage_dtype="int32")
+    assert t.data_id in fake.live and counts() == (base[0] + 2, base[1] + 2, base[2] + 16)
+    ENGINE.dispose_tensor(t=t)
+    ENGINE.dispose_tensor(t=a)
+    assert counts() == base and not fake.live
+    core = _native.BackendCore.__new__(_native.BackendCore)
+    core.dispose_data(data_id=DataId())
+    with pytest.raises(KeyError):
+        core.register(shape=[2, 3], dtype="float64", data_id=DataId())
+    for call in (lambda: ENGINE.run_kernel(), lambda: ENGINE.run_kernel(lambda be: be, forward=None),
+                 lambda: ENGINE.end_scope(a, a), lambda: ENGINE.dispose_tensor(tensor=a),
+                 lambda: core.register(DataId(), (1,))):
+        with pytest.raises(TypeError):
+            call()
+    assert ENGINE.scopes == []
+
+
 def test_nothing_is_held(fake):
     import tfhip as tf
     value = np.zeros(7, np.float32)

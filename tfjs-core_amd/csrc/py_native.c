@@ -95,6 +95,37 @@ static int there(PyObject* field, const char* name) {
   return field != NULL;
 }
 
+/* The arguments of a call by position or by name (METH_FASTCALL | METH_KEYWORDS) -> out, of which the first
+ * `needed` have to be there; the others stay NULL.  At most 4. */
+static int named(const char* call, PyObject* const* args, Py_ssize_t n, PyObject* keywords, const char* const* names,
+                 int count, int needed, PyObject** out) {
+  if (n > count) {
+    PyErr_Format(PyExc_TypeError, "%s takes %d arguments, got %zd", call, count, n);
+    return -1;
+  }
+  for (int i = 0; i < count; i++) out[i] = i < n ? args[i] : NULL;
+  for (Py_ssize_t k = 0; keywords && k < PyTuple_GET_SIZE(keywords); k++) {
+    PyObject* name = PyTuple_GET_ITEM(keywords, k);
+    int i = 0;
+    while (i < count && PyUnicode_CompareWithASCIIString(name, names[i])) i++;
+    if (i == count || out[i]) {
+      PyErr_Format(PyExc_TypeError, "%s: %s argument '%U'", call, i == count ? "no" : "a second", name);
+      return -1;
+    }
+    out[i] = args[n + k];
+  }
+  for (int i = 0; i < needed; i++)
+    if (!out[i]) {
+      PyErr_Format(PyExc_TypeError, "%s needs the argument '%s'", call, names[i]);
+      return -1;
+    }
+  return 0;
+}
+#define ARGUMENTS(call, count, needed, ...)                                      \
+  PyObject* a[count];                                                            \
+  static const char* const arg_names[] = {__VA_ARGS__};                          \
+  if (named(call, args, n, keywords, arg_names, count, needed, a)) return NULL
+
 /* ---- shapes ------------------------------------------------------------------------------------ */
 static PyObject* as_shape(PyObject* shape) {  /* a tuple of ints; new reference */
   if (!there(shape, "shape")) return NULL;
@@ -472,9 +503,19 @@ static PyObject* Engine_new(PyTypeObject* type, PyObject* args, PyObject* kwds) 
   if (!e->ref || !e->scopes) Py_CLEAR(e);
   return (PyObject*)e;
 }
-static PyObject* Engine_dispose_tensor(EngineObject* e, PyObject* t) {
-  if (!PyObject_TypeCheck(t, &Tensor_Type)) return PyErr_Format(PyExc_TypeError, "dispose_tensor: not a tensor");
-  if (engine_dispose(e, (TensorObject*)t)) return NULL;
+static PyObject* Engine_register_tensor(EngineObject* e, PyObject* const* args, Py_ssize_t n, PyObject* keywords) {
+  ARGUMENTS("register_tensor", 3, 3, "t", "backend", "storage_dtype");
+  if (!PyObject_TypeCheck(a[0], &Tensor_Type)) return PyErr_Format(PyExc_TypeError, "register_tensor: not a tensor");
+  TensorObject* t = (TensorObject*)a[0];
+  if (!there(t->data_id, "data_id") || !there(t->shape, "shape") || !there(t->size, "size")) return NULL;
+  const int given = PyObject_IsTrue(a[1]);
+  if (given < 0 || engine_register(e, t, given ? a[1] : Py_None, a[2])) return NULL;
+  Py_RETURN_NONE;
+}
+static PyObject* Engine_dispose_tensor(EngineObject* e, PyObject* const* args, Py_ssize_t n, PyObject* keywords) {
+  ARGUMENTS("dispose_tensor", 1, 1, "t");
+  if (!PyObject_TypeCheck(a[0], &Tensor_Type)) return PyErr_Format(PyExc_TypeError, "dispose_tensor: not a tensor");
+  if (engine_dispose(e, (TensorObject*)a[0])) return NULL;
   Py_RETURN_NONE;
 }
 static PyObject* Engine_start(EngineObject* e, PyObject* unused) {
@@ -482,18 +523,19 @@ static PyObject* Engine_start(EngineObject* e, PyObject* unused) {
   if (engine_start_scope(e)) return NULL;
   Py_RETURN_NONE;
 }
-static PyObject* Engine_end(EngineObject* e, PyObject* const* args, Py_ssize_t n) {
-  if (n > 1) return PyErr_Format(PyExc_TypeError, "end_scope takes one result");
-  if (engine_end_scope(e, n ? args[0] : Py_None)) return NULL;
+static PyObject* Engine_end(EngineObject* e, PyObject* const* args, Py_ssize_t n, PyObject* keywords) {
+  ARGUMENTS("end_scope", 1, 0, "result");
+  if (engine_end_scope(e, a[0] ? a[0] : Py_None)) return NULL;
   Py_RETURN_NONE;
 }
 static PyObject* Engine_scoped(EngineObject* e, PyObject* fn) { return engine_scoped(e, fn, NULL); }
-static PyObject* Engine_run_kernel(EngineObject* e, PyObject* forward) {
+static PyObject* Engine_run_kernel(EngineObject* e, PyObject* const* args, Py_ssize_t n, PyObject* keywords) {
+  ARGUMENTS("run_kernel", 1, 1, "forward");
   PyObject* be = e->backend;
   if (!there(be, "_backend")) return NULL;
   if (be != Py_None) Py_INCREF(be);
   else if (!(be = PyObject_GetAttr((PyObject*)e, s_backend))) return NULL;
-  PyObject* r = engine_scoped(e, forward, be);
+  PyObject* r = engine_scoped(e, a[0], be);
   Py_DECREF(be);
   return r;
 }
@@ -505,14 +547,16 @@ static PyMemberDef Engine_members[] = {
     {"num_bytes", T_LONGLONG, offsetof(EngineObject, num_bytes), 0, NULL},
     {"num_data_buffers", T_LONGLONG, offsetof(EngineObject, num_data_buffers), 0, NULL},
     {NULL}};
+#define NAMED(name, fn, doc) {name, (PyCFunction)(void (*)(void))fn, METH_FASTCALL | METH_KEYWORDS, doc}
 static PyMethodDef Engine_methods[] = {
-    {"dispose_tensor", (PyCFunction)Engine_dispose_tensor, METH_O, "engine.ts:502-572"},
+    NAMED("register_tensor", Engine_register_tensor, "register_tensor(t, backend, storage_dtype): engine.ts:502-530"),
+    NAMED("dispose_tensor", Engine_dispose_tensor, "dispose_tensor(t): engine.ts:540-572"),
     {"start_scope", (PyCFunction)Engine_start, METH_NOARGS, "engine.ts:675-690"},
-    {"end_scope", (PyCFunction)(void (*)(void))Engine_end, METH_FASTCALL, "engine.ts:691-718"},
+    NAMED("end_scope", Engine_end, "end_scope(result=None): engine.ts:691-718"),
     {"scoped", (PyCFunction)Engine_scoped, METH_O, "fn() inside a scope of its own; what it returns is kept."},
-    {"run_kernel", (PyCFunction)Engine_run_kernel, METH_O,
-     "ENGINE.runKernel without a tape (engine.ts:435-498): the forward function gets the active backend; "
-     "intermediates made inside are released when it returns."},
+    NAMED("run_kernel", Engine_run_kernel,
+          "run_kernel(forward): ENGINE.runKernel without a tape (engine.ts:435-498): the forward function gets the "
+          "active backend; intermediates made inside are released when it returns."),
     {NULL}};
 static PyTypeObject Engine_Type = {
     PyVarObject_HEAD_INIT(NULL, 0).tp_name = "tfhip._native.EngineCore",
@@ -745,17 +789,18 @@ static PyObject* Backend_bind(BackendObject* be, PyObject* address) {
   be->ctx = (tfhip_ctx*)p;
   Py_RETURN_NONE;
 }
-static PyObject* Backend_register(BackendObject* be, PyObject* const* args, Py_ssize_t n) {
-  NEED("register", 3);
-  PyObject* dims = as_shape(args[1]);
+static PyObject* Backend_register(BackendObject* be, PyObject* const* args, Py_ssize_t n, PyObject* keywords) {
+  ARGUMENTS("register", 3, 3, "data_id", "shape", "dtype");
+  PyObject* dims = as_shape(a[1]);
   if (!dims) return NULL;
-  const int rc = backend_register(be, args[0], dims, args[2]);
+  const int rc = backend_register(be, a[0], dims, a[2]);
   Py_DECREF(dims);
   if (rc) return NULL;
   Py_RETURN_NONE;
 }
-static PyObject* Backend_dispose_data(BackendObject* be, PyObject* data_id) {
-  if (backend_dispose_data(be, data_id)) return NULL;
+static PyObject* Backend_dispose_data(BackendObject* be, PyObject* const* args, Py_ssize_t n, PyObject* keywords) {
+  ARGUMENTS("dispose_data", 1, 1, "data_id");
+  if (backend_dispose_data(be, a[0])) return NULL;
   Py_RETURN_NONE;
 }
 /* _write(data_id, contiguous array): the caller has checked its type and length. */
@@ -967,8 +1012,8 @@ static PyMemberDef Backend_members[] = {
     {NULL}};
 static PyMethodDef Backend_methods[] = {
     {"_bind", (PyCFunction)Backend_bind, METH_O, "the address of the library's context, 0 for none"},
-    FAST("register", Backend_register),
-    {"dispose_data", (PyCFunction)Backend_dispose_data, METH_O, NULL},
+    NAMED("register", Backend_register, "register(data_id, shape, dtype)"),
+    NAMED("dispose_data", Backend_dispose_data, "dispose_data(data_id)"),
     FAST("_write", Backend_write),
     {"_h", (PyCFunction)Backend_h, METH_O, "the library's handle of a tensor's buffer"},
     FAST("_out", Backend_out),
