@@ -183,6 +183,46 @@ def test_arguments_by_name(fake):
     assert ENGINE.scopes == []
 
 
+@pytest.mark.parametrize("derived", [True, False])
+def test_replaced_product_methods_are_called(fake, derived):
+    """matMul goes through batch_mat_mul, fused_batch_mat_mul and reshape of a backend that replaces them, be it in
+    a class of its own or in the instance."""
+    import tfhip as tf
+    from tfhip.backend_hip import MathBackendHIP
+    from tfhip.engine import ENGINE
+    calls = []
+
+    def reshape(x, shape):
+        calls.append(tuple(shape))
+        return x
+
+    def batch_mat_mul(a, b, transpose_a, transpose_b):
+        calls.append((transpose_a, transpose_b))
+        return a
+
+    def fused_batch_mat_mul(a, b, transpose_a, transpose_b, bias, activation, weights):
+        calls.append((transpose_a, transpose_b, bias, activation))
+        return b
+    methods = dict(reshape=reshape, batch_mat_mul=batch_mat_mul, fused_batch_mat_mul=fused_batch_mat_mul)
+    if derived:
+        as_methods = {k: (lambda f: lambda self, *a: f(*a))(f) for k, f in methods.items()}
+        be = type("Derived", (MathBackendHIP,), dict(as_methods, __init__=lambda self: None))()
+    else:
+        be = MathBackendHIP.__new__(MathBackendHIP)
+        be.__dict__.update(methods)
+    a, b = tf.tensor(np.zeros((2, 3), np.float32)), tf.tensor(np.zeros((3, 4), np.float32))
+    backend, ENGINE._backend = ENGINE._backend, be
+    try:
+        assert tf.matmul(a, b) is a
+        assert calls == [(1, 2, 3), (1, 3, 4), (False, False), (2, 4)]
+        del calls[:]
+        assert tf.fused.matmul(a, b, activation="relu") is b
+        assert calls == [(1, 2, 3), (1, 3, 4), (False, False, None, "relu"), (2, 4)]
+    finally:
+        ENGINE._backend = backend
+    tf.dispose([a, b])
+
+
 def test_nothing_is_held(fake):
     import tfhip as tf
     value = np.zeros(7, np.float32)

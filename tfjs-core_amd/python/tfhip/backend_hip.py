@@ -116,6 +116,9 @@ class _PendingRead:
             b.lib.tfhip_read_finish(b.ctx if b.ctx else None, self._ticket, None, 0)
 
 
+_PRODUCT_METHODS = frozenset(("reshape", "batch_mat_mul", "fused_batch_mat_mul"))
+
+
 class MathBackendHIP(_native.BackendCore):
     # data: DataId -> (handle, storage dtype code, numel)
     def __new__(cls, *args, **kwargs):
@@ -339,7 +342,10 @@ class MathBackendHIP(_native.BackendCore):
                    activation="linear", prelu_activation_weights=None):
         """Extension of the plug-in API: the batched product straight from operands of any rank into
         `out_shape`, without a reshape before and after it.  None when the epilogue is one that
-        fused_batch_mat_mul does in separate passes."""
+        fused_batch_mat_mul does in separate passes, and where a derived class or the program
+        may have put its own methods in the place of those that this call stands for."""
+        if type(self) is not MathBackendHIP or not _PRODUCT_METHODS.isdisjoint(self.__dict__):
+            return None
         if activation not in capi.ACT or a.dtype != "float32":
             return None
         bk = pk = 0
