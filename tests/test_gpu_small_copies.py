@@ -61,3 +61,43 @@ def test_a_copy_is_no_kernel_of_a_timed_region(tf):
         x = tf.tensor(np.ones(300000, np.float32))
         info = tf.time(lambda: tf.add(tf.mul(x, 2.0), tf.tensor(np.ones(300000, np.float32))).data_sync())
         assert len(info["kernelTimes"]) == 2
+
+
+def _address_space():
+    with open("/proc/self/status") as f:
+        return next(int(line.split()[1]) << 10 for line in f if line.startswith("VmSize"))
+
+
+def test_reads_of_many_sizes_share_their_memory(tf):
+    """Page-locked memory for reads does not grow with the number of sizes that are read."""
+    sizes = [(512 << 10) - 4 * i for i in range(0, 128 * 160, 160)] + [1, 3, 128, 129]
+    with tf.tidy():
+        made = [tf.add(tf.tensor(np.full(n // 4 or 1, n, np.float32)), tf.tensor(np.float32(0.5))) for n in sizes]
+        made[0].data_sync()
+        before = _address_space()
+        for n, t in zip(sizes, made):
+            got = t.data_sync()
+            assert got.size == (n // 4 or 1) and np.all(got == np.float32(n + 0.5))
+        # (a block per size would be 56 MB)
+        assert _address_space() - before < 16 << 20
+
+
+def test_reads_on_several_threads(tf):
+    import threading
+    wrong = []
+    with tf.tidy():
+        made = [tf.add(tf.tensor(np.arange(n, dtype=np.float32)), tf.tensor(np.float32(i)))
+                for i, n in enumerate((1000, 70000, 250000, 200000))]
+        tf.backend().sync()
+
+        def read(i, t):
+            for _ in range(200):
+                got = t.data_sync()
+                if not np.array_equal(got, np.arange(got.size, dtype=np.float32) + i):
+                    wrong.append(i)
+        threads = [threading.Thread(target=read, args=(i, t)) for i, t in enumerate(made)]
+        for t in threads:
+            t.start()
+        for t in threads:
+            t.join()
+    assert not wrong

@@ -234,15 +234,17 @@ void tfhip_ctx::order(int earlier, int later) {
   (void)hipStreamSynchronize(streams[earlier]);
 }
 
-char* tfhip_ctx::idle_stage() {
-  if (!(idle >> cur & 1)) return nullptr;
-  char*& block = stages[cur];
-  if (!block && hipHostMalloc((void**)&block, tfhip::kCopyKernelBytes, hipHostMallocDefault) != hipSuccess) {
+namespace tfhip {
+static char* staging_block(char*& block) {
+  if (!block && hipHostMalloc((void**)&block, kCopyKernelBytes, hipHostMallocDefault) != hipSuccess) {
     (void)hipGetLastError();
     block = nullptr;
   }
   return block;
 }
+}  // namespace tfhip
+
+char* tfhip_ctx::idle_stage() { return idle >> cur & 1 ? tfhip::staging_block(stages[cur]) : nullptr; }
 
 hipEvent_t tfhip_ctx::ev_get() {
   if (!free_events.empty()) {
@@ -552,6 +554,7 @@ void tfhip_destroy(tfhip_ctx* ctx) {
   if (ctx->ring) (void)hipHostFree(ctx->ring);
   for (char* block : ctx->stages)
     if (block) (void)hipHostFree(block);
+  if (ctx->read_block) (void)hipHostFree(ctx->read_block);
   for (auto& pool : ctx->pools)
     for (auto& kv : pool)
       for (void* p : kv.second) (void)hipFree(p);
@@ -728,14 +731,17 @@ int tfhip_read(tfhip_ctx* ctx, int64_t id, void* host, size_t nbytes) {
   if (nbytes != b->nbytes)
     return ctx->fail(TFHIP_EINVAL, "read: asked %zu bytes of a buffer of %zu", nbytes, b->nbytes);
   hipStream_t last = ctx->streams[b->sidx];  // the stream that produced (or last used) the buffer
-  if (nbytes && nbytes <= tfhip::kCopyKernelBytes) {
-    size_t cap = 0;
-    if (void* staged = tfhip::staging_get(nbytes, &cap)) {
-      hipError_t e = tfhip::copy_block(b->ptr, staged, nbytes, last);
-      const hipError_t done = hipStreamSynchronize(last);  // (also after a failed launch: the block goes back)
+  if (nbytes && nbytes <= tfhip::kCopyKernelBytes && !ctx->read_block_taken.test_and_set(std::memory_order_acquire)) {
+    char* staged = tfhip::staging_block(ctx->read_block);
+    hipError_t e = hipSuccess;
+    if (staged) {
+      e = tfhip::copy_block(b->ptr, staged, nbytes, last);
+      const hipError_t done = hipStreamSynchronize(last);  // (also after a failed launch: the block is free again)
       if (e == hipSuccess) e = done;
       if (e == hipSuccess) memcpy(host, staged, nbytes);
-      tfhip::staging_put(staged, cap);
+    }
+    ctx->read_block_taken.clear(std::memory_order_release);
+    if (staged) {
       ctx->idle |= (unsigned char)(1u << b->sidx);
       if (e != hipSuccess) {
         (void)hipGetLastError();

@@ -1,5 +1,6 @@
 // Internal declarations shared by the translation units of libtfjs_hip.so.
 #pragma once
+#include <atomic>
 #include <hip/hip_runtime.h>
 #include <hip/hip_ext.h>
 
@@ -143,6 +144,10 @@ struct tfhip_ctx {
   // runs on that stream, so an idle stream also says that the block is free.
   char* stages[kStreams] = {};
   char* idle_stage();  // the selected stream's block, or nullptr (work is queued, or no memory)
+  // The same for reads, which wait for their copy: one block, of every size up to its own.  A read that
+  // finds it taken (by a read on another thread) copies straight into the caller's memory.
+  char* read_block = nullptr;
+  std::atomic_flag read_block_taken = ATOMIC_FLAG_INIT;
   // Streams that may hold queued work which a graph replay has not been ordered behind yet (a bit
   // per stream, set when the stream is selected): a replay waits for these, see tfhip_graph_launch.
   unsigned char dirty = 1;
