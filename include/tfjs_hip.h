@@ -211,9 +211,10 @@ int tfhip_matmul(tfhip_ctx* ctx, int64_t a, int64_t b, int64_t out, int batch, i
  * few tiles to fill the GPU), this entry point uses a static device array of 8 MiB that the
  * library holds on every GPU it runs on until the process ends.  A product whose partial
  * tiles need more fails with TFHIP_ENOTSUP, as does an operand that is not stored as float32
- * (its converted copy would need a block; b may be TFHIP_UINT8Q).  One kind of product differs:
- * transposed or batched, cut by tfhip_matmul's bf16 kernels into more partial tiles than the array
- * holds.  It takes the float32 kernels here, and agrees to rounding.  All calls on one GPU share
+ * (its converted copy would need a block; b may be TFHIP_UINT8Q).  Products that tfhip_matmul cuts into
+ * more partial tiles than the array holds are served all the same where they can be computed
+ * otherwise: transposed or batched ones by the float32 kernels instead of the bf16 ones, others whole or with fewer
+ * cuts.  These results agree with tfhip_matmul's to rounding.  All calls on one GPU share
  * the array: calls that overlap on one GPU (two contexts, two threads) race on it.  Calls on
  * one context do not: under one stream index they run in order, a call under the other index
  * (and a replay of a captured graph that recorded such a call) is put behind the array's last

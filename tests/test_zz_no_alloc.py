@@ -159,3 +159,29 @@ def test_noalloc_takes_the_same_kernels_for_transposed_operands(tf, m, k, n, ta,
     assert kernel == want
     assert np.array_equal(r1, r2)
     assert mem[0] == mem[1], "the pool changed during a no-alloc call: %s" % (mem,)
+
+
+@pytest.mark.parametrize("m,k,n,same", [
+    (1648, 3036, 708, True), (980, 12672, 1568, True),    # whole for tfhip_matmul: nothing to keep in the array
+    (516, 788, 796, False), (1412, 1412, 644, False),     # cut there into more than the array holds
+])
+def test_noalloc_serves_what_needs_no_more_than_the_array(tf, m, k, n, same):
+    rng = np.random.default_rng(m + k)
+    a = rng.uniform(-1, 1, (1, m, k)).astype(np.float32)
+    b = rng.uniform(-1, 1, (1, k, n)).astype(np.float32)
+    be = tf.backend()
+    with tf.tidy():
+        tf.matmul(tf.tensor(a[0]), tf.tensor(b[0]))
+        kernel_of_matmul = be.lib.tfhip_last_kernel(be.ctx).decode()
+    r1, r2, kernel, mem = _both(tf, a, b)
+    print("noalloc", m, k, n, kernel_of_matmul, kernel if r1 is not None else r2, flush=True)
+    assert r1 is not None, r2
+    assert mem[0] == mem[1], "the pool changed during a no-alloc call: %s" % (mem,)
+    if same:
+        assert kernel == kernel_of_matmul and np.array_equal(r1, r2)
+        return
+    # both round k products and sums of at most these magnitudes
+    bound = 2 * (k + 1) * 2.0 ** -24 * (np.abs(a[0]).astype(np.float64) @ np.abs(b[0]))
+    assert np.all(np.abs(r1[0].astype(np.float64) - r2[0]) <= bound)
+    want = a[0].astype(np.float64) @ b[0]
+    assert np.all(np.abs(r2[0] - want) <= bound)

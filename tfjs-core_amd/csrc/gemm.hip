@@ -1725,17 +1725,16 @@ static int launch_mode(tfhip_ctx* ctx, GemmArgs& p, int batch) {
   Plan plans[NCFG];
   int best = cheapest(plans, resident_blocks<Small, PLAN_MODE, BMODE, KBLOCKED, FAST>(ctx));
   if (KBLOCKED && ctx->no_alloc) {
-    // A program that allocates nothing is served where the partial tiles of a plan for six workgroups (five
-    // without FAST or of a transposed A) fit the scratch memory, which does not depend on how the 64 x 64
-    // tile is built; that plan takes over where the one above does not fit.
+    // A program that allocates nothing gets the plan above where its partial tiles fit the scratch memory.
+    // Where they do not, a plan for more workgroups on a CU may do without: it would cut further, which costs
+    // more partial tiles, and so leaves some products whole ([516, 788] x [788, 796]: six ways for four
+    // workgroups, 11.5 MB; whole for six).  Six, five without FAST or of a transposed A, is what this call was first
+    // planned for, and stays as a number so that what it has served does not depend on the occupancy of a tile.
     auto fits = [&](const Plan& pl, int i) {
       return pl.splits <= 1 || (size_t)pl.tail_tiles * pl.splits * bms[i] * bns[i] * sizeof(float) <= kScratchBytes;
     };
-    Plan six[NCFG];
-    const int which = cheapest(six, AMODE == A_ROWMAJOR && FAST ? 6 : 5);
-    if (!fits(six[which], which) || !fits(plans[best], best)) {
-      best = which;
-      plans[best] = six[best];
+    if (!fits(plans[best], best)) {
+      best = cheapest(plans, AMODE == A_ROWMAJOR && FAST ? 6 : 5);
     }
   }
   switch (best) {
