@@ -40,3 +40,23 @@ def test_filter_gradient(tf, n, h, w, c, stride, pad):
             want, magnitude = (part * dy).sum((0, 1, 2)), np.abs(part * dy).sum((0, 1, 2))
             # a lane adds at most 64 products in float32, the rest is added in float64
             assert np.all(np.abs(got[i, j, :, 0] - want) <= 66 * 2.0 ** -24 * magnitude)
+
+
+@pytest.mark.parametrize("n,h,w,c,stride,chain", [
+    (8, 14, 14, 512, 1, 8), (32, 28, 28, 128, 1, 8), (16, 14, 14, 256, 2, 8), (6, 17, 20, 64, 1, 8), (1, 14, 14, 512, 1, 8),
+    (1, 10, 6, 16, 1, 1), (2, 8, 4, 16, 1, 1), (1, 28, 28, 32, 1, 7),
+])
+def test_chains_of_low_images_are_short(tf, n, h, w, c, stride, chain):
+    """Where there are lanes for them, no lane adds more than 8 products in float32, and fewer of a tiny image:
+    a column of 2^25 and ones keeps the ones that its first sum does not meet."""
+    print("chains", n, h, w, c, stride, flush=True)
+    oh, ow = -(-h // stride), -(-w // stride)
+    dy = np.ones((n, oh, ow, c), np.float32)
+    columns = n * ow
+    assert columns % 2 == 0
+    dy[:, 0] = np.where(np.arange(columns) % 2, -2.0 ** 25, 2.0 ** 25).reshape(n, ow, 1)
+    with tf.tidy():
+        got = tf.depthwise_conv2d_der_filter(tf.tensor(np.ones((n, h, w, c), np.float32)), tf.tensor(dy),
+                                             (3, 3, c, 1), stride, "same").data_sync()
+    lost = columns * (oh - 1) - got[1, 1, :, 0]
+    assert np.all(lost >= 0) and np.all(lost <= columns * (chain - 1)), (lost.min(), lost.max(), columns)

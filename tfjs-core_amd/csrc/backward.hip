@@ -651,11 +651,15 @@ extern "C" int tfhip_depthwise_conv2d_der_filter(tfhip_ctx* ctx, int64_t x, int6
     while (qpw < 64 && qpw < c4) qpw *= 2;
     const int64_t blocks_c = ceil_div(c4, qpw);
     const int subs = 256 / qpw;
-    // The columns of the output are cut into segments of at least 8 rows (a segment reads two rows of
-    // x more than it has) until four workgroups per CU, which is what their LDS allows, have
-    // one each.
+    // The columns of the output are cut into segments until four workgroups per CU, which is what their LDS
+    // allows, have one each.  A segment reads two rows of x more than it has, so it is made no shorter
+    // than its chain of float32 additions may be long: 8, or what dealing the pixels evenly over
+    // workgroups of 8 pixels a lane gives.  (Segments of at least 8 rows, 14 where the image has 14:
+    // [8, 14, 14, 512] 6.0 us and 7.2e-8 from the sum in 64 bits, 5.5 us and 5.5e-8 in halves; [1, 14, 14, 512]
+    // 5.9 and 4.7; [16, 28, 28, 256] 9.2 and 9.4; [64, 28, 28, 256] at stride 2 13.7 and 14.3, 7.3e-8 and 5.6e-8.)
     const int64_t columns = (int64_t)ci->batch * ci->out_w, most = ceil_div((int64_t)ctx->num_cus * 4, blocks_c);
-    int64_t segs = std::max<int64_t>(1, std::min<int64_t>(most * subs / columns, ci->out_h / 8));
+    const int64_t chain = ceil_div(ceil_div(pixels, ceil_div(pixels, (int64_t)subs * 8)), subs);
+    int64_t segs = std::max<int64_t>(1, std::min<int64_t>(most * subs / columns, ceil_div(ci->out_h, chain)));
     const int64_t rows = ceil_div(ci->out_h, segs);
     segs = ceil_div(ci->out_h, rows);
     const int64_t units = columns * segs, per_lane = ceil_div(units, most * subs);
