@@ -1,9 +1,11 @@
 // Index-driven data movement and the resampling kernels around it: gatherND, scatterND /
 // sparseToDense, resizeBilinearBackprop, resizeNearestNeighborBackprop, cropAndResize.
 // Replaces backend_cpu.ts:2938-3013, 3070-3165, 3622-3757, 3759-3836, 3842-3889 of the
-// reference.  Every result element is produced by one lane that visits its contributions in
-// the order the reference's loops do, so sums round the same way and nothing depends on
-// scheduling (no atomics on data).
+// reference.  Every result element is the sum of its contributions in the order the reference's
+// loops visit them, so sums round the same way, with one exception: sums in double that are rounded once
+// (unsortedSegmentSum) are taken in parts where a row has very many entries
+// (scatter_groups_kernel), in an order that the indices alone decide.  Nothing depends on scheduling (no
+// atomics on data).
 #include <algorithm>
 #include <climits>
 #include <type_traits>
