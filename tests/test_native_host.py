@@ -223,6 +223,19 @@ def test_replaced_product_methods_are_called(fake, derived):
     tf.dispose([a, b])
 
 
+def test_copies_of_records(fake):
+    import copy
+    import tfhip as tf
+    base = counts()
+    t = tf.tensor(np.zeros((2, 3), np.float32))
+    t.note = "kept"
+    c = copy.copy(t)
+    assert [getattr(c, f) for f in FIELDS] == [getattr(t, f) for f in FIELDS] and c.note == "kept" and c is not t
+    assert type(c) is type(t) and counts() == (base[0] + 1, base[1] + 1, base[2] + 24)
+    t.dispose()
+    assert counts() == base and not c.is_disposed
+
+
 def test_nothing_is_held(fake):
     import tfhip as tf
     value = np.zeros(7, np.float32)

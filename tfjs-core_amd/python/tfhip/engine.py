@@ -54,6 +54,16 @@ class Tensor(_native.TensorBase):
                 return (vals.astype(np.uint8) if as_bool else vals).reshape(shape)
         return _Data()
 
+    def __copy__(self):
+        """The same record again, its data counted once (copy.copy; the base class's fields are not in
+        __dict__, where it would look for them)."""
+        other = type(self).__new__(type(self))
+        for name in ("shape", "dtype", "size", "rank", "data_id", "quant", "is_disposed", "id"):
+            if hasattr(self, name):
+                setattr(other, name, getattr(self, name))
+        other.__dict__.update(self.__dict__)
+        return other
+
     def reshape(self, shape):
         self._check()
         return ENGINE.backend.reshape(self, shape)
