@@ -84,11 +84,12 @@ int tfhip_write(tfhip_ctx* ctx, int64_t id, const void* host, size_t nbytes);
 int tfhip_read(tfhip_ctx* ctx, int64_t id, void* host, size_t nbytes);
 int tfhip_dispose(tfhip_ctx* ctx, int64_t id);
 /* How the copies are ordered.  Kernels run on one in-order stream.  tfhip_write sends up to
- * 64 KiB (1 MiB when nothing was queued since the host last waited for that stream) through pinned memory on that stream and returns without
- * waiting; larger writes run on a second stream, so that they overlap with the kernels queued before
- * them, and the first kernel that uses the buffer waits for the copy (the device backends of the reference upload
+ * 64 KiB (from ordinary memory 1 MiB, when nothing was queued since the host last waited for that
+ * stream) through pinned memory on that stream and returns without waiting; larger writes run on
+ * a second stream, so that they overlap with the kernels queued before them, and the first
+ * kernel that uses the buffer waits for the copy (the device backends of the reference upload
  * lazily for the same reason: tfjs-webgpu/src/backend_webgpu.ts:191-245,
- * backends/webgl/backend_webgl.ts:425-499).  From ordinary memory the call returns when the
+ * backends/webgl/backend_webgl.ts:425-499).  Larger writes from ordinary memory return when the
  * copy is done (the caller's array is its own again).  From memory of tfhip_host_alloc the call
  * returns at once and the copy reads the caller's buffer later: leave it unchanged until
  * tfhip_sync, tfhip_read or a finished asynchronous read of a result that depends on it — the

@@ -684,11 +684,12 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N * 64) void gemm_kernel(const GemmA
 
   // Software pipeline over the k steps (BK = 16 = two fragments of 8 k each).  In flight at
   // any time: the matrix cores on tile i out of LDS buffer i&1, tile i+1 on its way from
-  // registers into the other LDS buffer, and the global loads of tile i+2 into registers.
+  // registers into the other LDS buffer, and the global loads of the tiles up to i+AHEAD (two or
+  // three, see below) into registers.
   // One step, for tile i:
   //   read fragment 1 of tile i          (LDS latency hidden by the next MFMAs)
   //   MFMAs of fragment 0, first half
-  //   park tile i+1 in the other LDS buffer; issue the global loads of tile i+2
+  //   park tile i+1 in the other LDS buffer; issue the global loads of tile i+AHEAD
   //   MFMAs of fragment 0, second half
   //   barrier                            (tile i+1 visible, buffer i&1 free next step)
   //   read fragment 0 of tile i+1        (latency hidden by the MFMAs of fragment 1)

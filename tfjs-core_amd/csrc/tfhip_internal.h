@@ -141,7 +141,9 @@ struct tfhip_ctx {
   // it may be let go before anything of its own was queued.)
   std::unordered_set<void*> quiet, exported;
   // A pinned block per compute stream for a larger write that finds the stream idle: the copy out of it
-  // runs on that stream, so an idle stream also says that the block is free.
+  // runs on that stream, so an idle stream also says that the block is free.  (The first such write
+  // of a process makes the block and launches the first kernel: 512 KB 0.8 ms, against 0.35 by the
+  // copy engine; from then on 12 us, against 33.)
   char* stages[kStreams] = {};
   char* idle_stage();  // the selected stream's block, or nullptr (work is queued, or no memory)
   // The same for reads, which wait for their copy: one block, of every size up to its own.  A read that
