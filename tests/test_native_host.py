@@ -156,8 +156,9 @@ def test_an_engine_without_its_backend_field_raises(fake):
 def test_arguments_by_name(fake):
     """The engine's and the backend's methods take their arguments by name, as Python functions do."""
     import tfhip as tf
-    from tfhip import _native
+    from tfhip import _capi, _native
     from tfhip.engine import ENGINE, DataId, Tensor
+    _capi.lib()
     base = counts()
     ENGINE.start_scope()
     a, b = tf.tensor(1.0), tf.tensor(2.0)
