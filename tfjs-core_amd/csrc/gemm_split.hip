@@ -753,11 +753,11 @@ static int launch_mode(tfhip_ctx* ctx, const GemmArgs& p, int batch, int amode32
 
 // Which products come here: transposed and batched ones and the gradients of convolutions, where
 // the two estimates above say so.  Measured on MI355X with normal values, float32 kernels against
-// these: [3000, 1000]^T-shaped x [1000, 3000] 203 -> 177 us, [1500, 3000] x [3000, 900]^T 102 -> 84,
-// 3 x [1280, 1600] x [1600, 2240] 289 -> 230, 96 x [201, 67] x [67, 201] 24.1 -> 13.2, 3 x 3 filter
-// gradient of [32, 56, 56, 64] -> 128 159 -> 109, its input gradient 209 -> 139, 128 in tiles of
-// [256, 64] and with the taps' places in scalar registers (5 x 5 of [8, 28, 28, 64] <- 256 77 -> 55).
-// Small products are quicker there (16 x [128, 128] x [128, 128] 5.8 against 8.2, [1000, 256] x [256, 100] 10.6 against
+// these, kernel times: [3000, 1000]^T-shaped x [1000, 3000] 192 -> 165 us, [1500, 3000] x [3000, 900]^T
+// 94 -> 81, 3 x [1280, 1600] x [1600, 2240] 245 -> 203, 96 x [201, 67] x [67, 201] 24.6 -> 13.2, 3 x 3 filter
+// gradient of [32, 56, 56, 64] -> 128 157 -> 114, its input gradient 185 -> 116 (139 in tiles of [128, 64] and
+// with the taps placed per lane), 5 x 5 of [8, 28, 28, 64] <- 256 84 -> 52.
+// Small products are quicker there (16 x [128, 128] x [128, 128] 5.3 against 8.2, [1000, 256] x [256, 100] 10.4 against
 // 12.5).  Row-major products of one batch entry, and with them the pointwise convolutions, and
 // forward convolutions have not been moved: the float32 kernels' tile choice for them is asserted by
 // name at some sizes, and the results of relu and max pooling behind a forward convolution change
