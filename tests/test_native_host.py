@@ -210,7 +210,9 @@ def test_replaced_product_methods_are_called(fake, derived):
         be = type("Derived", (MathBackendHIP,), dict(as_methods, __init__=lambda self: None))()
     else:
         be = MathBackendHIP.__new__(MathBackendHIP)
-        be.__dict__.update(methods)
+        for name, method in methods.items():
+            setattr(be, name, method)
+    assert type("Plain", (MathBackendHIP,), {})._own_product and MathBackendHIP._own_product
     a, b = tf.tensor(np.zeros((2, 3), np.float32)), tf.tensor(np.zeros((3, 4), np.float32))
     backend, ENGINE._backend = ENGINE._backend, be
     try:
